@@ -62,11 +62,46 @@ __device__ __forceinline__ double rsqrt_core(double m)
   return (Tu < 0.0) ? up : ((Td > 0.0) ? dn : y);
 }
 
+// The same value from one cubic step and one residual: with
+// e = 1 - m y0^2 (|e| < 2^-22, the hardware seed), y = y0 (1 + e/2 + 3/8 e^2)
+// is within an ulp of 1/sqrt(m); e1 = 1 - m y^2, formed from the exact product
+// m y = h + l, has |e1| < 2^-51 and an error below 2^-104, so 1/sqrt(m) =
+// y + y e1/2 up to 2^-102.5 relative (the next term, 3/8 e1^2, included).
+// Rounding y + (y/2)(e1 +- 2^-100) therefore brackets the rounding of the
+// exact value: equal results are the correctly rounded 1/sqrt(m).  They differ
+// only for values within 2^-101 of a midpoint of two doubles: sure is false
+// there (and true for a NaN), and the caller takes rsqrt_core.  Any m whose
+// sqrt is far from the ends of the exponent range will do (the steps scale
+// with m): half the instructions of rsqrt_core, whose two midpoint residuals
+// cost more than its value.
+__device__ __forceinline__ double rsqrt_bracket(double m, bool &sure)
+{
+  double y = __builtin_amdgcn_rsq(m);
+  double h = m * y;
+  double e = __fma_rn(-h, y, 1.0);
+  y = __fma_rn(y * e, __fma_rn(e, 0.375, 0.5), y);
+  h = m * y;
+  const double l = __fma_rn(m, y, -h);
+  e = __fma_rn(-h, y, 1.0);
+  e = __fma_rn(-l, y, e);
+  const double yh = 0.5 * y;
+  const double lo = __fma_rn(yh, e - 0x1p-100, y), hi = __fma_rn(yh, e + 0x1p-100, y);
+  sure = !(hi > lo);
+  return lo;
+}
+
+// Whether x is a positive normal number with an exponent in [-927, 929): the
+// inputs rsqrt_bracket takes unscaled.
+__device__ __forceinline__ bool rsqrt_plain_range(double x)
+{
+  return (unsigned)__double2hiint(x) - 0x06000000u < 0x7a000000u - 0x06000000u;
+}
+
 // Correctly rounded 1/sqrt(x).  Replaces my_drsqrt_rn of
 // share/device_code_common.hpp:89-133 (whose contract is the correctly
 // rounded result).  Own method: x = m * 4^k with m in [1,4), rsqrt_core(m),
 // exact rescaling; IEEE special values as the reference returns them.
-__device__ __forceinline__ double dev_rsqrt(double x)
+__device__ __forceinline__ double dev_rsqrt_any(double x)
 {
   // special inputs resolved by selects (no branches: the callers' code stays
   // straight-line for the scheduler); the main path also runs on them, its
@@ -86,6 +121,29 @@ __device__ __forceinline__ double dev_rsqrt(double x)
   sp = (x == 0.0) ? u2d((b0 & 0x8000000000000000ull) | 0x7ff0000000000000ull) : sp;  // +-0: +-inf
   sp = (x != x) ? x + x : sp;                                        // NaN
   return special ? sp : normal;
+}
+
+// The same through rsqrt_bracket where every active lane's x allows it (a
+// wave-uniform branch): the general path is left for special, very large or
+// very small inputs and for values next to a midpoint.
+__device__ __forceinline__ double dev_rsqrt(double x)
+{
+  bool sure;
+  double y = rsqrt_bracket(x, sure);
+  if (__ballot(!(sure && rsqrt_plain_range(x))) != 0ull)
+    y = dev_rsqrt_any(x);
+  return y;
+}
+
+// Correctly rounded 1/sqrt(m) of a rotation's m = 1 +- t^2 (2^-26 < m <= 2,
+// or NaN): no scaling, no special values.
+__device__ __forceinline__ double rsqrt_near1(double m)
+{
+  bool sure;
+  double y = rsqrt_bracket(m, sure);
+  if (__ballot(!sure) != 0ull)
+    y = dev_rsqrt_any(m);
+  return y;
 }
 
 // 2x2 rotation of share/device_code_common_rotate.hpp:189-237 (USE_RSQRT),
@@ -119,7 +177,7 @@ __device__ __forceinline__ int dev_rot(bool trig, double Apq, double Dp, double 
   const double tt = fix ? TANH1_FIX : copysign(rcot, ct2);
   double cr = 1.0;
   if (__ballot(!large && !fix) != 0ull)
-    cr = pin(dev_rsqrt(__fma_rn(trig ? tt : -tt, tt, 1.0)));
+    cr = pin(rsqrt_near1(__fma_rn(trig ? tt : -tt, tt, 1.0)));
   c = large ? 1.0 : (fix ? COSHI_FIX : cr);
   t = tt;
   return large ? 0 : ((small || fix) ? 1 : (trig ? (cr < 1.0) : (cr > 1.0)));
@@ -133,29 +191,6 @@ __device__ __forceinline__ int dev_rot_t(double Apq, double Dp, double Dq, doubl
 __device__ __forceinline__ int dev_rot_h(double Apq, double Dp, double Dq, double &c, double &t)
 {
   return dev_rot(false, Apq, Dp, Dq, c, t);
-}
-
-// xor-swizzle of a double inside each 32-lane half of the wave
-// (ds_swizzle bit mode: and 0x1f, or 0, xor M).
-template <int M>
-__device__ __forceinline__ double swz_xor(double v)
-{
-  const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), (M << 10) | 0x1F);
-  const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), (M << 10) | 0x1F);
-  return __hiloint2double(hi, lo);
-}
-
-// Sum over the 32 lanes of a half wave by the xor butterfly 16,8,4,2,1
-// (the order of dSum32, share/device_code_common_Kepler.hpp:26-74).  Every
-// lane ends with the same bits (IEEE addition commutes).
-__device__ __forceinline__ double sum32(double v)
-{
-  v = v + swz_xor<16>(v);
-  v = v + swz_xor<8>(v);
-  v = v + swz_xor<4>(v);
-  v = v + swz_xor<2>(v);
-  v = v + swz_xor<1>(v);
-  return v;
 }
 
 // Lane exchanges inside groups of 8 lanes by DPP (no LDS traffic):
@@ -174,16 +209,103 @@ __device__ __forceinline__ double lane_xor4(double v) { return dpp_mov<0x1B>(dpp
 __device__ __forceinline__ double lane_xor2(double v) { return dpp_mov<0x4E>(v); }
 __device__ __forceinline__ double lane_xor1(double v) { return dpp_mov<0xB1>(v); }
 
-// Sum of the 32 rows of one pivot pair held by 8 lanes, lane r holding rows
-// r, r+8, r+16, r+24 as v0..v3: the xor butterfly 16,8,4,2,1 of the 32-lane
-// reduction (levels 16 and 8 inside the lane, 4,2,1 across lanes).
-__device__ __forceinline__ double sum8x4(double v0, double v1, double v2, double v3)
+// Row held by lane l of a group of LANES (8 or 16) lanes that share the 32 rows
+// of a pivot pair: lane l keeps rows row_of(l) + LANES i.  The reduction's
+// partners at distance 4, 2 and 1 are then lanes l ^ 7, l ^ 2 and l ^ 1, each
+// one DPP move (half-row mirror, quad permutations); distance 8 is a
+// rotation of the 16-lane row by 8.
+__device__ __forceinline__ unsigned row_of(unsigned l)
 {
-  double s = (v0 + v2) + (v1 + v3);
-  s = s + lane_xor4(s);
-  s = s + lane_xor2(s);
-  s = s + lane_xor1(s);
-  return s;
+  return l ^ ((l & 4u) ? 3u : 0u);
+}
+
+// a, b, c computed before anything after this point uses one of them
+__device__ __forceinline__ void pin3(double &a, double &b, double &c)
+{
+  asm volatile("" : "+v"(a), "+v"(b), "+v"(c));
+}
+
+// One reduction level of three sums, side by side (one after the other each
+// would wait out its own add -> DPP latency).
+template <int CTRL>
+__device__ __forceinline__ void level3(double &a, double &b, double &c)
+{
+  const double x = dpp_mov<CTRL>(a), y = dpp_mov<CTRL>(b), z = dpp_mov<CTRL>(c);
+  a = a + x;
+  b = b + y;
+  c = c + z;
+  pin3(a, b, c);
+}
+
+// Dp = p.p, Dq = q.q, Apq = p.q over the 32 rows of a pivot pair, p[i], q[i]
+// being row row_of(l) + LANES i: each by the xor butterfly 16,8,4,2,1 of the
+// 32-lane reduction, the first levels inside the lane.
+template <unsigned LANES>
+__device__ __forceinline__ void dots3(const double *p, const double *q, double &Dp, double &Dq,
+                                      double &Apq)
+{
+  constexpr unsigned ROWS = 32u / LANES;
+  double tp[ROWS], tq[ROWS], tx[ROWS];
+#pragma unroll
+  for (unsigned i = 0u; i < ROWS; ++i) {
+    tp[i] = __fma_rn(p[i], p[i], 0.0);
+    tq[i] = __fma_rn(q[i], q[i], 0.0);
+    tx[i] = __fma_rn(p[i], q[i], 0.0);
+  }
+#pragma unroll
+  for (unsigned n = ROWS / 2u; n >= 1u; n >>= 1) {
+#pragma unroll
+    for (unsigned i = 0u; i < n; ++i) {
+      tp[i] = tp[i] + tp[i + n];
+      tq[i] = tq[i] + tq[i + n];
+      tx[i] = tx[i] + tx[i + n];
+    }
+  }
+  Dp = tp[0];
+  Dq = tq[0];
+  Apq = tx[0];
+  pin3(Dp, Dq, Apq);
+  if constexpr (LANES >= 16u) level3<0x128>(Dp, Dq, Apq);  // rows 8 apart
+  if constexpr (LANES >= 8u) level3<0x141>(Dp, Dq, Apq);   // 4 apart (see row_of)
+  level3<0x4E>(Dp, Dq, Apq);
+  level3<0xB1>(Dp, Dq, Apq);
+}
+
+// dev_rot for a pivot pair whose lanes (a multiple of four, from a multiple of
+// four on) all hold the same Apq, Dp, Dq: also sqrt(Dp) sqrt(Dq).  The three
+// square roots -- of zeta^2 +- 1, Dp and Dq -- are one instruction sequence,
+// on lanes 0, 1 and 2 of every quad, spread by DPP moves (the roots of the
+// norms are wanted late, by the convergence test).  HYP: trig is set per
+// pair, else every pair is trigonometric.  (Pinned values: operands of
+// selects, which would otherwise become branches.)
+template <bool HYP>
+__device__ __forceinline__ bool rot_quad(bool trig, double Apq, double Dp, double Dq, unsigned l,
+                                         double &c, double &t, double &Dpq_)
+{
+  if (!HYP) trig = true;
+  const double h = Dq + (trig ? -Dp : Dp);
+  const double qz = h / (2.0 * Apq);
+  const double ct2 = trig ? qz : -qz;
+  const double CT2 = fabs(ct2);
+  const bool large = CT2 >= SQRT_2_HEPS;
+  const bool small = trig & (CT2 < SQRT_HEPS);
+  const bool fix = !trig & !large & !(CT2 > 1.0);
+  const double z = pin(__fma_rn(CT2, CT2, trig ? 1.0 : -1.0));
+  const unsigned q = l & 3u;
+  const double s3 = sqrt((q == 1u) ? Dp : ((q == 2u) ? Dq : z));
+  const double sq = dpp_mov<0x00>(s3);
+  Dpq_ = dpp_mov<0x55>(s3) * dpp_mov<0xAA>(s3);
+  // CT2 + CT2, CT2 + 1 or CT2 + sqrt
+  const double cot = CT2 + (large ? CT2 : (small ? 1.0 : sq));
+  const double rcot = pin(1.0 / cot);
+  const double tt = fix ? TANH1_FIX : copysign(rcot, ct2);
+  double cr = 1.0;
+  if (__ballot(!large & !fix) != 0ull)
+    cr = pin(rsqrt_near1(__fma_rn(trig ? tt : -tt, tt, 1.0)));
+  c = large ? 1.0 : (fix ? COSHI_FIX : cr);
+  t = tt;
+  const bool off1 = HYP ? (trig ? (cr < 1.0) : (cr > 1.0)) : (cr < 1.0);
+  return !large & (small | fix | off1);
 }
 
 __device__ __forceinline__ double readlane_d(double v, int lane)
@@ -215,9 +337,52 @@ __device__ __forceinline__ void wave_lds_sync()
 // (USE_RSQRT): column k is scaled by rsqrt(A(k,k)), the diagonal set to
 // sqrt(A(k,k)), then A(x,j) = fma(-A(x,k), A(j,k), A(x,j)) for the rows
 // x >= j > k.  A: the Gram's lower triangle in LDS (A[c * LD + r] = A(r,c),
-// c <= r); on return A holds R = L^T (zeros below the diagonal).  col: 32
-// doubles of LDS for the column broadcast.
+// c <= r); on return A holds R = L^T (zeros below the diagonal).  col: 64
+// doubles of LDS for the column broadcast.  check: whether every factor entry
+// is finite and the diagonal positive (wave-uniform).
 //
+// chol32_any takes any input: column by column in LDS, lane l on row l % 32
+// of the columns j = l/32, l/32 + 2, ...
+template <unsigned LD>
+__device__ __forceinline__ bool chol32_any(lds_f64 *A, lds_f64 *col, unsigned l, bool check)
+{
+  const unsigned x = l & 31u, h = l >> 5;
+#pragma unroll 1
+  for (unsigned k = 0u; k < 32u; ++k) {
+    const double akk = A[k * LD + k];
+    const double v = A[k * LD + x];
+    const double rk = dev_rsqrt_any(akk), dk = sqrt(akk);
+    const double w = (x == k) ? dk : v * rk;
+    wave_lds_sync();
+    if (x >= k) A[k * LD + x] = w;
+    col[x] = w;
+    wave_lds_sync();
+#pragma unroll 1
+    for (unsigned j = k + 1u + h; j < 32u; j += 2u)
+      if (x >= j) A[j * LD + x] = __fma_rn(-w, col[j], A[j * LD + x]);
+    wave_lds_sync();
+  }
+  bool ok = true;
+#pragma unroll 1
+  for (unsigned c = h; c < 32u; c += 2u) {
+    const double v = A[c * LD + x];
+    if (check && c <= x) ok = ok && (fabs(v) <= 0x1.fffffffffffffp+1023);
+    if (check && c == x) ok = ok && (v > 0.0);
+  }
+  // R = L^T in place, one column against one row at a time
+#pragma unroll 1
+  for (unsigned c = 0u; c < 32u; ++c) {
+    const double v = A[c * LD + x];
+    wave_lds_sync();
+    if (h == 0u && x > c) {
+      A[x * LD + c] = v;
+      A[c * LD + x] = 0.0;
+    }
+    wave_lds_sync();
+  }
+  return !check || (__ballot(ok) == ~0ull);
+}
+
 // Lane l keeps row x = l % 32 of the columns c = 2i + l/32 (i = 0..15), so
 // one instruction updates an even column in one half of the wave and an odd
 // one in the other: 16 registers and half the update instructions of a
@@ -225,9 +390,11 @@ __device__ __forceinline__ void wave_lds_sync()
 // they produce values that no later step reads (the pivot is read on the
 // diagonal, the broadcast column below it) and that are not stored.  The
 // next pivot A(k+1,k+1) - L(k+1,k)^2 is formed from two readlanes as soon
-// as column k is scaled, so its rsqrt runs beside the column's updates.
-// check: whether every factor entry is finite and the diagonal positive
-// (wave-uniform).
+// as column k is scaled, so its rsqrt (rsqrt_bracket: the chain of the 32
+// pivots is this routine's time) runs beside the column's updates.  The
+// diagonal stays unscaled until the end, where one square root instruction
+// serves all 32 entries.  A pivot that rsqrt_bracket does not settle sends
+// the matrix, still whole in LDS, to chol32_any.
 template <unsigned LD>
 __device__ __forceinline__ bool chol32_wave(double *A_, double *col_, unsigned l, bool check)
 {
@@ -240,45 +407,63 @@ __device__ __forceinline__ bool chol32_wave(double *A_, double *col_, unsigned l
     const unsigned c = 2u * i + h;
     b[i] = (c <= x) ? A[c * LD + x] : 0.0;
   }
+  // the lanes of the other half than the pivot column's write beside col
+  // (no branch, no select); xh[hk]: x in the half of the even (odd) columns,
+  // 0 in the other
+  lds_f64 *const cw[2] = {col + x + 32u * h, col + x + 32u * (h ^ 1u)};
+  const unsigned xh[2] = {h ? 0u : x, h ? x : 0u};
   double akk = readlane_d(b[0], 0);
-  double rk = dev_rsqrt(akk), dk = sqrt(akk);
+  bool sure;
+  double rk = rsqrt_bracket(akk, sure);
+  unsigned long long bad = __ballot(!(sure && rsqrt_plain_range(akk)));
 #pragma unroll
-  for (unsigned k = 0u; k < 32u; ++k) {
-    const unsigned ik = k >> 1, hk = k & 1u;
-    const bool own = (h == hk);
-    if (own && x > k) b[ik] = b[ik] * rk;
-    else if (own && x == k) b[ik] = dk;
-    if (k + 1u < 32u) {
-      const unsigned k1 = k + 1u;
-      if (own) col[x] = b[ik];
-      const double lk = readlane_d(b[ik], hk * 32u + k1);
-      const double d1 = readlane_d(b[k1 >> 1], (k1 & 1u) * 32u + k1);
-      akk = __fma_rn(-lk, lk, d1);
-      const double rn = dev_rsqrt(akk), dn = sqrt(akk);
-      // the other half reads what this half stored: without the fence the
-      // compiler may issue a lane's read of col[x] before the (conditional,
-      // other-lane) store, as no store of its own precedes it
-      wave_lds_sync();
-      const double lx = col[x];
+  for (unsigned k = 0u; k + 1u < 32u; ++k) {
+    const unsigned ik = k >> 1, hk = k & 1u, k1 = k + 1u;
+    const double u = pin(b[ik] * rk);
+    *cw[hk] = u;
+    b[ik] = pin((xh[hk] > k) ? u : b[ik]);
+    const double lk = readlane_d(u, hk * 32u + k1);
+    const double d1 = readlane_d(b[k1 >> 1], (k1 & 1u) * 32u + k1);
+    akk = __fma_rn(-lk, lk, d1);
+    // the other half reads what this half stored: without the fence the
+    // compiler may issue a lane's read of col[x] before the other lane's
+    // store
+    wave_lds_sync();
+    const double lx = col[x];
+    double cv[16];
 #pragma unroll
-      for (unsigned i = k1 >> 1; i < 16u; ++i) {
-        // column 2i + h; for i = k1/2 with k1 odd, only half 1's column is
-        // beyond k
-        if ((k1 & 1u) && i == (k1 >> 1) && h == 0u) continue;
-        b[i] = __fma_rn(-lx, col[2u * i + h], b[i]);
-      }
-      rk = rn;
-      dk = dn;
-      wave_lds_sync();
+    for (unsigned i = k1 >> 1; i < 16u; ++i)
+      cv[i] = col[2u * i + h];
+    // the column's reads are issued here, all of them, and used after the
+    // pivot's chain has started
+    __builtin_amdgcn_sched_barrier(0);
+    rk = rsqrt_bracket(akk, sure);
+    bad |= __ballot(!(sure && rsqrt_plain_range(akk)));
+#pragma unroll
+    for (unsigned i = k1 >> 1; i < 16u; ++i) {
+      // column 2i + h; for i = k1/2 with k1 odd, only half 1's column is
+      // beyond k
+      const double f = __fma_rn(-lx, cv[i], b[i]);
+      b[i] = ((k1 & 1u) && i == (k1 >> 1) && h == 0u) ? b[i] : f;
     }
+    // settled here: left to itself the compiler delays the updates to their
+    // columns' pivots and the test to the end, all operands in registers
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+s"(bad));
+#pragma unroll
+    for (unsigned i = k1 >> 1; i < 16u; ++i)
+      asm volatile("" : "+v"(b[i]));
+    wave_lds_sync();
   }
+  if (bad)
+    return chol32_any<LD>(A, col, l, check);
   bool ok = true;
   if (check) {
+    // (the diagonal is positive: its pivots were in rsqrt_bracket's range)
 #pragma unroll
     for (unsigned i = 0u; i < 16u; ++i) {
       const unsigned c = 2u * i + h;
-      if (c <= x) ok = ok && (fabs(b[i]) <= 0x1.fffffffffffffp+1023);
-      if (c == x) ok = ok && (b[i] > 0.0);
+      if (c < x) ok = ok && (fabs(b[i]) <= 0x1.fffffffffffffp+1023);
     }
     ok = (__ballot(ok) == ~0ull);
   }
@@ -287,6 +472,10 @@ __device__ __forceinline__ bool chol32_wave(double *A_, double *col_, unsigned l
     const unsigned c = 2u * i + h;
     A[x * LD + c] = (c <= x) ? b[i] : 0.0;
   }
+  wave_lds_sync();
+  const double d = sqrt(A[x * LD + x]);
+  wave_lds_sync();
+  A[x * LD + x] = d;
   return ok;
 }
 
@@ -346,31 +535,23 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
         Gq[k] = L0A(R, r + 4u * k, q);
       }
       double Dp, Dq, Apq;
-      {
-        double t[8];
-#pragma unroll
-        for (unsigned k = 0u; k < 8u; ++k)
-          t[k] = __fma_rn(Gp[k], Gp[k], 0.0);
-        Dp = sum4x8(t);
-#pragma unroll
-        for (unsigned k = 0u; k < 8u; ++k)
-          t[k] = __fma_rn(Gq[k], Gq[k], 0.0);
-        Dq = sum4x8(t);
-#pragma unroll
-        for (unsigned k = 0u; k < 8u; ++k)
-          t[k] = __fma_rn(Gp[k], Gq[k], 0.0);
-        Apq = sum4x8(t);
-      }
-      const double Dp_ = sqrt(Dp), Dq_ = sqrt(Dq), Apq_ = fabs(Apq), Dpq_ = Dp_ * Dq_;
-      const int transf_s = !(Apq_ < (Dpq_ * MYTOL));
-      if (COS && swp == 0u)
-        my_cos = fmax(my_cos, (Dpq_ > 0.0) ? (Apq_ / Dpq_) : 0.0);
+      dots3<4u>(Gp, Gq, Dp, Dq, Apq);
       int pdef = def;
       if (hyp) {
         if ((p < npos) && (q < npos)) pdef = +1;
         else if ((p >= npos) && (q >= npos)) pdef = -1;
         else pdef = 0;
       }
+      bool trig;
+      if (!SORT) trig = !hyp || pdef;
+      else trig = (pdef != 0);
+      // the rotation on every lane; only a transforming pair uses it
+      double c, t, Dpq_;
+      const bool rot_b = rot_quad<true>(trig, Apq, Dp, Dq, l, c, t, Dpq_);
+      const double Apq_ = fabs(Apq);
+      const int transf_s = !(Apq_ < (Dpq_ * MYTOL));
+      if (COS && swp == 0u)
+        my_cos = fmax(my_cos, (Dpq_ > 0.0) ? (Apq_ / Dpq_) : 0.0);
       int transf_b = 0;
       // W's columns p, q (the same lane reads and writes the same entries
       // within a step, so they may be read this late)
@@ -381,12 +562,8 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
         Vq[k] = L0A(W, r + 4u * k, q);
       }
       if (transf_s) {
-        double c, t, t_;
-        bool trig;
-        if (!SORT) trig = !hyp || pdef;
-        else trig = (pdef != 0);
-        transf_b = dev_rot(trig, Apq, Dp, Dq, c, t);
-        t_ = trig ? -t : t;
+        transf_b = rot_b ? 1 : 0;
+        const double t_ = trig ? -t : t;
         if (SORT && trig) {
           Dp = __fma_rn(t, Apq, Dp);
           Dq = __fma_rn(t_, Apq, Dq);

@@ -489,7 +489,6 @@ static unsigned issue_sweep_staged(hipStream_t s, const Work &w, bool sort, unsi
   base.fsplit = (split && g_fused_split) ? 1 : 0;
   auto visits = [&](StageArgs &x, unsigned st, const uint16_t *list, unsigned n) {
     x.npl = n;
-    x.npw = (n + 1u) / 2u;
     x.plist = list;
     x.ppairs = w.d_s1 + (size_t)st * np * 2u;
     x.ppart = w.part(st & 1u);
@@ -526,7 +525,7 @@ static unsigned issue_sweep_staged(hipStream_t s, const Work &w, bool sort, unsi
     // workgroups take one each while they fit the slots beside the visits
     // (two resident workgroups per CU), else two each
     x.qact = skipping ? w.d_qact + 2u * st + (q0 ? 1u : 0u) : nullptr;
-    x.islots = (2u * ncu > x.npw) ? 2u * ncu - x.npw : 1u;
+    x.islots = (2u * ncu > x.npl) ? 2u * ncu - x.npl : 1u;
     x.upart = w.part((st + 1u) & 1u);
     x.uplan = plan ? plan + (size_t)(st + 1u) * np : nullptr;
   };

@@ -5,8 +5,8 @@
 //   k_gram   : partial 32x32 Gram of each block pair over a row chunk, on
 //              FP64 MFMA 16x16x4 (one wave per (pair, chunk));
 //   k_pair   : per pair, sum of the partials, 32x32 Cholesky, the inner
-//              Jacobi sweep(s) on R in LDS accumulating W (one 128-thread
-//              workgroup per pair, 8 lanes per pivot pair);
+//              Jacobi sweep(s) on R in LDS accumulating W (one workgroup
+//              per pair, waves for R and waves for W);
 //   k_update : [G_i G_j] <- [G_i G_j] W and [V_i V_j] <- [V_i V_j] W on FP64
 //              MFMA (one wave per (pair, row chunk)).
 // The reference fuses the three into one CUDA block per pair
@@ -309,61 +309,211 @@ __global__ __launch_bounds__(256, 2) void k_gram_split(const double *__restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Block pair: Gram -> Cholesky -> inner Jacobi -> W, two waves per pair.
+// Block pair: Gram -> Cholesky -> inner Jacobi -> W, one workgroup per pair.
 // R and W live in LDS, column-major with a padded leading dimension.
-// Cholesky: wave 0, lane x (x < 32) keeps row x of the Gram in registers;
-// the pivot column is broadcast with readlane, no barriers.
-// Inner Jacobi: pivot-pair slot y = t/8 (0..15); lane r = t%8 of the slot
-// keeps rows r, r+8, r+16, r+24 of the two columns of R and of W.
+// Cholesky: one wave (chol32_wave).  Inner Jacobi: pair_visit.
 
 #define LDR 33u
 #define RA(A, r, c) (A)[(c) * LDR + (r)]
 #define F32(A, r, c) (A)[(c) * 32u + (r)]
+// lanes per pivot pair of level-0 (see pair_visit) in k_pair and k_stage
+constexpr unsigned PAIR_LANES = 16u;
+constexpr unsigned STAGE_LANES = 8u;
 
-// LDS of one pair visit (128 threads)
+// LDS of one pair visit
 struct PairLds {
   double R[32u * LDR];
   double W[32u * LDR];
-  double cholcol[32];
-  unsigned cnt_s[16], cnt_b[16];
-  float cmax[16];
+  double cholcol[64];
+  double diag[32];        // the Gram's diagonal
+  double rot[2][16][4];   // per step parity and pivot pair: c, t, |Apq|, |p| |q|
+  unsigned act[2][16];    // ... what happens to its columns (ACT_*)
+  unsigned cs[2], cb[2];  // rotations of an inner sweep, by its parity
+  unsigned cmax;          // bits of the largest cosine of the first inner sweep
   float bnorm[2];
   int chol_ok;
-  int go;     // the visit still runs inner sweeps
   int swp;    // a pivot pair was swapped by the sort rule
+  __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
 };
 
-// One pair visit by the 128 threads tid = 0..127 of a workgroup that may
-// run two visits side by side (256 threads, one PairLds each): both halves
-// execute the same barriers, a half without work (no pair, a skipped visit,
-// a failed split Cholesky, converged inner sweeps) passes them idle.
-// go_other: the other half's go flag, or null when the workgroup holds one
-// visit.  plan: the visit's plan (PLAN_FP64 without a plan).
-template <bool SORT>
-__device__ __forceinline__ void pair_visit(unsigned tid, bool present, unsigned pi, PairLds &L,
-                                           const int *go_other, const uint16_t *__restrict__ pairs,
+// what a step does to a pivot pair's columns of R and W
+constexpr unsigned ACT_ROT = 1u;    // rotated
+constexpr unsigned ACT_CROSS = 2u;  // the results change places (with ACT_ROT or alone)
+constexpr unsigned ACT_TRIG = 4u;   // the rotation is trigonometric
+
+// The columns of M (R or W) of a pivot pair after the step: lane l of the
+// pair's group holds rows row + LANES i as P[i], Q[i]; ap, aq: the first of
+// them in LDS.  Without branches: an untouched pair is stored as it is.
+template <unsigned LANES, bool HYP>
+__device__ __forceinline__ void apply_pair(lds_f64 *ap, lds_f64 *aq, const double *P,
+                                           const double *Q, bool rot, bool cross, bool trig,
+                                           double c, double t)
+{
+  constexpr unsigned ROWS = 32u / LANES;
+  lds_f64 *const A = cross ? aq : ap, *const B = cross ? ap : aq;
+  const double t_ = (!HYP || trig) ? -t : t;
+  double a[ROWS], b[ROWS];
+#pragma unroll
+  for (unsigned i = 0u; i < ROWS; ++i) {
+    // big rotation: scale by c; otherwise c == 1 exactly (dev_rot), and
+    // c * x is x
+    const double x = pin(c * __fma_rn(t_, Q[i], P[i])), y = pin(c * __fma_rn(t, P[i], Q[i]));
+    a[i] = rot ? x : P[i];
+    b[i] = rot ? y : Q[i];
+  }
+#pragma unroll
+  for (unsigned i = 0u; i < ROWS; ++i) {
+    A[LANES * i] = a[i];
+    B[LANES * i] = b[i];
+  }
+}
+
+// LDS column of a pivot index, fetched ahead: the operands of the next step's
+// reads are ready when its barrier opens
+__device__ __forceinline__ unsigned pinu(unsigned x)
+{
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// One level-0 sweep on R: lane r of group y takes pivot pair y of every step.
+// Counts its rotations and leaves each step's (c, t, ...) for the W waves.
+template <bool SORT, unsigned LANES, bool HYP>
+__device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
+                                         int def, unsigned npos, unsigned &my_s, unsigned &my_b,
+                                         bool &swapped)
+{
+  constexpr unsigned ROWS = 32u / LANES;
+  lds_f64 *const M = (lds_f64 *)L.R + row_of(r);
+  const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
+  // sorted definite pairs: columns by decreasing D for J = I, by increasing
+  // D for J = -I: descending in D xor this sign
+  const uint64_t neg0 = (!HYP && def < 0) ? 0x8000000000000000ull : 0ull;
+  unsigned pq = S0[0];
+  unsigned p = pq & 255u, q = pq >> 8, op = p * LDR, oq = q * LDR;
+#pragma unroll 1
+  for (unsigned step = 0u; step < s0steps; ++step) {
+    lds_f64 *const ap = M + op, *const aq = M + oq;
+    double Gp[ROWS], Gq[ROWS];
+#pragma unroll
+    for (unsigned i = 0u; i < ROWS; ++i) {
+      Gp[i] = ap[LANES * i];
+      Gq[i] = aq[LANES * i];
+    }
+    pq = S0[16u * min(step + 1u, s0steps - 1u)];
+    bool trig = true, inorder = SORT;
+    uint64_t neg = neg0;
+    if (HYP) {
+      const bool pp = p < npos, qp = q < npos;
+      trig = (pp == qp);
+      neg = pp ? 0ull : 0x8000000000000000ull;
+      inorder = SORT & trig;
+    }
+    double Dp, Dq, Apq;
+    dots3<LANES>(Gp, Gq, Dp, Dq, Apq);
+    // the rotation on every lane; only a transforming pair uses it
+    double c, t, Dpq_;
+    const bool big = rot_quad<HYP>(trig, Apq, Dp, Dq, r, c, t, Dpq_);
+    const double Apq_ = fabs(Apq);
+    const bool transf = !(Apq_ < (Dpq_ * MYTOL));
+    bool cross = false;
+    if (SORT) {
+      // rotated: unless in order afterwards; not rotated: when out of order
+      const double Ep = pin(__fma_rn(t, Apq, Dp)), Eq = pin(__fma_rn(-t, Apq, Dq));
+      const bool ge = u2d(d2u(Ep) ^ neg) >= u2d(d2u(Eq) ^ neg);
+      const bool lt = u2d(d2u(Dp) ^ neg) < u2d(d2u(Dq) ^ neg);
+      cross = inorder & ((transf & !ge) | (!transf & lt));
+      swapped = swapped | (cross & !transf);
+    }
+    apply_pair<LANES, HYP>(ap, aq, Gp, Gq, transf, cross, trig, c, t);
+    if (r == 0u) {
+      double *const o = L.rot[step & 1u][y];
+      o[0] = c;
+      o[1] = t;
+      o[2] = Apq_;
+      o[3] = Dpq_;
+      L.act[step & 1u][y] = (transf ? ACT_ROT : 0u) | (cross ? ACT_CROSS : 0u) |
+                            (trig ? ACT_TRIG : 0u);
+    }
+    my_s += transf ? 1u : 0u;
+    my_b += (transf & big) ? 1u : 0u;
+    p = pq & 255u;
+    q = pq >> 8;
+    op = pinu(p * LDR);
+    oq = pinu(q * LDR);
+    __syncthreads();
+  }
+}
+
+// The same sweep's rotations applied to W, each step's between the barrier
+// that ends it on the R waves and the next; with cosines, the largest
+// |Apq| / (|p| |q|).
+template <unsigned LANES>
+__device__ __forceinline__ void level0_w(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
+                                         bool cosines)
+{
+  constexpr unsigned ROWS = 32u / LANES;
+  lds_f64 *const M = (lds_f64 *)L.W + row_of(r);
+  const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
+  double my_cos = 0.0;
+#pragma unroll 1
+  for (unsigned step = 0u; step < s0steps; ++step) {
+    const unsigned pq = S0[16u * step];
+    const unsigned op = pinu((pq & 255u) * LDR), oq = pinu((pq >> 8) * LDR);
+    __syncthreads();
+    lds_f64 *const ap = M + op, *const aq = M + oq;
+    double P[ROWS], Q[ROWS];
+#pragma unroll
+    for (unsigned i = 0u; i < ROWS; ++i) {
+      P[i] = ap[LANES * i];
+      Q[i] = aq[LANES * i];
+    }
+    const double *const o = L.rot[step & 1u][y];
+    const unsigned act = L.act[step & 1u][y];
+    const double cn = o[2], cd = o[3];
+    apply_pair<LANES, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
+                            (act & ACT_TRIG) != 0u, o[0], o[1]);
+    if (cosines)
+      my_cos = fmax(my_cos, (cd > 0.0) ? cn / cd : 0.0);
+  }
+  // (a nonnegative float's bits order as the float does)
+  if (cosines && r == 0u)
+    atomicMax(&L.cmax, __float_as_uint((float)my_cos));
+}
+
+// One pair visit by the 32 LANES threads of a workgroup (LANES = 16 or 8
+// lanes per pivot pair).  The first half of the waves keeps R: per level-0
+// step the dot products, the rotation, the update of R.  The other half
+// applies the same rotations to W one step behind, from the step's (c, t) in
+// LDS, and does the bookkeeping (the largest cosine), so that neither is in
+// the chain of the 31 dependent steps; a barrier per step is all that orders
+// the two (the pivot pairs of a step touch disjoint columns).  A step is
+// bound by that chain -- LDS reads, five reduction levels, division, square
+// root, division, reciprocal root, the update and the barrier -- and by the
+// instructions one wave issues on it, so the lanes share the square roots
+// (rot_quad), the rows are laid out for one-move reduction levels (row_of)
+// and the next step's pivot indices are fetched ahead.
+//
+// Measured (cycles of 2.4 GHz, 512 x 256 in k_pair's LANES = 16): partial sums
+// 3.3K, Cholesky 11.4K (23.4K with the column's reads waited for one by one),
+// a level-0 sweep 46K = 1490 a step, end 3K; 27 us a visit, 29 us a launch,
+// where two waves of 8 lanes a pair, each with both R and W, took 51 us.
+// LANES = 8 (half the waves): 33.5 us, 4: 42 us.  k_stage takes 8, the
+// largest that its 256-thread workgroups hold; its items set its pace, and
+// one visit a workgroup there times the same as two (8192 x 8192: 1.29 s).
+// plan: the visit's plan (PLAN_FP64 without a plan); not PLAN_SKIP.
+template <bool SORT, unsigned LANES>
+__device__ __forceinline__ void pair_visit(unsigned tid, unsigned pi, PairLds &L,
+                                           const uint16_t *__restrict__ pairs,
                                            const double *__restrict__ part, unsigned nchunk,
                                            double *__restrict__ Wout, unsigned *__restrict__ flags,
                                            RunCtl *__restrict__ ctl, VisitRec *__restrict__ rec,
-                                           uint8_t plan, const uint8_t *S0, unsigned s0steps,
-                                           unsigned nswp, int definite, unsigned nplus)
+                                           uint8_t plan, const uint8_t *__restrict__ strat0,
+                                           unsigned s0steps, unsigned nswp, int definite,
+                                           unsigned nplus)
 {
-  double *const R = L.R;
-  double *const W = L.W;
-  if (tid == 0u)
-    L.swp = 0;
-  if (present && plan == PLAN_SKIP && tid == 0u) {
-    // skipped visit: no update, the record keeps the last executed visit
-    flags[pi] = 0u;
-    rec[pi].skips += 1u;
-    atomicAdd(&ctl->skipped, 1u);
-  }
-  bool live = present && plan != PLAN_SKIP;
-  unsigned iBlk = 0u, jBlk = 0u;
-  if (live) {
-    iBlk = pairs[2u * pi];
-    jBlk = pairs[2u * pi + 1u];
-  }
+  constexpr unsigned NT = 32u * LANES, ROWS = 32u / LANES;
+  const unsigned iBlk = pairs[2u * pi], jBlk = pairs[2u * pi + 1u];
 
   // local J structure, share/device_code_nosort_accumV.hpp:53-76
   bool hyp = false;
@@ -379,56 +529,63 @@ __device__ __forceinline__ void pair_visit(unsigned tid, bool present, unsigned 
     hyp = (def == 0);
   }
 
-  if (live) {
-    // sum of the chunk partials in chunk order: the six entries of a thread
-    // with all their chunk loads in flight together (one memory round trip)
+  {
+    // sum of the chunk partials in chunk order: a thread's entries with all
+    // their chunk loads in flight together (one memory round trip)
     const double *const pp = part + (size_t)pi * nchunk * 768u;
-    {
-      const unsigned e0 = tid;
-      double v[6][MAX_GRAM_CHUNKS];
+    constexpr unsigned NE = (768u + NT - 1u) / NT;
+    double v[NE][MAX_GRAM_CHUNKS];
 #pragma unroll
-      for (unsigned q = 0u; q < 6u; ++q)
+    for (unsigned q = 0u; q < NE; ++q)
 #pragma unroll
-        for (unsigned c = 0u; c < MAX_GRAM_CHUNKS; ++c)
-          if (c < nchunk) v[q][c] = pp[(size_t)c * 768u + e0 + 128u * q];
-#pragma unroll
-      for (unsigned q = 0u; q < 6u; ++q) {
-        const unsigned e = e0 + 128u * q;
-        const unsigned tile = e >> 8;
-        double s = v[q][0];
-#pragma unroll
-        for (unsigned c = 1u; c < MAX_GRAM_CHUNKS; ++c)
-          if (c < nchunk) s = s + v[q][c];
-        const unsigned l = (e >> 2) & 63u, r = e & 3u;
-        const unsigned i = 4u * r + (l >> 4), j = l & 15u;
-        const unsigned row = (tile == 0u) ? i : (16u + i);
-        const unsigned col = (tile == 2u) ? (16u + j) : j;
-        RA(R, row, col) = s;
-      }
+      for (unsigned c = 0u; c < MAX_GRAM_CHUNKS; ++c)
+        if (c < nchunk && tid + NT * q < 768u) v[q][c] = pp[(size_t)c * 768u + tid + NT * q];
+    // the level-0 table, 16 bytes a thread, and W = I while they arrive
+    if (tid < STRAT0_TAB_BYTES / 16u)
+      reinterpret_cast<uint4 *>(L.S0)[tid] = reinterpret_cast<const uint4 *>(strat0)[tid];
+    for (unsigned e = tid; e < 1024u; e += NT)
+      RA(L.W, e & 31u, e >> 5) = ((e & 31u) == (e >> 5)) ? 1.0 : 0.0;
+    if (tid == 0u) {
+      L.swp = 0;
+      L.cmax = 0u;
+      L.cs[0] = L.cb[0] = 0u;
     }
-    for (unsigned e = tid; e < 1024u; e += 128u)
-      RA(W, e & 31u, e >> 5) = ((e & 31u) == (e >> 5)) ? 1.0 : 0.0;
+#pragma unroll
+    for (unsigned q = 0u; q < NE; ++q) {
+      const unsigned e = tid + NT * q;
+      if (e >= 768u) break;
+      const unsigned tile = e >> 8;
+      double s = v[q][0];
+#pragma unroll
+      for (unsigned c = 1u; c < MAX_GRAM_CHUNKS; ++c)
+        if (c < nchunk) s = s + v[q][c];
+      const unsigned l = (e >> 2) & 63u, r = e & 3u;
+      const unsigned i = 4u * r + (l >> 4), j = l & 15u;
+      const unsigned row = (tile == 0u) ? i : (16u + i);
+      const unsigned col = (tile == 2u) ? (16u + j) : j;
+      RA(L.R, row, col) = s;
+      if (row == col) L.diag[row] = s;
+    }
   }
   __syncthreads();
-  if (live && tid < 2u) {
-    // squared Frobenius norms of the two blocks, for the visit record
-    double sn = 0.0;
-    for (unsigned k = 0u; k < 16u; ++k)
-      sn = sn + RA(R, 16u * tid + k, 16u * tid + k);
-    L.bnorm[tid] = (float)log2(sn);
-  }
-
   // Cholesky, share/device_code_common_Cholesky.hpp:58-158 (USE_RSQRT):
   // column k scaled by rsqrt(A(k,k)), diagonal sqrt(A(k,k)), then
   // A(x,j) = fma(-A(x,k), A(j,k), A(x,j)) for x >= j > k; R = L^T.
-  if (live && tid < 64u) {
+  if (tid < 64u) {
     // a Gram from the split products may miss positive definiteness (nearly
     // dependent columns): then no update, FP64 at the next visit
-    const bool ok = chol32_wave<LDR>(R, L.cholcol, tid, plan == PLAN_SPLIT);
-    if (plan == PLAN_SPLIT && tid == 0u) L.chol_ok = ok ? 1 : 0;
+    const bool ok = chol32_wave<LDR>(L.R, L.cholcol, tid, plan == PLAN_SPLIT);
+    if (tid == 0u) L.chol_ok = ok ? 1 : 0;
+  }
+  else if (tid < 66u) {
+    // squared Frobenius norms of the two blocks, for the visit record
+    double sn = 0.0;
+    for (unsigned k = 0u; k < 16u; ++k)
+      sn = sn + L.diag[16u * (tid - 64u) + k];
+    L.bnorm[tid - 64u] = (float)log2(sn);
   }
   __syncthreads();
-  if (live && plan == PLAN_SPLIT && !L.chol_ok) {
+  if (plan == PLAN_SPLIT && !L.chol_ok) {
     if (tid == 0u) {
       flags[pi] = 0u;
       VisitRec v;
@@ -443,138 +600,45 @@ __device__ __forceinline__ void pair_visit(unsigned tid, bool present, unsigned 
       rec[pi] = v;
       atomicAdd(&ctl->split, 1u);
     }
-    live = false;
+    return;
   }
 
   // Inner Jacobi: share/device_code_nosort.hpp:4-222 (SORT false),
   // share/device_code_cdsort_KISS.hpp:4-260 and share/device_code_cdsort.hpp:25-167
-  // (SORT true).  One barrier per step: the pivot pairs of a step touch
-  // disjoint columns; rotation counts are kept per slot and summed per sweep.
-  const unsigned y = tid >> 3, r = tid & 7u;
+  // (SORT true).
+  const bool onR = tid < NT / 2u;  // this wave's matrix: R or W
+  const unsigned ht = tid & (NT / 2u - 1u);
+  const unsigned y = ht / LANES, r = ht & (LANES - 1u);
   unsigned blk_s = 0u, blk_b = 0u;
-  bool swapped = false;
-  double my_cos = 0.0;
-  // |Apq| / (|p| |q|) of the previous step, divided during the next step's
-  // loads (off the step's chain of dependent operations)
-  double cos_n = 0.0, cos_d = 0.0;
-  bool sweeping = live;
   for (unsigned swp = 0u; swp < nswp; ++swp) {
-    // the halves go on while either still sweeps
-    if (tid == 0u) L.go = sweeping ? 1 : 0;
-    __syncthreads();
-    if (!L.go && !(go_other && *go_other))
-      break;
     unsigned my_s = 0u, my_b = 0u;
-    for (unsigned step = 0u; step < s0steps; ++step) {
-      if (sweeping) {
-      const unsigned p = S0[(step * 16u + y) * 2u], q = S0[(step * 16u + y) * 2u + 1u];
-      double Gp[4], Gq[4], Vp[4], Vq[4];
-#pragma unroll
-      for (unsigned i = 0u; i < 4u; ++i) {
-        Gp[i] = RA(R, r + 8u * i, p);
-        Gq[i] = RA(R, r + 8u * i, q);
-        Vp[i] = RA(W, r + 8u * i, p);
-        Vq[i] = RA(W, r + 8u * i, q);
-      }
-      if (swp == 0u) {
-        const double cr = pin(cos_n / cos_d);
-        my_cos = fmax(my_cos, (cos_d > 0.0) ? cr : 0.0);
-      }
-      double Dp = sum8x4(__fma_rn(Gp[0], Gp[0], 0.0), __fma_rn(Gp[1], Gp[1], 0.0),
-                         __fma_rn(Gp[2], Gp[2], 0.0), __fma_rn(Gp[3], Gp[3], 0.0));
-      double Dq = sum8x4(__fma_rn(Gq[0], Gq[0], 0.0), __fma_rn(Gq[1], Gq[1], 0.0),
-                         __fma_rn(Gq[2], Gq[2], 0.0), __fma_rn(Gq[3], Gq[3], 0.0));
-      const double Apq = sum8x4(__fma_rn(Gp[0], Gq[0], 0.0), __fma_rn(Gp[1], Gq[1], 0.0),
-                                __fma_rn(Gp[2], Gq[2], 0.0), __fma_rn(Gp[3], Gq[3], 0.0));
-      const double Dp_ = sqrt(Dp), Dq_ = sqrt(Dq), Apq_ = fabs(Apq), Dpq_ = Dp_ * Dq_;
-      const int transf_s = !(Apq_ < (Dpq_ * MYTOL));
-      cos_n = Apq_;
-      cos_d = Dpq_;
-      int pdef = def;
-      if (hyp) {
-        if ((p < npos) && (q < npos)) pdef = +1;
-        else if ((p >= npos) && (q >= npos)) pdef = -1;
-        else pdef = 0;
-      }
-      bool trig;
-      if (!SORT) trig = !hyp || pdef;
-      else trig = (pdef != 0);
-      // the rotation is computed beside the norms and the test, on every
-      // lane; only a transforming pair uses it
-      double c, t;
-      const int rot_b = dev_rot(trig, Apq, Dp, Dq, c, t);
-      int transf_b = 0;
-      if (transf_s) {
-        transf_b = rot_b;
-        const double t_ = trig ? -t : t;
-        if (SORT && trig) {
-          Dp = __fma_rn(t, Apq, Dp);
-          Dq = __fma_rn(t_, Apq, Dq);
-        }
-        bool keep = true;
-        if (SORT)
-          keep = (!pdef) || ((pdef > 0) && (Dp >= Dq)) || ((pdef < 0) && (Dp <= Dq));
-        const unsigned P = keep ? p : q, Q = keep ? q : p;
-#pragma unroll
-        for (unsigned i = 0u; i < 4u; ++i) {
-          // big rotation: scale by c; otherwise c == 1 exactly (dev_rot), and
-          // c * x is x
-          const double rp = __fma_rn(t_, Gq[i], Gp[i]), rq = __fma_rn(t, Gp[i], Gq[i]);
-          const double wp = __fma_rn(t_, Vq[i], Vp[i]), wq = __fma_rn(t, Vp[i], Vq[i]);
-          RA(R, r + 8u * i, P) = c * rp;
-          RA(R, r + 8u * i, Q) = c * rq;
-          RA(W, r + 8u * i, P) = c * wp;
-          RA(W, r + 8u * i, Q) = c * wq;
-        }
-      }
-      else if (SORT && (((pdef > 0) && (Dp < Dq)) || ((pdef < 0) && (Dq < Dp)))) {
-#pragma unroll
-        for (unsigned i = 0u; i < 4u; ++i) {
-          RA(R, r + 8u * i, p) = Gq[i];
-          RA(R, r + 8u * i, q) = Gp[i];
-          RA(W, r + 8u * i, p) = Vq[i];
-          RA(W, r + 8u * i, q) = Vp[i];
-        }
-        swapped = true;
-      }
-      my_s += (unsigned)transf_s;
-      my_b += (unsigned)transf_b;
-      }
-      __syncthreads();
+    bool swapped = false;
+    if (!onR)
+      level0_w<LANES>(L, y, r, s0steps, swp == 0u);
+    else if (hyp)
+      level0_r<SORT, LANES, true>(L, y, r, s0steps, def, npos, my_s, my_b, swapped);
+    else
+      level0_r<SORT, LANES, false>(L, y, r, s0steps, def, npos, my_s, my_b, swapped);
+    // every lane of a pair's group holds its counts
+    if (onR && r == 0u && my_s) {
+      atomicAdd(&L.cs[swp & 1u], my_s);
+      atomicAdd(&L.cb[swp & 1u], my_b);
     }
-    if (sweeping && swp == 0u) {
-      const double cr = pin(cos_n / cos_d);
-      my_cos = fmax(my_cos, (cos_d > 0.0) ? cr : 0.0);
-      cos_d = 0.0;
-    }
-    if (sweeping && r == 0u) {
-      L.cnt_s[y] = my_s;
-      L.cnt_b[y] = my_b;
-    }
+    if (onR && swapped)
+      L.swp = 1;
     __syncthreads();
-    if (sweeping) {
-      unsigned swp_s = 0u, swp_b = 0u;
-      for (unsigned i = 0u; i < 16u; ++i) {
-        swp_s += L.cnt_s[i];
-        swp_b += L.cnt_b[i];
-      }
-      if (swp_s) {
-        blk_s += swp_s;
-        blk_b += swp_b;
-      }
-      else
-        sweeping = false;
-    }
-    __syncthreads();
+    const unsigned swp_s = L.cs[swp & 1u];
+    // (the other parity was read before this sweep's steps)
+    if (tid == 0u)
+      L.cs[(swp + 1u) & 1u] = 0u;
+    if (tid == 64u)
+      L.cb[(swp + 1u) & 1u] = 0u;
+    if (!swp_s)
+      break;
+    blk_s += swp_s;
+    blk_b += L.cb[swp & 1u];
   }
 
-  if (live && r == 0u)
-    L.cmax[y] = (float)my_cos;
-  if (live && swapped)
-    L.swp = 1;
-  __syncthreads();
-  if (!live)
-    return;
   // convergence counter, share/device_code_nosort.hpp:94-103
   if (tid == 0u) {
     unsigned long long *const cvg = &ctl->cvg;
@@ -587,13 +651,10 @@ __device__ __forceinline__ void pair_visit(unsigned tid, bool present, unsigned 
     // the block update is left out exactly when W is the identity (no
     // rotation, no swap)
     flags[pi] = (blk_s || L.swp) ? 1u : 0u;
-    float cm = 0.0f;
-    for (unsigned i = 0u; i < 16u; ++i)
-      cm = fmaxf(cm, L.cmax[i]);
     VisitRec v;
     v.rot_s = blk_s;
     v.rot_b = blk_b;
-    v.maxcos = cm;
+    v.maxcos = __uint_as_float(L.cmax);
     v.l2ni = L.bnorm[0];
     v.l2nj = L.bnorm[1];
     v.sweep = ctl->sweep;
@@ -604,8 +665,19 @@ __device__ __forceinline__ void pair_visit(unsigned tid, bool present, unsigned 
       atomicAdd(&ctl->split, 1u);
   }
   double *const wo = Wout + (size_t)pi * 1024u;
-  for (unsigned e = tid; e < 1024u; e += 128u)
-    wo[e] = RA(W, e & 31u, e >> 5);
+  for (unsigned e = tid; e < 1024u; e += NT)
+    wo[e] = RA(L.W, e & 31u, e >> 5);
+}
+
+// a skipped visit: no update, the record keeps the last executed visit
+__device__ __forceinline__ void skip_visit(unsigned tid, unsigned pi, unsigned *flags, RunCtl *ctl,
+                                           VisitRec *rec)
+{
+  if (tid == 0u) {
+    flags[pi] = 0u;
+    rec[pi].skips += 1u;
+    atomicAdd(&ctl->skipped, 1u);
+  }
 }
 
 // The plan a visit runs: a visit planned split whose Gram partials come from
@@ -620,33 +692,21 @@ __device__ __forceinline__ uint8_t visit_plan(uint8_t plan, bool split_src)
 // k_gram_split (a standalone Gram launch), so split-planned pairs hold split
 // Grams
 template <bool SORT>
-__global__ __launch_bounds__(128) void k_pair(const uint16_t *__restrict__ pairs,
-                                              const double *__restrict__ part, unsigned nchunk,
-                                              double *__restrict__ Wout, unsigned *__restrict__ flags,
-                                              RunCtl *__restrict__ ctl, VisitRec *__restrict__ rec,
-                                              const uint8_t *__restrict__ skip, int split_src,
-                                              const uint8_t *__restrict__ strat0, unsigned s0steps,
-                                              unsigned nswp, int definite, unsigned nplus)
+__global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
+    const uint16_t *__restrict__ pairs, const double *__restrict__ part, unsigned nchunk,
+    double *__restrict__ Wout, unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
+    VisitRec *__restrict__ rec, const uint8_t *__restrict__ skip, int split_src,
+    const uint8_t *__restrict__ strat0, unsigned s0steps, unsigned nswp, int definite,
+    unsigned nplus)
 {
   __shared__ PairLds L;
-  __shared__ __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
   const unsigned tid = threadIdx.x, pi = blockIdx.x;
   const uint8_t plan = visit_plan(skip ? skip[pi] : PLAN_FP64, split_src != 0);
-  if (plan == PLAN_SKIP) {
-    // skipped visit: no update, the record keeps the last executed visit
-    if (tid == 0u) {
-      flags[pi] = 0u;
-      rec[pi].skips += 1u;
-      atomicAdd(&ctl->skipped, 1u);
-    }
-    return;
-  }
-  // the level-0 table (STRAT0_TAB_BYTES, 16-byte aligned) in one pass of
-  // 16-byte loads
-  if (tid < STRAT0_TAB_BYTES / 16u)
-    reinterpret_cast<uint4 *>(S0)[tid] = reinterpret_cast<const uint4 *>(strat0)[tid];
-  pair_visit<SORT>(tid, true, pi, L, nullptr, pairs, part, nchunk, Wout, flags, ctl, rec, plan, S0,
-                   s0steps, nswp, definite, nplus);
+  if (plan == PLAN_SKIP)
+    skip_visit(tid, pi, flags, ctl, rec);
+  else
+    pair_visit<SORT, PAIR_LANES>(tid, pi, L, pairs, part, nchunk, Wout, flags, ctl, rec, plan,
+                                 strat0, s0steps, nswp, definite, nplus);
 }
 
 // ---------------------------------------------------------------------------
@@ -932,15 +992,15 @@ void k_upgram(double *__restrict__ G, unsigned ldG, const uint16_t *__restrict__
 // Staged sweep: the fused transition of half the quads of step s runs in the
 // same launch as the visits of the pairs of another step whose inputs the
 // previous launch completed, so the visits' latency hides under the fused
-// items' HBM stream.  Workgroups [0, npw) hold two visits each; then come
+// items' HBM stream.  Workgroups [0, npl) hold a visit each; then come
 // the niw item workgroups, j taking items j, j + niw, ..., and, with V,
 // the V workgroups (one (pair, row chunk) update of V per wave).  The
 // launch boundaries order everything else; the arithmetic is that of
 // k_pair / k_upgram / k_update.
-// LDS of a staged workgroup: a fused item's, or two pair visits'
+// LDS of a staged workgroup: a fused item's, or a pair visit's
 union StageLds {
   UpgLds upg;
-  PairLds pair[2];
+  PairLds pair;
 };
 
 template <bool SORT>
@@ -948,25 +1008,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UPGRAM_WAVE
 void k_stage(StageArgs A)
 {
   __shared__ StageLds S;
-  __shared__ __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
   const unsigned tid = threadIdx.x, b = blockIdx.x;
-  if (b < A.npw) {
-    if (tid < STRAT0_TAB_BYTES / 16u)
-      reinterpret_cast<uint4 *>(S0)[tid] = reinterpret_cast<const uint4 *>(A.strat0)[tid];
-    const unsigned half = tid >> 7, ht = tid & 127u, k = 2u * b + half;
-    const bool present = k < A.npl;
-    const unsigned pi = present ? A.plist[k] : 0u;
+  if (b < A.npl) {
+    const unsigned pi = A.plist[b];
     // every Gram a staged launch's visits read comes from fused items (split
     // for split-planned pairs exactly when they form split Grams)
-    const uint8_t plan =
-        visit_plan((present && A.pplan) ? A.pplan[pi] : PLAN_FP64, A.fsplit != 0);
-    pair_visit<SORT>(ht, present, pi, S.pair[half], &S.pair[half ^ 1u].go, A.ppairs, A.ppart,
-                     A.nchunk, A.pW, A.pflags, A.ctl, A.prec, plan, S0, A.s0steps, A.nswp,
-                     A.definite, A.nplus);
+    const uint8_t plan = visit_plan(A.pplan ? A.pplan[pi] : PLAN_FP64, A.fsplit != 0);
+    if (plan == PLAN_SKIP)
+      skip_visit(tid, pi, A.pflags, A.ctl, A.prec);
+    else if (tid < 32u * STAGE_LANES)
+      pair_visit<SORT, STAGE_LANES>(tid, pi, S.pair, A.ppairs, A.ppart, A.nchunk, A.pW, A.pflags, A.ctl,
+                           A.prec, plan, A.strat0, A.s0steps, A.nswp, A.definite, A.nplus);
   }
-  else if (b - A.npw >= A.niw) {
+  else if (b - A.npl >= A.niw) {
     // V items: one (pair, row chunk) per wave
-    const unsigned j = b - A.npw - A.niw;
+    const unsigned j = b - A.npl - A.niw;
     const unsigned v = 4u * j + (tid >> 6);
     if (v < A.nvitems) {
       const unsigned pi = v / A.nchV, c = v - pi * A.nchV;
@@ -987,7 +1043,7 @@ void k_stage(StageArgs A)
       nitems = min(nitems, ld_relaxed(A.qact) * A.nchunk);
       stride = (nitems <= A.islots) ? nitems : (nitems + 1u) / 2u;
     }
-    const unsigned j = b - A.npw;
+    const unsigned j = b - A.npl;
     for (unsigned i = j; i < nitems && j < stride; i += stride) {
       const unsigned qi = i / A.nchunk, c = i - qi * A.nchunk;
       // a copy in registers: through a reference into global memory its
@@ -1228,7 +1284,7 @@ void launch_upgram(hipStream_t s, double *G, unsigned ldG, const uint16_t *pairs
 
 void launch_stage(hipStream_t s, bool sort, const StageArgs &a)
 {
-  const unsigned nb = a.npw + a.niw + a.nvw;
+  const unsigned nb = a.npl + a.niw + a.nvw;
   if (!nb)
     return;
   if (sort)
@@ -1252,10 +1308,10 @@ void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, c
 {
   const int ss = split_src ? 1 : 0;
   if (sort)
-    hipLaunchKernelGGL(k_pair<true>, dim3(np), dim3(128), 0, s, pairs, part, nchunk, W, flags, ctl,
+    hipLaunchKernelGGL(k_pair<true>, dim3(np), dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl,
                        rec, skip, ss, strat0, s0steps, nswp, definite, nplus);
   else
-    hipLaunchKernelGGL(k_pair<false>, dim3(np), dim3(128), 0, s, pairs, part, nchunk, W, flags, ctl,
+    hipLaunchKernelGGL(k_pair<false>, dim3(np), dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl,
                        rec, skip, ss, strat0, s0steps, nswp, definite, nplus);
 }
 

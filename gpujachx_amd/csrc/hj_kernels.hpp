@@ -89,7 +89,7 @@ void launch_upgram(hipStream_t s, double *G, unsigned ldG, const uint16_t *pairs
                    unsigned CH, double *part, const uint8_t *plan_next, bool fsplit);
 
 // One launch of a staged sweep: the visits of a list of pairs of one step
-// (two per workgroup) beside the fused transition of a range of closed quads
+// (one per workgroup) beside the fused transition of a range of closed quads
 // of another (nchunk items per quad) and, when V is accumulated, the update
 // of V by the W of a step whose visits are complete.  The parts touch
 // disjoint data: the visits read Gram partials and write W / flags of their
@@ -99,7 +99,7 @@ void launch_upgram(hipStream_t s, double *G, unsigned ldG, const uint16_t *pairs
 struct StageArgs {
   double *G;
   unsigned ldG;
-  unsigned npl, npw;       // pair visits, their workgroups (ceil(npl / 2))
+  unsigned npl;            // pair visits, one workgroup each
   const uint16_t *plist;   // [npl] pair slots of the visits' step
   const uint16_t *ppairs;  // level-1 pairs of the visits' step
   const double *ppart;     // Gram partials the visits read
