@@ -248,8 +248,8 @@ __device__ void wave_upgram(double *__restrict__ G, unsigned ldG, unsigned nrow,
   d4 z = {0.0, 0.0, 0.0, 0.0};
   d4 g00 = z, g10 = z, g11 = z, h00 = z, h10 = z, h11 = z;
   double xa[8], xb[8];
-  slab_load(G, ldG, 0u, A0, B0, u0, l, xa);
-  slab_load(G, ldG, 0u, A1, B1, u1, l, xb);
+  slab_load<true>(G, ldG, 0u, A0, B0, u0, l, xa);
+  slab_load<true>(G, ldG, 0u, A1, B1, u1, l, xb);
   for (unsigned r = 0u; r < nrow; r += 16u) {
     double ca[8], cb[8];
 #pragma unroll
@@ -258,12 +258,12 @@ __device__ void wave_upgram(double *__restrict__ G, unsigned ldG, unsigned nrow,
       cb[u] = xb[u];
     }
     if (r + 16u < nrow) {
-      slab_load(G, ldG, r + 16u, A0, B0, u0, l, xa);
-      slab_load(G, ldG, r + 16u, A1, B1, u1, l, xb);
+      slab_load<true>(G, ldG, r + 16u, A0, B0, u0, l, xa);
+      slab_load<true>(G, ldG, r + 16u, A1, B1, u1, l, xb);
     }
     d4 t0, t1, t2, t3;
-    slab_compute(G, ldG, r, A0, B0, u0, W0, l, ca, t0, t1, T);
-    slab_compute(G, ldG, r, A1, B1, u1, W1, l, cb, t2, t3, T);
+    slab_compute<true>(G, ldG, r, A0, B0, u0, W0, l, ca, t0, t1, T);
+    slab_compute<true>(G, ldG, r, A1, B1, u1, W1, l, cb, t2, t3, T);
     {
       const d4 X = sel4(Q.x0, t0, t1, t2, t3), Y = sel4(Q.y0, t0, t1, t2, t3);
       gram_fp64_slab(X, Y, g00, g10, g11);

@@ -39,26 +39,35 @@ __device__ __forceinline__ d4 sel4(unsigned i, d4 a, d4 b, d4 c, d4 d)
 #ifndef UPGRAM_WAVES
 #define UPGRAM_WAVES 2
 #endif
-#ifndef UPGRAM_PREFETCH
-#define UPGRAM_PREFETCH 1
-#endif
-// streaming (non-temporal) loads and stores of G in the fused kernel
-#ifndef UPGRAM_NT
-#define UPGRAM_NT 1
-#endif
-#if UPGRAM_NT
-#define UG_LOAD(p) __builtin_nontemporal_load(p)
-#define UG_STORE(v, p) __builtin_nontemporal_store(v, p)
-#else
-#define UG_LOAD(p) (*(p))
-#define UG_STORE(v, p) (*(p) = (v))
-#endif
+// Accesses of G in a fused transition, non-temporal or not.  A matrix that
+// stays in the 256 MB last-level cache from step to step is read from there
+// (4096 x 4096, 134 MB: a step 92 -> 86 us with plain accesses); one that does
+// not only wastes the allocation (8192 x 8192: 1.286 s with non-temporal
+// accesses, 1.294 s without).
+template <bool NT>
+__device__ __forceinline__ double ug_load(const double *p)
+{
+  if constexpr (NT)
+    return __builtin_nontemporal_load(p);
+  else
+    return *p;
+}
+
+template <bool NT>
+__device__ __forceinline__ void ug_store(double v, double *p)
+{
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
 
 // One 16-row slab of a pair, in the update's operand layout (lane l: row
 // l%16 of pair column 4u + l/16, x[u], u = 0..7; 128 contiguous bytes of a
 // column per instruction).  A pair without an update is read the same way
 // and turned into the Gram layout in LDS (slab_compute); la / lb false: no
 // next pair's Gram wants block a / b, nothing to read.
+template <bool NT>
 __device__ __forceinline__ void slab_load(const double *__restrict__ G, unsigned ldG, size_t row,
                                           unsigned a, unsigned b, bool upd, unsigned l, double *x,
                                           bool la = true, bool lb = true)
@@ -68,7 +77,7 @@ __device__ __forceinline__ void slab_load(const double *__restrict__ G, unsigned
     for (unsigned u = 0u; u < 8u; ++u) {
       const unsigned cc = 4u * u + (l >> 4);
       const unsigned gc = (cc < 16u) ? (16u * a + cc) : (16u * b + cc - 16u);
-      x[u] = UG_LOAD(G + (size_t)gc * ldG + row + (l & 15u));
+      x[u] = ug_load<NT>(G + (size_t)gc * ldG + row + (l & 15u));
     }
   }
   else {
@@ -78,7 +87,7 @@ __device__ __forceinline__ void slab_load(const double *__restrict__ G, unsigned
     if (la) {
 #pragma unroll
       for (unsigned u = 0u; u < 4u; ++u)
-        x[u] = UG_LOAD(ia + (size_t)(4u * u) * ldG);
+        x[u] = ug_load<NT>(ia + (size_t)(4u * u) * ldG);
     }
     else {
 #pragma unroll
@@ -88,7 +97,7 @@ __device__ __forceinline__ void slab_load(const double *__restrict__ G, unsigned
     if (lb) {
 #pragma unroll
       for (unsigned u = 0u; u < 4u; ++u)
-        x[4u + u] = UG_LOAD(ib + (size_t)(4u * u) * ldG);
+        x[4u + u] = ug_load<NT>(ib + (size_t)(4u * u) * ldG);
     }
     else {
 #pragma unroll
@@ -98,19 +107,16 @@ __device__ __forceinline__ void slab_load(const double *__restrict__ G, unsigned
   }
 }
 
-#ifndef UPGRAM_LDS_STORE
-#define UPGRAM_LDS_STORE 1
-#endif
 #define LDT 17u  // padded column length of a wave's 16x16 transpose buffer
 
 // stores a 16x16 tile held in the Gram layout (lane l, register r: row
 // 4r + l/16, column l%16) to columns 16 blk .. of G, rows row .. row+15: via
 // the wave's LDS buffer T the lanes write 16 consecutive rows (128 bytes) of
 // one column per instruction
+template <bool NT>
 __device__ __forceinline__ void store_tile(double *__restrict__ G, unsigned ldG, size_t row,
                                            unsigned blk, const d4 &t, unsigned l, double *T)
 {
-#if UPGRAM_LDS_STORE
 #pragma unroll
   for (unsigned r = 0u; r < 4u; ++r)
     T[(l & 15u) * LDT + 4u * r + (l >> 4)] = t[r];
@@ -126,17 +132,12 @@ __device__ __forceinline__ void store_tile(double *__restrict__ G, unsigned ldG,
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (unsigned q = 0u; q < 4u; ++q)
-    UG_STORE(v[q], G + (size_t)(16u * blk + 4u * q + (l >> 4)) * ldG + row + (l & 15u));
-#else
-  double *const o = G + (size_t)(16u * blk + (l & 15u)) * ldG + row + (l >> 4);
-#pragma unroll
-  for (unsigned r = 0u; r < 4u; ++r)
-    o[4u * r] = t[r];
-#endif
+    ug_store<NT>(v[q], G + (size_t)(16u * blk + 4u * q + (l >> 4)) * ldG + row + (l & 15u));
 }
 
 // [G_a G_b] W of the slab, W(k, j) = Wl[k * LDW + j] in LDS, written back;
 // t0, t1: the slab of blocks a, b in the Gram layout
+template <bool NT>
 __device__ __forceinline__ void slab_compute(double *__restrict__ G, unsigned ldG, size_t row,
                                              unsigned a, unsigned b, bool upd, const double *Wl,
                                              unsigned l, const double *x, d4 &t0, d4 &t1, double *T)
@@ -149,8 +150,8 @@ __device__ __forceinline__ void slab_compute(double *__restrict__ G, unsigned ld
       acc0 = mfma(x[u], wr[0], acc0);
       acc1 = mfma(x[u], wr[16], acc1);
     }
-    store_tile(G, ldG, row, a, acc0, l, T);
-    store_tile(G, ldG, row, b, acc1, l, T);
+    store_tile<NT>(G, ldG, row, a, acc0, l, T);
+    store_tile<NT>(G, ldG, row, b, acc1, l, T);
     t0 = acc0;
     t1 = acc1;
   }

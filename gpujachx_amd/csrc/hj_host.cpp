@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <algorithm>
 #include <array>
 #include <vector>
 
@@ -75,10 +76,13 @@ static int g_fact = HJ_FACT_CHOLESKY;
 // least STAGE_MIN_BYTES, 2 wherever they apply
 static int g_stage = 1;
 // Two staged launches cost about 2 max(Th, Tv) + 22 us per step against
-// 2 Th + Tv step by step (Th: half the step's block updates at the HBM
-// rate, Tv ~ 70 us: a visit's latency): they pay once Th exceeds about
-// 46 us, i.e. 4.8e8 bytes read and written per step (N = 8192: 1.07e9;
-// M = 4096, N = 2048 with V: 2.0e8, measured 86.5 -> 104 ms staged).
+// 2 Th + Tv step by step (Th: half the step's block updates at the HBM rate,
+// Tv: a visit, 30 us): they pay from about 4.8e8 bytes read and written per
+// step on, where the Gram's chunks fill their workgroups' four waves (a
+// workgroup of one wave holds the same LDS, and two fit a CU).  Measured, us a
+// step staged / step by step: 4096 x 4096 93 / 86, 8192 x 4096 136 / 148,
+// 8192 x 8192 247 / 252, with V 473 / 521; one wave a chunk: 7168 x 4096 with
+// V 329 / 196, 7680 x 4096 605 / 169.
 constexpr double STAGE_MIN_BYTES = 4.8e8;
 static int g_last_stage = 0;
 static void *g_trace_buf = nullptr;
@@ -332,6 +336,57 @@ static void check_tables(unsigned ncol)
     HJ_DIE("init_strats: level-1 strategy order differs from ncol/16");
 }
 
+// Whether k_step (hj_step.hip) takes a step rather than k_gram, k_pair and
+// k_update: the pair fits its LDS, and its rows of G and V through one CU cost
+// less than two launches.  Measured, us a step (k_step against the three
+// launches): 64 x 64 39 / 44, 256 x 256 35 / 38, with V 37.3 / 37.7,
+// 384 x 256 37.5 / 39.7, 512 x 512 39.1 / 37.2, with V 44 / 37.5.
+static bool step_fits(unsigned nrow, unsigned nrowV)
+{
+  return nrow + nrowV <= STEP_MAX_ROWS;
+}
+
+// One level-1 step in one launch (plain form, Cholesky).
+static void issue_whole_step(hipStream_t s, const Work &w, unsigned step, bool sort, unsigned nswp,
+                             int definite, unsigned nplus, double *dG, unsigned lddG,
+                             unsigned nrow, double *dV, unsigned lddV, unsigned ncol)
+{
+  StepArgs a{};
+  a.G = dG;
+  a.ldG = lddG;
+  a.nrow = nrow;
+  a.V = dV;
+  a.ldV = lddV;
+  a.nrowV = dV ? ncol : 0u;
+  a.pairs = w.d_s1 + (size_t)step * w.np * 2u;
+  a.nsub = w.nchunk;
+  a.SUB = w.CH;
+  a.ctl = w.d_ctl;
+  a.rec = w.d_rec + (size_t)step * w.np;
+  a.strat0 = w.d_s0;
+  a.s0steps = w.s0steps;
+  a.nswp = nswp;
+  a.definite = definite;
+  a.nplus = nplus;
+  launch_step(s, sort, w.np, a);
+}
+
+// V by the W of step st (of its parity's buffers)
+static VItems v_items(const Work &w, unsigned st, double *dV, unsigned lddV, unsigned ncol)
+{
+  VItems v;
+  v.V = dV;
+  v.ld = lddV;
+  v.nrow = ncol;
+  v.ch = w.chV;
+  v.nch = (ncol + w.chV - 1u) / w.chV;
+  v.n = w.np * v.nch;
+  v.pairs = w.d_s1 + (size_t)st * w.np * 2u;
+  v.W = w.W(st & 1u);
+  v.flags = w.flags(st & 1u);
+  return v;
+}
+
 // One level-1 step: Gram partials, pair kernels, block update.
 static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, unsigned nswp,
                        int definite, unsigned nplus, double *dG, unsigned lddG, unsigned nrow,
@@ -352,6 +407,10 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
     if (ev) HIP_CALL(hipEventRecord(ev[3], s));
     return;
   }
+  if (!ev && !skip && step_fits(nrow, dV ? ncol : 0u)) {
+    issue_whole_step(s, w, step, sort, nswp, definite, nplus, dG, lddG, nrow, dV, lddV, ncol);
+    return;
+  }
   launch_gram(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, skip);
   if (split)
     launch_gram_split(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, skip);
@@ -361,6 +420,28 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
   if (ev) HIP_CALL(hipEventRecord(ev[2], s));
   launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags);
   if (ev) HIP_CALL(hipEventRecord(ev[3], s));
+}
+
+// G of up to this many bytes stays in the last-level cache (256 MB) from step
+// to step: plain accesses in the fused transition, else non-temporal ones
+constexpr double UPGRAM_CACHED_BYTES = 2e8;
+
+// Whether a closed transition runs as one launch (k_upgram) rather than as
+// k_update and the next step's k_gram, by the time of each in us.  k_upgram
+// reads and writes G once at 4.7 TB/s, but a wave takes 2.6 us for each
+// 16-row slab of its sub-chunk (56 FP64 MFMAs and their loads), and two
+// workgroups a CU fit; the two launches move half as much again at 5.2 TB/s,
+// no wave of theirs waits on a chain of products like that.  Measured, us a
+// step fused / not: 1024 x 1024 49 / 41, 1280 x 1024 (4 chunks of 320 rows)
+// 87 / 47, 1088 x 1024 (one of 1088) 201 / 56, 2048 x 1024 49 / 52, 4096 x
+// 1024 50 / 56, 2560 x 2048 90 / 57, 4096 x 2048 61 / 74, 5632 x 4096 151 /
+// 135, 4096 x 4096 86 / 110.
+static bool fuse_pays(const Work &w, unsigned nrow, unsigned ncol)
+{
+  const double e = (double)nrow * ncol;
+  const unsigned rounds = (w.np / 2u * w.nchunk + 511u) / 512u;
+  const double chain = 10.0 + 2.6 * rounds * (w.CH / gram_waves(w.CH) / 16u);
+  return std::max(16.0 * e / 4.7e6, chain) < 8.5 + 24.0 * e / 5.2e6;
 }
 
 // One level-2 sweep: a standalone Gram where the previous transition was not
@@ -375,13 +456,16 @@ static unsigned issue_sweep(hipStream_t s, const Work &w, bool sort, unsigned ns
 {
   bool have_gram = false;
   unsigned issued = 0u;
+  const bool whole = !evs && !planned && step_fits(nrow, dV ? ncol : 0u);
+  VItems vlate;  // V's items of the step before (none when profiling)
   for (unsigned st = 0u; st < w.steps; ++st) {
     if (steps_left) {
       if (*steps_left <= 0) return issued;
       --*steps_left;
     }
+    const bool last = st + 1u == w.steps || (steps_left && *steps_left <= 0);
     ++issued;
-    if (g_fact != HJ_FACT_CHOLESKY) {
+    if (g_fact != HJ_FACT_CHOLESKY || whole) {
       if (gram_launched) (*gram_launched)[st] = 0;
       issue_step(s, w, st, sort, nswp, definite, nplus, dG, lddG, nrow, dV, lddV, ncol,
                  evs ? evs + (size_t)4u * st : nullptr, false, false);
@@ -392,6 +476,8 @@ static unsigned issue_sweep(hipStream_t s, const Work &w, bool sort, unsigned ns
     const size_t off = (size_t)st * w.np;
     const uint16_t *pairs = w.d_s1 + off * 2u;
     const uint8_t *plan = planned ? w.d_skip + off : nullptr;
+    double *const W = w.W(st & 1u);
+    unsigned *const flags = w.flags(st & 1u);
     if (ev) HIP_CALL(hipEventRecord(ev[0], s));
     if (!have_gram) {
       launch_gram(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, plan);
@@ -401,21 +487,26 @@ static unsigned issue_sweep(hipStream_t s, const Work &w, bool sort, unsigned ns
     if (ev) HIP_CALL(hipEventRecord(ev[1], s));
     // a split-planned visit holds a split Gram after a standalone Gram
     // launch, and after a fused transition that forms split Grams
-    launch_pair(s, sort, pairs, w.np, w.d_part, w.nchunk, w.d_W, w.d_flags, w.d_ctl, w.d_rec + off,
+    launch_pair(s, sort, pairs, w.np, w.d_part, w.nchunk, W, flags, w.d_ctl, w.d_rec + off,
                 plan, split && (!have_gram || g_fused_split), w.d_s0, w.s0steps, nswp, definite,
-                nplus);
+                nplus, vlate);
     if (ev) HIP_CALL(hipEventRecord(ev[2], s));
-    const bool fused = (st + 1u < w.steps) && w.fuse[st] &&
-                       !(steps_left && *steps_left <= 0);
-    if (fused) {
-      launch_upgram(s, dG, lddG, pairs, w.d_W, w.d_flags, w.d_quads + (size_t)st * (w.np / 2u),
+    vlate = VItems();
+    // (the split form's visits follow which Grams are fused: always as before)
+    const bool fused = !last && w.fuse[st] && (split || fuse_pays(w, nrow, ncol));
+    // V by this step's W rides in the next step's visits' launch (W and the
+    // flags are kept by step parity), or, at the end, goes with G
+    const bool vnow = dV && (last || ev);
+    if (fused)
+      launch_upgram(s, dG, lddG, pairs, W, flags, w.d_quads + (size_t)st * (w.np / 2u),
                     w.np / 2u, w.nchunk, w.CH, w.d_part,
-                    planned ? w.d_skip + off + w.np : nullptr, split && g_fused_split);
-      if (dV)
-        launch_update(s, dG, lddG, 0u, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags);
-    }
-    else
-      launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags);
+                    planned ? w.d_skip + off + w.np : nullptr, split && g_fused_split,
+                    sizeof(double) * (double)nrow * ncol > UPGRAM_CACHED_BYTES);
+    if (!fused || vnow)
+      launch_update(s, dG, lddG, fused ? 0u : nrow, w.chG, vnow ? dV : nullptr, lddV, ncol, w.chV,
+                    pairs, w.np, W, flags);
+    if (dV && !vnow)
+      vlate = v_items(w, st, dV, lddV, ncol);
     if (ev) HIP_CALL(hipEventRecord(ev[3], s));
     have_gram = fused;
   }
@@ -500,18 +591,7 @@ static unsigned issue_sweep_staged(hipStream_t s, const Work &w, bool sort, unsi
   // V by the W of step st (all its visits done: those of P_A(st) in Y_{st-1},
   // of P_B(st) in X_st), in Y_st
   auto vupdate = [&](StageArgs &x, unsigned st) {
-    if (!dV)
-      return;
-    x.V = dV;
-    x.ldV = lddV;
-    x.nrowV = ncol;
-    x.chV = w.chV;
-    x.nchV = (ncol + w.chV - 1u) / w.chV;
-    x.nvitems = np * x.nchV;
-    x.nvw = (x.nvitems + 3u) / 4u;
-    x.vpairs = w.d_s1 + (size_t)st * np * 2u;
-    x.vW = w.W(st & 1u);
-    x.vflags = w.flags(st & 1u);
+    if (dV) x.v = v_items(w, st, dV, lddV, ncol);
   };
   auto fused = [&](StageArgs &x, unsigned st, unsigned q0, unsigned n) {
     x.upairs = w.d_s1 + (size_t)st * np * 2u;
@@ -604,8 +684,9 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   Work w;
   w.alloc(nrow, ncol, full_svd);
   const double step_bytes = 512.0 * (ncol / 32u) * ((double)nrow + (full_svd ? ncol : 0u));
-  const bool staged = g_stage && (g_stage == 2 || step_bytes >= STAGE_MIN_BYTES) &&
-                      g_step_limit <= 0 && g_fact == HJ_FACT_CHOLESKY && w.build_stage();
+  const bool stage_pays = step_bytes >= STAGE_MIN_BYTES && gram_waves(w.CH) == GRAM_WAVES;
+  const bool staged = g_stage && (g_stage == 2 || stage_pays) && g_step_limit <= 0 &&
+                      g_fact == HJ_FACT_CHOLESKY && w.build_stage();
   g_last_stage = staged ? 1 : 0;
   if (full_svd)
     launch_initV(s, dV, 0u, ncol, lddV);

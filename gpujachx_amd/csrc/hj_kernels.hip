@@ -15,6 +15,7 @@
 #include "hj_device.hpp"
 #include "hj_fused.hpp"
 #include "hj_kernels.hpp"
+#include "hj_visit.hpp"
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
@@ -101,6 +102,79 @@ __global__ __launch_bounds__(256, 2) void k_gram(const double *__restrict__ G, u
       o[512u + r] = a11[r];
     }
   }
+}
+
+// The same partials where the sub-chunks are too few to fill the chip (a few
+// pairs, or a row count without powers of two: 1344 = 21 x 64 rows are one
+// chain of 336 MFMAs a tile): four waves a sub-chunk, three of them with one
+// tile's chain each, all four reading 64-row panels of the pair's columns
+// into LDS two panels ahead.  Workgroup (pair, chunk), NW sub-chunks.  One
+// wave with all three chains and one 32-row group in flight took 46 us for
+// 1344 x 672.
+constexpr unsigned GT_LD = 66u;  // padded panel column: operands in 32 different banks
+template <unsigned NW>
+__global__ __launch_bounds__(256u * NW) void k_gram_tiles(const double *__restrict__ G, unsigned ldG,
+                                                          const uint16_t *__restrict__ pairs,
+                                                          unsigned nchunk, unsigned CH,
+                                                          double *__restrict__ part,
+                                                          const uint8_t *__restrict__ skip)
+{
+  __shared__ double P[NW][2][32u * GT_LD];
+  __shared__ d4 red[3][NW > 1u ? NW - 1u : 1u][64];
+  const unsigned tid = threadIdx.x, l = tid & 63u, sub = tid >> 8, w = (tid >> 6) & 3u;
+  const unsigned pi = blockIdx.x / nchunk, c = blockIdx.x - pi * nchunk;
+  if (skip && skip[pi])
+    return;
+  const unsigned iBlk = pairs[2u * pi], jBlk = pairs[2u * pi + 1u];
+  const unsigned SUB = CH / NW;
+  // wave w of the sub-chunk reads columns w, w + 4, ... of the pair, row l of
+  // a panel
+  const size_t r0 = (size_t)c * CH + (size_t)sub * SUB + l;
+  const double *const gi = G + (size_t)(16u * iBlk + w) * ldG + r0;
+  const double *const gj = G + (size_t)(16u * jBlk + w) * ldG + r0;
+  const size_t cs = (size_t)4u * ldG;
+  double x[8];
+#pragma unroll
+  for (unsigned k = 0u; k < 4u; ++k) {
+    x[k] = gi[k * cs];
+    x[4u + k] = gj[k * cs];
+  }
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  // tile 0: block i with itself, 1: block j with block i, 2: j with itself
+  const unsigned ox = ((w ? 16u : 0u) + (l & 15u)) * GT_LD + (l >> 4);
+  const unsigned oy = ((w == 2u ? 16u : 0u) + (l & 15u)) * GT_LD + (l >> 4);
+#pragma unroll 1
+  for (unsigned g = 0u, b = 0u; g < SUB; g += 64u, b ^= 1u) {
+    lds_f64 *const p = (lds_f64 *)P[sub][b];
+#pragma unroll
+    for (unsigned k = 0u; k < 8u; ++k)
+      p[(w + 4u * k) * GT_LD + l] = x[k];
+    if (g + 64u < SUB) {
+#pragma unroll
+      for (unsigned k = 0u; k < 4u; ++k) {
+        x[k] = gi[k * cs + g + 64u];
+        x[4u + k] = gj[k * cs + g + 64u];
+      }
+    }
+    // (two buffers: a wave writes this one again only after the next
+    // panel's barrier, when every wave has left it)
+    __syncthreads();
+    if (w < 3u) {
+#pragma unroll
+      for (unsigned r = 0u; r < 64u; r += 4u)
+        acc = mfma(p[ox + r], p[oy + r], acc);
+    }
+  }
+  if (NW > 1u) {
+    if (sub && w < 3u) red[w][sub - 1u][l] = acc;
+    __syncthreads();
+    if (sub || w >= 3u)
+      return;
+    for (unsigned v = 1u; v < NW; ++v)
+      acc = acc + red[w][v - 1u][l];
+  }
+  if (w < 3u)
+    *reinterpret_cast<d4 *>(part + (size_t)blockIdx.x * 768u + 256u * w + 4u * l) = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -313,372 +387,13 @@ __global__ __launch_bounds__(256, 2) void k_gram_split(const double *__restrict_
 // R and W live in LDS, column-major with a padded leading dimension.
 // Cholesky: one wave (chol32_wave).  Inner Jacobi: pair_visit.
 
-#define LDR 33u
-#define RA(A, r, c) (A)[(c) * LDR + (r)]
+// (hj_visit.hpp)
+
 #define F32(A, r, c) (A)[(c) * 32u + (r)]
-// lanes per pivot pair of level-0 (see pair_visit) in k_pair and k_stage
+// lanes per pivot pair of level-0 (see visit_core) in k_pair and k_stage
 constexpr unsigned PAIR_LANES = 16u;
 constexpr unsigned STAGE_LANES = 8u;
-
-// LDS of one pair visit
-struct PairLds {
-  double R[32u * LDR];
-  double W[32u * LDR];
-  double cholcol[64];
-  double diag[32];        // the Gram's diagonal
-  double rot[2][16][4];   // per step parity and pivot pair: c, t, |Apq|, |p| |q|
-  unsigned act[2][16];    // ... what happens to its columns (ACT_*)
-  unsigned cs[2], cb[2];  // rotations of an inner sweep, by its parity
-  unsigned cmax;          // bits of the largest cosine of the first inner sweep
-  float bnorm[2];
-  int chol_ok;
-  int swp;    // a pivot pair was swapped by the sort rule
-  __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
-};
-
-// what a step does to a pivot pair's columns of R and W
-constexpr unsigned ACT_ROT = 1u;    // rotated
-constexpr unsigned ACT_CROSS = 2u;  // the results change places (with ACT_ROT or alone)
-constexpr unsigned ACT_TRIG = 4u;   // the rotation is trigonometric
-
-// The columns of M (R or W) of a pivot pair after the step: lane l of the
-// pair's group holds rows row + LANES i as P[i], Q[i]; ap, aq: the first of
-// them in LDS.  Without branches: an untouched pair is stored as it is.
-template <unsigned LANES, bool HYP>
-__device__ __forceinline__ void apply_pair(lds_f64 *ap, lds_f64 *aq, const double *P,
-                                           const double *Q, bool rot, bool cross, bool trig,
-                                           double c, double t)
-{
-  constexpr unsigned ROWS = 32u / LANES;
-  lds_f64 *const A = cross ? aq : ap, *const B = cross ? ap : aq;
-  const double t_ = (!HYP || trig) ? -t : t;
-  double a[ROWS], b[ROWS];
-#pragma unroll
-  for (unsigned i = 0u; i < ROWS; ++i) {
-    // big rotation: scale by c; otherwise c == 1 exactly (dev_rot), and
-    // c * x is x
-    const double x = pin(c * __fma_rn(t_, Q[i], P[i])), y = pin(c * __fma_rn(t, P[i], Q[i]));
-    a[i] = rot ? x : P[i];
-    b[i] = rot ? y : Q[i];
-  }
-#pragma unroll
-  for (unsigned i = 0u; i < ROWS; ++i) {
-    A[LANES * i] = a[i];
-    B[LANES * i] = b[i];
-  }
-}
-
-// LDS column of a pivot index, fetched ahead: the operands of the next step's
-// reads are ready when its barrier opens
-__device__ __forceinline__ unsigned pinu(unsigned x)
-{
-  asm volatile("" : "+v"(x));
-  return x;
-}
-
-// One level-0 sweep on R: lane r of group y takes pivot pair y of every step.
-// Counts its rotations and leaves each step's (c, t, ...) for the W waves.
-template <bool SORT, unsigned LANES, bool HYP>
-__device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
-                                         int def, unsigned npos, unsigned &my_s, unsigned &my_b,
-                                         bool &swapped)
-{
-  constexpr unsigned ROWS = 32u / LANES;
-  lds_f64 *const M = (lds_f64 *)L.R + row_of(r);
-  const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
-  // sorted definite pairs: columns by decreasing D for J = I, by increasing
-  // D for J = -I: descending in D xor this sign
-  const uint64_t neg0 = (!HYP && def < 0) ? 0x8000000000000000ull : 0ull;
-  unsigned pq = S0[0];
-  unsigned p = pq & 255u, q = pq >> 8, op = p * LDR, oq = q * LDR;
-#pragma unroll 1
-  for (unsigned step = 0u; step < s0steps; ++step) {
-    lds_f64 *const ap = M + op, *const aq = M + oq;
-    double Gp[ROWS], Gq[ROWS];
-#pragma unroll
-    for (unsigned i = 0u; i < ROWS; ++i) {
-      Gp[i] = ap[LANES * i];
-      Gq[i] = aq[LANES * i];
-    }
-    pq = S0[16u * min(step + 1u, s0steps - 1u)];
-    bool trig = true, inorder = SORT;
-    uint64_t neg = neg0;
-    if (HYP) {
-      const bool pp = p < npos, qp = q < npos;
-      trig = (pp == qp);
-      neg = pp ? 0ull : 0x8000000000000000ull;
-      inorder = SORT & trig;
-    }
-    double Dp, Dq, Apq;
-    dots3<LANES>(Gp, Gq, Dp, Dq, Apq);
-    // the rotation on every lane; only a transforming pair uses it
-    double c, t, Dpq_;
-    const bool big = rot_quad<HYP>(trig, Apq, Dp, Dq, r, c, t, Dpq_);
-    const double Apq_ = fabs(Apq);
-    const bool transf = !(Apq_ < (Dpq_ * MYTOL));
-    bool cross = false;
-    if (SORT) {
-      // rotated: unless in order afterwards; not rotated: when out of order
-      const double Ep = pin(__fma_rn(t, Apq, Dp)), Eq = pin(__fma_rn(-t, Apq, Dq));
-      const bool ge = u2d(d2u(Ep) ^ neg) >= u2d(d2u(Eq) ^ neg);
-      const bool lt = u2d(d2u(Dp) ^ neg) < u2d(d2u(Dq) ^ neg);
-      cross = inorder & ((transf & !ge) | (!transf & lt));
-      swapped = swapped | (cross & !transf);
-    }
-    apply_pair<LANES, HYP>(ap, aq, Gp, Gq, transf, cross, trig, c, t);
-    if (r == 0u) {
-      double *const o = L.rot[step & 1u][y];
-      o[0] = c;
-      o[1] = t;
-      o[2] = Apq_;
-      o[3] = Dpq_;
-      L.act[step & 1u][y] = (transf ? ACT_ROT : 0u) | (cross ? ACT_CROSS : 0u) |
-                            (trig ? ACT_TRIG : 0u);
-    }
-    my_s += transf ? 1u : 0u;
-    my_b += (transf & big) ? 1u : 0u;
-    p = pq & 255u;
-    q = pq >> 8;
-    op = pinu(p * LDR);
-    oq = pinu(q * LDR);
-    __syncthreads();
-  }
-}
-
-// The same sweep's rotations applied to W, each step's between the barrier
-// that ends it on the R waves and the next; with cosines, the largest
-// |Apq| / (|p| |q|).
-template <unsigned LANES>
-__device__ __forceinline__ void level0_w(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
-                                         bool cosines)
-{
-  constexpr unsigned ROWS = 32u / LANES;
-  lds_f64 *const M = (lds_f64 *)L.W + row_of(r);
-  const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
-  double my_cos = 0.0;
-#pragma unroll 1
-  for (unsigned step = 0u; step < s0steps; ++step) {
-    const unsigned pq = S0[16u * step];
-    const unsigned op = pinu((pq & 255u) * LDR), oq = pinu((pq >> 8) * LDR);
-    __syncthreads();
-    lds_f64 *const ap = M + op, *const aq = M + oq;
-    double P[ROWS], Q[ROWS];
-#pragma unroll
-    for (unsigned i = 0u; i < ROWS; ++i) {
-      P[i] = ap[LANES * i];
-      Q[i] = aq[LANES * i];
-    }
-    const double *const o = L.rot[step & 1u][y];
-    const unsigned act = L.act[step & 1u][y];
-    const double cn = o[2], cd = o[3];
-    apply_pair<LANES, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
-                            (act & ACT_TRIG) != 0u, o[0], o[1]);
-    if (cosines)
-      my_cos = fmax(my_cos, (cd > 0.0) ? cn / cd : 0.0);
-  }
-  // (a nonnegative float's bits order as the float does)
-  if (cosines && r == 0u)
-    atomicMax(&L.cmax, __float_as_uint((float)my_cos));
-}
-
-// One pair visit by the 32 LANES threads of a workgroup (LANES = 16 or 8
-// lanes per pivot pair).  The first half of the waves keeps R: per level-0
-// step the dot products, the rotation, the update of R.  The other half
-// applies the same rotations to W one step behind, from the step's (c, t) in
-// LDS, and does the bookkeeping (the largest cosine), so that neither is in
-// the chain of the 31 dependent steps; a barrier per step is all that orders
-// the two (the pivot pairs of a step touch disjoint columns).  A step is
-// bound by that chain -- LDS reads, five reduction levels, division, square
-// root, division, reciprocal root, the update and the barrier -- and by the
-// instructions one wave issues on it, so the lanes share the square roots
-// (rot_quad), the rows are laid out for one-move reduction levels (row_of)
-// and the next step's pivot indices are fetched ahead.
-//
-// Measured (cycles of 2.4 GHz, 512 x 256 in k_pair's LANES = 16): partial sums
-// 3.3K, Cholesky 11.4K (23.4K with the column's reads waited for one by one),
-// a level-0 sweep 46K = 1490 a step, end 3K; 27 us a visit, 29 us a launch,
-// where two waves of 8 lanes a pair, each with both R and W, took 51 us.
-// LANES = 8 (half the waves): 33.5 us, 4: 42 us.  k_stage takes 8, the
-// largest that its 256-thread workgroups hold; its items set its pace, and
-// one visit a workgroup there times the same as two (8192 x 8192: 1.29 s).
-// plan: the visit's plan (PLAN_FP64 without a plan); not PLAN_SKIP.
-template <bool SORT, unsigned LANES>
-__device__ __forceinline__ void pair_visit(unsigned tid, unsigned pi, PairLds &L,
-                                           const uint16_t *__restrict__ pairs,
-                                           const double *__restrict__ part, unsigned nchunk,
-                                           double *__restrict__ Wout, unsigned *__restrict__ flags,
-                                           RunCtl *__restrict__ ctl, VisitRec *__restrict__ rec,
-                                           uint8_t plan, const uint8_t *__restrict__ strat0,
-                                           unsigned s0steps, unsigned nswp, int definite,
-                                           unsigned nplus)
-{
-  constexpr unsigned NT = 32u * LANES, ROWS = 32u / LANES;
-  const unsigned iBlk = pairs[2u * pi], jBlk = pairs[2u * pi + 1u];
-
-  // local J structure, share/device_code_nosort_accumV.hpp:53-76
-  bool hyp = false;
-  int def = definite;
-  unsigned npos = 0u;
-  if (!definite) {
-    const unsigned ifc0 = iBlk * 16u, ifc1 = jBlk * 16u;
-    if (nplus <= ifc0) { npos = 0u; def = -1; }
-    else if (nplus <= ifc0 + 16u) { npos = nplus - ifc0; def = 0; }
-    else if (nplus <= ifc1) { npos = 16u; def = 0; }
-    else if (nplus <= ifc1 + 16u) { npos = 16u + (nplus - ifc1); def = 0; }
-    else { npos = 32u; def = +1; }
-    hyp = (def == 0);
-  }
-
-  {
-    // sum of the chunk partials in chunk order: a thread's entries with all
-    // their chunk loads in flight together (one memory round trip)
-    const double *const pp = part + (size_t)pi * nchunk * 768u;
-    constexpr unsigned NE = (768u + NT - 1u) / NT;
-    double v[NE][MAX_GRAM_CHUNKS];
-#pragma unroll
-    for (unsigned q = 0u; q < NE; ++q)
-#pragma unroll
-      for (unsigned c = 0u; c < MAX_GRAM_CHUNKS; ++c)
-        if (c < nchunk && tid + NT * q < 768u) v[q][c] = pp[(size_t)c * 768u + tid + NT * q];
-    // the level-0 table, 16 bytes a thread, and W = I while they arrive
-    if (tid < STRAT0_TAB_BYTES / 16u)
-      reinterpret_cast<uint4 *>(L.S0)[tid] = reinterpret_cast<const uint4 *>(strat0)[tid];
-    for (unsigned e = tid; e < 1024u; e += NT)
-      RA(L.W, e & 31u, e >> 5) = ((e & 31u) == (e >> 5)) ? 1.0 : 0.0;
-    if (tid == 0u) {
-      L.swp = 0;
-      L.cmax = 0u;
-      L.cs[0] = L.cb[0] = 0u;
-    }
-#pragma unroll
-    for (unsigned q = 0u; q < NE; ++q) {
-      const unsigned e = tid + NT * q;
-      if (e >= 768u) break;
-      const unsigned tile = e >> 8;
-      double s = v[q][0];
-#pragma unroll
-      for (unsigned c = 1u; c < MAX_GRAM_CHUNKS; ++c)
-        if (c < nchunk) s = s + v[q][c];
-      const unsigned l = (e >> 2) & 63u, r = e & 3u;
-      const unsigned i = 4u * r + (l >> 4), j = l & 15u;
-      const unsigned row = (tile == 0u) ? i : (16u + i);
-      const unsigned col = (tile == 2u) ? (16u + j) : j;
-      RA(L.R, row, col) = s;
-      if (row == col) L.diag[row] = s;
-    }
-  }
-  __syncthreads();
-  // Cholesky, share/device_code_common_Cholesky.hpp:58-158 (USE_RSQRT):
-  // column k scaled by rsqrt(A(k,k)), diagonal sqrt(A(k,k)), then
-  // A(x,j) = fma(-A(x,k), A(j,k), A(x,j)) for x >= j > k; R = L^T.
-  if (tid < 64u) {
-    // a Gram from the split products may miss positive definiteness (nearly
-    // dependent columns): then no update, FP64 at the next visit
-    const bool ok = chol32_wave<LDR>(L.R, L.cholcol, tid, plan == PLAN_SPLIT);
-    if (tid == 0u) L.chol_ok = ok ? 1 : 0;
-  }
-  else if (tid < 66u) {
-    // squared Frobenius norms of the two blocks, for the visit record
-    double sn = 0.0;
-    for (unsigned k = 0u; k < 16u; ++k)
-      sn = sn + L.diag[16u * (tid - 64u) + k];
-    L.bnorm[tid - 64u] = (float)log2(sn);
-  }
-  __syncthreads();
-  if (plan == PLAN_SPLIT && !L.chol_ok) {
-    if (tid == 0u) {
-      flags[pi] = 0u;
-      VisitRec v;
-      v.rot_s = 0u;
-      v.rot_b = 0u;
-      v.maxcos = 1.0f;
-      v.l2ni = L.bnorm[0];
-      v.l2nj = L.bnorm[1];
-      v.sweep = ctl->sweep;
-      v.skips = 0u;
-      v.flags = REC_SPLIT | REC_SPLIT_FAIL;
-      rec[pi] = v;
-      atomicAdd(&ctl->split, 1u);
-    }
-    return;
-  }
-
-  // Inner Jacobi: share/device_code_nosort.hpp:4-222 (SORT false),
-  // share/device_code_cdsort_KISS.hpp:4-260 and share/device_code_cdsort.hpp:25-167
-  // (SORT true).
-  const bool onR = tid < NT / 2u;  // this wave's matrix: R or W
-  const unsigned ht = tid & (NT / 2u - 1u);
-  const unsigned y = ht / LANES, r = ht & (LANES - 1u);
-  unsigned blk_s = 0u, blk_b = 0u;
-  for (unsigned swp = 0u; swp < nswp; ++swp) {
-    unsigned my_s = 0u, my_b = 0u;
-    bool swapped = false;
-    if (!onR)
-      level0_w<LANES>(L, y, r, s0steps, swp == 0u);
-    else if (hyp)
-      level0_r<SORT, LANES, true>(L, y, r, s0steps, def, npos, my_s, my_b, swapped);
-    else
-      level0_r<SORT, LANES, false>(L, y, r, s0steps, def, npos, my_s, my_b, swapped);
-    // every lane of a pair's group holds its counts
-    if (onR && r == 0u && my_s) {
-      atomicAdd(&L.cs[swp & 1u], my_s);
-      atomicAdd(&L.cb[swp & 1u], my_b);
-    }
-    if (onR && swapped)
-      L.swp = 1;
-    __syncthreads();
-    const unsigned swp_s = L.cs[swp & 1u];
-    // (the other parity was read before this sweep's steps)
-    if (tid == 0u)
-      L.cs[(swp + 1u) & 1u] = 0u;
-    if (tid == 64u)
-      L.cb[(swp + 1u) & 1u] = 0u;
-    if (!swp_s)
-      break;
-    blk_s += swp_s;
-    blk_b += L.cb[swp & 1u];
-  }
-
-  // convergence counter, share/device_code_nosort.hpp:94-103
-  if (tid == 0u) {
-    unsigned long long *const cvg = &ctl->cvg;
-    if (blk_s) {
-      if (blk_b)
-        atomicAdd(cvg, (((unsigned long long)blk_b) << 32) | blk_s);
-      else
-        atomicAdd(reinterpret_cast<unsigned *>(cvg), blk_s);
-    }
-    // the block update is left out exactly when W is the identity (no
-    // rotation, no swap)
-    flags[pi] = (blk_s || L.swp) ? 1u : 0u;
-    VisitRec v;
-    v.rot_s = blk_s;
-    v.rot_b = blk_b;
-    v.maxcos = __uint_as_float(L.cmax);
-    v.l2ni = L.bnorm[0];
-    v.l2nj = L.bnorm[1];
-    v.sweep = ctl->sweep;
-    v.skips = 0u;
-    v.flags = (plan == PLAN_SPLIT) ? REC_SPLIT : 0u;
-    rec[pi] = v;
-    if (plan == PLAN_SPLIT)
-      atomicAdd(&ctl->split, 1u);
-  }
-  double *const wo = Wout + (size_t)pi * 1024u;
-  for (unsigned e = tid; e < 1024u; e += NT)
-    wo[e] = RA(L.W, e & 31u, e >> 5);
-}
-
-// a skipped visit: no update, the record keeps the last executed visit
-__device__ __forceinline__ void skip_visit(unsigned tid, unsigned pi, unsigned *flags, RunCtl *ctl,
-                                           VisitRec *rec)
-{
-  if (tid == 0u) {
-    flags[pi] = 0u;
-    rec[pi].skips += 1u;
-    atomicAdd(&ctl->skipped, 1u);
-  }
-}
+constexpr unsigned GRAM_TILES_MAX = 512u;
 
 // The plan a visit runs: a visit planned split whose Gram partials come from
 // the FP64 Gram (a fused transition's that forms FP64 Grams only) is an FP64
@@ -686,27 +401,6 @@ __device__ __forceinline__ void skip_visit(unsigned tid, unsigned pi, unsigned *
 __device__ __forceinline__ uint8_t visit_plan(uint8_t plan, bool split_src)
 {
   return (plan == PLAN_SPLIT && !split_src) ? PLAN_FP64 : plan;
-}
-
-// split_src: the partials of this launch's pairs came from k_gram followed by
-// k_gram_split (a standalone Gram launch), so split-planned pairs hold split
-// Grams
-template <bool SORT>
-__global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
-    const uint16_t *__restrict__ pairs, const double *__restrict__ part, unsigned nchunk,
-    double *__restrict__ Wout, unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
-    VisitRec *__restrict__ rec, const uint8_t *__restrict__ skip, int split_src,
-    const uint8_t *__restrict__ strat0, unsigned s0steps, unsigned nswp, int definite,
-    unsigned nplus)
-{
-  __shared__ PairLds L;
-  const unsigned tid = threadIdx.x, pi = blockIdx.x;
-  const uint8_t plan = visit_plan(skip ? skip[pi] : PLAN_FP64, split_src != 0);
-  if (plan == PLAN_SKIP)
-    skip_visit(tid, pi, flags, ctl, rec);
-  else
-    pair_visit<SORT, PAIR_LANES>(tid, pi, L, pairs, part, nchunk, Wout, flags, ctl, rec, plan,
-                                 strat0, s0steps, nswp, definite, nplus);
 }
 
 // ---------------------------------------------------------------------------
@@ -795,6 +489,51 @@ __global__ __launch_bounds__(64) void k_update(double *__restrict__ G, unsigned 
   update_rows(M, ld, r0, r1, pairs[2u * pi], pairs[2u * pi + 1u], Wbuf + (size_t)pi * 1024u, l);
 }
 
+// The update of V by the W of a step whose visits are complete: (pair, row
+// chunk) items, one per wave of workgroup b.  V is read by no visit, so it
+// rides in a launch that leaves CUs idle: a later step's visits, or a staged
+// launch.
+template <unsigned WAVES>
+__device__ __forceinline__ void v_item(const VItems &V, unsigned b, unsigned tid)
+{
+  const unsigned v = WAVES * b + (tid >> 6);
+  if (v >= V.n)
+    return;
+  const unsigned pi = v / V.nch, c = v - pi * V.nch;
+  if (!V.flags[pi])
+    return;
+  const unsigned r0 = c * V.ch;
+  update_rows(V.V, V.ld, r0, min(r0 + V.ch, V.nrow), V.pairs[2u * pi], V.pairs[2u * pi + 1u],
+              V.W + (size_t)pi * 1024u, tid & 63u);
+}
+
+// Workgroups [0, np): the visits; then V's items of the step before (V.n of
+// them, none without V).
+// split_src: the partials of this launch's pairs came from k_gram followed by
+// k_gram_split (a standalone Gram launch), so split-planned pairs hold split
+// Grams
+template <bool SORT>
+__global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
+    const uint16_t *__restrict__ pairs, const double *__restrict__ part, unsigned nchunk,
+    double *__restrict__ Wout, unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
+    VisitRec *__restrict__ rec, const uint8_t *__restrict__ skip, int split_src,
+    const uint8_t *__restrict__ strat0, unsigned s0steps, unsigned nswp, int definite,
+    unsigned nplus, unsigned np, VItems V)
+{
+  __shared__ PairLds L;
+  const unsigned tid = threadIdx.x, pi = blockIdx.x;
+  if (pi >= np) {
+    v_item<PAIR_LANES / 2u>(V, pi - np, tid);
+    return;
+  }
+  const uint8_t plan = visit_plan(skip ? skip[pi] : PLAN_FP64, split_src != 0);
+  if (plan == PLAN_SKIP)
+    skip_visit(tid, pi, flags, ctl, rec);
+  else
+    pair_visit<SORT, PAIR_LANES>(tid, pi, L, pairs, part, nchunk, Wout, flags, ctl, rec, plan,
+                                 strat0, s0steps, nswp, definite, nplus);
+}
+
 // ---------------------------------------------------------------------------
 // Column norms, G -> U, D = +-||g||^2 (share/device_code_common.hpp:187-219).
 // One wave per column: lane l sums rows l, l+64, ... by fma, then an xor
@@ -850,6 +589,7 @@ struct UpgLds {
 // gets its Gram from the updated slabs in registers: the split Gram (the
 // slab arithmetic and partial layout of k_gram_split) when fsplit is set and
 // the pair is planned split, else the FP64 Gram.
+template <bool NT>
 __device__ __forceinline__ void upgram_item(UpgLds &S, double *__restrict__ G, unsigned ldG,
                                             const uint16_t *__restrict__ pairs,
                                             const double *__restrict__ Wbuf,
@@ -889,51 +629,22 @@ __device__ __forceinline__ void upgram_item(UpgLds &S, double *__restrict__ G, u
   d4 g00 = z, g10 = z, g11 = z, h00 = z, h10 = z, h11 = z;
   if (w < nw) {
     double xa[8], xb[8];
-#if UPGRAM_PREFETCH
-    slab_load(G, ldG, rbeg, A0, B0, u0, l, xa, nt0, nt1);
-    slab_load(G, ldG, rbeg, A1, B1, u1, l, xb, nt2, nt3);
-#endif
-#if UPGRAM_PREFETCH >= 2
-    // a second slab in flight
-    double ya[8], yb[8];
-    if (16u < SUB) {
-      slab_load(G, ldG, rbeg + 16u, A0, B0, u0, l, ya, nt0, nt1);
-      slab_load(G, ldG, rbeg + 16u, A1, B1, u1, l, yb, nt2, nt3);
-    }
-#endif
+    slab_load<NT>(G, ldG, rbeg, A0, B0, u0, l, xa, nt0, nt1);
+    slab_load<NT>(G, ldG, rbeg, A1, B1, u1, l, xb, nt2, nt3);
     for (unsigned g = 0u; g < SUB; g += 16u) {
       d4 t0, t1, t2, t3;
-#if UPGRAM_PREFETCH
       double ca[8], cb[8];
 #pragma unroll
       for (unsigned u = 0u; u < 8u; ++u) {
         ca[u] = xa[u];
         cb[u] = xb[u];
       }
-#if UPGRAM_PREFETCH >= 2
-#pragma unroll
-      for (unsigned u = 0u; u < 8u; ++u) {
-        xa[u] = ya[u];
-        xb[u] = yb[u];
-      }
-      if (g + 32u < SUB) {
-        slab_load(G, ldG, rbeg + g + 32u, A0, B0, u0, l, ya, nt0, nt1);
-        slab_load(G, ldG, rbeg + g + 32u, A1, B1, u1, l, yb, nt2, nt3);
-      }
-#else
       if (g + 16u < SUB) {
-        slab_load(G, ldG, rbeg + g + 16u, A0, B0, u0, l, xa, nt0, nt1);
-        slab_load(G, ldG, rbeg + g + 16u, A1, B1, u1, l, xb, nt2, nt3);
+        slab_load<NT>(G, ldG, rbeg + g + 16u, A0, B0, u0, l, xa, nt0, nt1);
+        slab_load<NT>(G, ldG, rbeg + g + 16u, A1, B1, u1, l, xb, nt2, nt3);
       }
-#endif
-      slab_compute(G, ldG, rbeg + g, A0, B0, u0, S.Wl[0], l, ca, t0, t1, Tw);
-      slab_compute(G, ldG, rbeg + g, A1, B1, u1, S.Wl[1], l, cb, t2, t3, Tw);
-#else
-      slab_load(G, ldG, rbeg + g, A0, B0, u0, l, xa, nt0, nt1);
-      slab_load(G, ldG, rbeg + g, A1, B1, u1, l, xb, nt2, nt3);
-      slab_compute(G, ldG, rbeg + g, A0, B0, u0, S.Wl[0], l, xa, t0, t1, Tw);
-      slab_compute(G, ldG, rbeg + g, A1, B1, u1, S.Wl[1], l, xb, t2, t3, Tw);
-#endif
+      slab_compute<NT>(G, ldG, rbeg + g, A0, B0, u0, S.Wl[0], l, ca, t0, t1, Tw);
+      slab_compute<NT>(G, ldG, rbeg + g, A1, B1, u1, S.Wl[1], l, cb, t2, t3, Tw);
       if (pn0 != PLAN_SKIP) {
         const d4 X = sel4(Q.x0, t0, t1, t2, t3), Y = sel4(Q.y0, t0, t1, t2, t3);
         if (sp0)
@@ -975,6 +686,7 @@ __device__ __forceinline__ void upgram_item(UpgLds &S, double *__restrict__ G, u
   }
 }
 
+template <bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(UPGRAM_WAVES)))
 void k_upgram(double *__restrict__ G, unsigned ldG, const uint16_t *__restrict__ pairs,
               const double *__restrict__ Wbuf, const unsigned *__restrict__ flags,
@@ -984,7 +696,7 @@ void k_upgram(double *__restrict__ G, unsigned ldG, const uint16_t *__restrict__
   __shared__ UpgLds S;
   const unsigned qi = blockIdx.x / nchunk, c = blockIdx.x - qi * nchunk;
   const Quad Q = quads[qi];
-  upgram_item(S, G, ldG, pairs, Wbuf, flags, Q, c, nchunk, CH, part, plan_next, blockDim.x >> 6,
+  upgram_item<NT>(S, G, ldG, pairs, Wbuf, flags, Q, c, nchunk, CH, part, plan_next, blockDim.x >> 6,
               fsplit != 0);
 }
 
@@ -1021,17 +733,7 @@ void k_stage(StageArgs A)
                            A.prec, plan, A.strat0, A.s0steps, A.nswp, A.definite, A.nplus);
   }
   else if (b - A.npl >= A.niw) {
-    // V items: one (pair, row chunk) per wave
-    const unsigned j = b - A.npl - A.niw;
-    const unsigned v = 4u * j + (tid >> 6);
-    if (v < A.nvitems) {
-      const unsigned pi = v / A.nchV, c = v - pi * A.nchV;
-      if (A.vflags[pi]) {
-        const unsigned r0 = c * A.chV;
-        update_rows(A.V, A.ldV, r0, min(r0 + A.chV, A.nrowV), A.vpairs[2u * pi],
-                    A.vpairs[2u * pi + 1u], A.vW + (size_t)pi * 1024u, tid & 63u);
-      }
-    }
+    v_item<4u>(A.v, b - A.npl - A.niw, tid);
   }
   else {
     // item workgroup j takes items j, j + stride, ...: stride niw, or with
@@ -1049,7 +751,7 @@ void k_stage(StageArgs A)
       // a copy in registers: through a reference into global memory its
       // byte fields would be reloaded after every store of the item
       const Quad Q = A.quads[A.qord ? A.qord[qi] : qi];
-      upgram_item(S.upg, A.G, A.ldG, A.upairs, A.uW, A.uflags, Q, c, A.nchunk, A.CH, A.upart,
+      upgram_item<true>(S.upg, A.G, A.ldG, A.upairs, A.uW, A.uflags, Q, c, A.nchunk, A.CH, A.upart,
                   A.uplan, A.nw, A.fsplit != 0);
       __syncthreads();
     }
@@ -1269,22 +971,29 @@ void launch_gram(hipStream_t s, const double *G, unsigned ldG, const uint16_t *p
                  unsigned nchunk, unsigned CH, double *part, const uint8_t *skip)
 {
   const unsigned nw = gram_waves(CH);
+  if (np * nchunk * nw <= GRAM_TILES_MAX) {
+    const auto k = (nw == 1u) ? k_gram_tiles<1u> : (nw == 2u) ? k_gram_tiles<2u> : k_gram_tiles<4u>;
+    hipLaunchKernelGGL(k, dim3(np * nchunk), dim3(256u * nw), 0, s, G, ldG, pairs, nchunk, CH, part,
+                       skip);
+    return;
+  }
   hipLaunchKernelGGL(k_gram, dim3(np * nchunk), dim3(64u * nw), 0, s, G, ldG, pairs, nchunk, CH, part,
                      skip);
 }
 
 void launch_upgram(hipStream_t s, double *G, unsigned ldG, const uint16_t *pairs, const double *W,
                    const unsigned *flags, const Quad *quads, unsigned nquads, unsigned nchunk,
-                   unsigned CH, double *part, const uint8_t *plan_next, bool fsplit)
+                   unsigned CH, double *part, const uint8_t *plan_next, bool fsplit, bool stream)
 {
   const unsigned nw = gram_waves(CH);
-  hipLaunchKernelGGL(k_upgram, dim3(nquads * nchunk), dim3(64u * nw), 0, s, G, ldG, pairs, W, flags,
+  const auto k = stream ? k_upgram<true> : k_upgram<false>;
+  hipLaunchKernelGGL(k, dim3(nquads * nchunk), dim3(64u * nw), 0, s, G, ldG, pairs, W, flags,
                      quads, nchunk, CH, part, plan_next, fsplit ? 1 : 0);
 }
 
 void launch_stage(hipStream_t s, bool sort, const StageArgs &a)
 {
-  const unsigned nb = a.npl + a.niw + a.nvw;
+  const unsigned nb = a.npl + a.niw + (a.v.n + 3u) / 4u;
   if (!nb)
     return;
   if (sort)
@@ -1304,15 +1013,12 @@ void launch_gram_split(hipStream_t s, const double *G, unsigned ldG, const uint1
 void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, const double *part,
                  unsigned nchunk, double *W, unsigned *flags, RunCtl *ctl, VisitRec *rec,
                  const uint8_t *skip, bool split_src, const uint8_t *strat0, unsigned s0steps,
-                 unsigned nswp, int definite, unsigned nplus)
+                 unsigned nswp, int definite, unsigned nplus, const VItems &v)
 {
-  const int ss = split_src ? 1 : 0;
-  if (sort)
-    hipLaunchKernelGGL(k_pair<true>, dim3(np), dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl,
-                       rec, skip, ss, strat0, s0steps, nswp, definite, nplus);
-  else
-    hipLaunchKernelGGL(k_pair<false>, dim3(np), dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl,
-                       rec, skip, ss, strat0, s0steps, nswp, definite, nplus);
+  const auto k = sort ? k_pair<true> : k_pair<false>;
+  hipLaunchKernelGGL(k, dim3(np + (v.n + PAIR_LANES / 2u - 1u) / (PAIR_LANES / 2u)),
+                     dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl, rec, skip,
+                     split_src ? 1 : 0, strat0, s0steps, nswp, definite, nplus, np, v);
 }
 
 void launch_update(hipStream_t s, double *G, unsigned ldG, unsigned nrowG, unsigned chG,

@@ -86,7 +86,17 @@ bool closed_quads(const uint16_t *tab, unsigned steps, unsigned np, std::vector<
 
 void launch_upgram(hipStream_t s, double *G, unsigned ldG, const uint16_t *pairs, const double *W,
                    const unsigned *flags, const Quad *quads, unsigned nquads, unsigned nchunk,
-                   unsigned CH, double *part, const uint8_t *plan_next, bool fsplit);
+                   unsigned CH, double *part, const uint8_t *plan_next, bool fsplit, bool stream);
+
+// The update of V by the W of one step: n = pairs x nch (pair, row chunk) items
+// of ch rows.
+struct VItems {
+  double *V = nullptr;
+  unsigned ld = 0u, nrow = 0u, ch = 0u, nch = 0u, n = 0u;
+  const uint16_t *pairs = nullptr;  // the step's level-1 pairs
+  const double *W = nullptr;        // its W
+  const unsigned *flags = nullptr;  // its update flags
+};
 
 // One launch of a staged sweep: the visits of a list of pairs of one step
 // (one per workgroup) beside the fused transition of a range of closed quads
@@ -121,13 +131,7 @@ struct StageArgs {
   const uint8_t *uplan;    // plans of the next step, or null
   int fsplit;              // items form split Grams for split-planned pairs
                            // (and the visits' Grams were formed that way)
-  // update of V by the W of one step: (pair, row chunk) items, one per wave
-  double *V;
-  unsigned ldV, nrowV, chV, nchV;
-  unsigned nvitems, nvw;   // items (pairs x nchV), their workgroups (ceil(nvitems / 4))
-  const uint16_t *vpairs;  // level-1 pairs of that step
-  const double *vW;        // its W
-  const unsigned *vflags;  // its update flags
+  VItems v;                // update of V by the W of one step
   RunCtl *ctl;
   const uint8_t *strat0;
   unsigned s0steps, nswp;
@@ -151,14 +155,32 @@ void launch_pair_qr(hipStream_t s, bool sort, bool drmac, const double *G, unsig
                     int definite, unsigned nplus);
 
 
+// A whole level-1 step in one launch (hj_step.hip): a workgroup per pair, of
+// up to STEP_MAX_ROWS rows (of G; V has no more).
+constexpr unsigned STEP_MAX_ROWS = 512u;
+struct StepArgs {
+  double *G, *V;           // V null with nrowV 0
+  unsigned ldG, nrow, ldV, nrowV;
+  const uint16_t *pairs;   // the step's level-1 pairs
+  unsigned nsub, SUB;      // the Gram's row chunks (one wave each) and their rows
+  RunCtl *ctl;
+  VisitRec *rec;
+  const uint8_t *strat0;
+  unsigned s0steps, nswp;
+  int definite;
+  unsigned nplus;
+};
+void launch_step(hipStream_t s, bool sort, unsigned np, const StepArgs &a);
+
 void launch_gram_split(hipStream_t s, const double *G, unsigned ldG, const uint16_t *pairs,
                        unsigned np, unsigned nchunk, unsigned CH, double *part, const uint8_t *plan);
 // split_src: the partials come from a standalone Gram launch, so pairs
-// planned split hold split Grams (else every pair is an FP64 visit)
+// planned split hold split Grams (else every pair is an FP64 visit); v: V's
+// items of an earlier step, in the same launch
 void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, const double *part,
                  unsigned nchunk, double *W, unsigned *flags, RunCtl *ctl, VisitRec *rec,
                  const uint8_t *skip, bool split_src, const uint8_t *strat0, unsigned s0steps,
-                 unsigned nswp, int definite, unsigned nplus);
+                 unsigned nswp, int definite, unsigned nplus, const VItems &v = VItems());
 void launch_update(hipStream_t s, double *G, unsigned ldG, unsigned nrowG, unsigned chG,
                    double *V, unsigned ldV, unsigned nrowV, unsigned chV, const uint16_t *pairs,
                    unsigned np, const double *W, const unsigned *flags);
