@@ -237,14 +237,13 @@ __device__ __forceinline__ void level3(double &a, double &b, double &c)
   pin3(a, b, c);
 }
 
-// Dp = p.p, Dq = q.q, Apq = p.q over the 32 rows of a pivot pair, p[i], q[i]
-// being row row_of(l) + LANES i: each by the xor butterfly 16,8,4,2,1 of the
-// 32-lane reduction, the first levels inside the lane.
-template <unsigned LANES>
+// Dp = p.p, Dq = q.q, Apq = p.q over the LANES ROWS (32 or 64) rows of a pivot
+// pair, p[i], q[i] being row row_of(l) + LANES i: each by the xor butterfly
+// (32,) 16,8,4,2,1 of the row distances, the first levels inside the lane.
+template <unsigned LANES, unsigned ROWS = 32u / LANES>
 __device__ __forceinline__ void dots3(const double *p, const double *q, double &Dp, double &Dq,
                                       double &Apq)
 {
-  constexpr unsigned ROWS = 32u / LANES;
   double tp[ROWS], tq[ROWS], tx[ROWS];
 #pragma unroll
   for (unsigned i = 0u; i < ROWS; ++i) {

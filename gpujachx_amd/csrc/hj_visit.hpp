@@ -14,6 +14,8 @@ namespace hj {
 #define RA(A, r, c) (A)[(c) * LDR + (r)]
 // LDS of one pair visit
 struct PairLds {
+  static constexpr unsigned N = 32u, LD = LDR;  // order and leading dimension of R and W
+  static constexpr double TOL = MYTOL;          // of the convergence test
   double R[32u * LDR];
   double W[32u * LDR];
   double cholcol[64];
@@ -36,12 +38,11 @@ constexpr unsigned ACT_TRIG = 4u;   // the rotation is trigonometric
 // The columns of M (R or W) of a pivot pair after the step: lane l of the
 // pair's group holds rows row + LANES i as P[i], Q[i]; ap, aq: the first of
 // them in LDS.  Without branches: an untouched pair is stored as it is.
-template <unsigned LANES, bool HYP>
+template <unsigned LANES, unsigned ROWS, bool HYP>
 __device__ __forceinline__ void apply_pair(lds_f64 *ap, lds_f64 *aq, const double *P,
                                            const double *Q, bool rot, bool cross, bool trig,
                                            double c, double t)
 {
-  constexpr unsigned ROWS = 32u / LANES;
   lds_f64 *const A = cross ? aq : ap, *const B = cross ? ap : aq;
   const double t_ = (!HYP || trig) ? -t : t;
   double a[ROWS], b[ROWS];
@@ -70,19 +71,19 @@ __device__ __forceinline__ unsigned pinu(unsigned x)
 
 // One level-0 sweep on R: lane r of group y takes pivot pair y of every step.
 // Counts its rotations and leaves each step's (c, t, ...) for the W waves.
-template <bool SORT, unsigned LANES, bool HYP>
-__device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
+template <bool SORT, unsigned LANES, bool HYP, class Lds>
+__device__ __forceinline__ void level0_r(Lds &L, unsigned y, unsigned r, unsigned s0steps,
                                          int def, unsigned npos, unsigned &my_s, unsigned &my_b,
                                          bool &swapped)
 {
-  constexpr unsigned ROWS = 32u / LANES;
+  constexpr unsigned ROWS = Lds::N / LANES, LD = Lds::LD, PAIRS = Lds::N / 2u;
   lds_f64 *const M = (lds_f64 *)L.R + row_of(r);
   const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
   // sorted definite pairs: columns by decreasing D for J = I, by increasing
   // D for J = -I: descending in D xor this sign
   const uint64_t neg0 = (!HYP && def < 0) ? 0x8000000000000000ull : 0ull;
   unsigned pq = S0[0];
-  unsigned p = pq & 255u, q = pq >> 8, op = p * LDR, oq = q * LDR;
+  unsigned p = pq & 255u, q = pq >> 8, op = p * LD, oq = q * LD;
 #pragma unroll 1
   for (unsigned step = 0u; step < s0steps; ++step) {
     lds_f64 *const ap = M + op, *const aq = M + oq;
@@ -92,7 +93,7 @@ __device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, uns
       Gp[i] = ap[LANES * i];
       Gq[i] = aq[LANES * i];
     }
-    pq = S0[16u * min(step + 1u, s0steps - 1u)];
+    pq = S0[PAIRS * min(step + 1u, s0steps - 1u)];
     bool trig = true, inorder = SORT;
     uint64_t neg = neg0;
     if (HYP) {
@@ -102,12 +103,12 @@ __device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, uns
       inorder = SORT & trig;
     }
     double Dp, Dq, Apq;
-    dots3<LANES>(Gp, Gq, Dp, Dq, Apq);
+    dots3<LANES, ROWS>(Gp, Gq, Dp, Dq, Apq);
     // the rotation on every lane; only a transforming pair uses it
     double c, t, Dpq_;
     const bool big = rot_quad<HYP>(trig, Apq, Dp, Dq, r, c, t, Dpq_);
     const double Apq_ = fabs(Apq);
-    const bool transf = !(Apq_ < (Dpq_ * MYTOL));
+    const bool transf = !(Apq_ < (Dpq_ * Lds::TOL));
     bool cross = false;
     if (SORT) {
       // rotated: unless in order afterwards; not rotated: when out of order
@@ -117,7 +118,7 @@ __device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, uns
       cross = inorder & ((transf & !ge) | (!transf & lt));
       swapped = swapped | (cross & !transf);
     }
-    apply_pair<LANES, HYP>(ap, aq, Gp, Gq, transf, cross, trig, c, t);
+    apply_pair<LANES, ROWS, HYP>(ap, aq, Gp, Gq, transf, cross, trig, c, t);
     if (r == 0u) {
       double *const o = L.rot[step & 1u][y];
       o[0] = c;
@@ -131,8 +132,8 @@ __device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, uns
     my_b += (transf & big) ? 1u : 0u;
     p = pq & 255u;
     q = pq >> 8;
-    op = pinu(p * LDR);
-    oq = pinu(q * LDR);
+    op = pinu(p * LD);
+    oq = pinu(q * LD);
     __syncthreads();
   }
 }
@@ -140,18 +141,18 @@ __device__ __forceinline__ void level0_r(PairLds &L, unsigned y, unsigned r, uns
 // The same sweep's rotations applied to W, each step's between the barrier
 // that ends it on the R waves and the next; with cosines, the largest
 // |Apq| / (|p| |q|).
-template <unsigned LANES>
-__device__ __forceinline__ void level0_w(PairLds &L, unsigned y, unsigned r, unsigned s0steps,
+template <unsigned LANES, class Lds>
+__device__ __forceinline__ void level0_w(Lds &L, unsigned y, unsigned r, unsigned s0steps,
                                          bool cosines)
 {
-  constexpr unsigned ROWS = 32u / LANES;
+  constexpr unsigned ROWS = Lds::N / LANES, LD = Lds::LD, PAIRS = Lds::N / 2u;
   lds_f64 *const M = (lds_f64 *)L.W + row_of(r);
   const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
   double my_cos = 0.0;
 #pragma unroll 1
   for (unsigned step = 0u; step < s0steps; ++step) {
-    const unsigned pq = S0[16u * step];
-    const unsigned op = pinu((pq & 255u) * LDR), oq = pinu((pq >> 8) * LDR);
+    const unsigned pq = S0[PAIRS * step];
+    const unsigned op = pinu((pq & 255u) * LD), oq = pinu((pq >> 8) * LD);
     __syncthreads();
     lds_f64 *const ap = M + op, *const aq = M + oq;
     double P[ROWS], Q[ROWS];
@@ -163,7 +164,7 @@ __device__ __forceinline__ void level0_w(PairLds &L, unsigned y, unsigned r, uns
     const double *const o = L.rot[step & 1u][y];
     const unsigned act = L.act[step & 1u][y];
     const double cn = o[2], cd = o[3];
-    apply_pair<LANES, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
+    apply_pair<LANES, ROWS, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
                             (act & ACT_TRIG) != 0u, o[0], o[1]);
     if (cosines)
       my_cos = fmax(my_cos, (cd > 0.0) ? cn / cd : 0.0);
@@ -195,6 +196,63 @@ __device__ __forceinline__ PairSigns pair_signs16(int definite, unsigned nplus, 
     s.hyp = (s.def == 0);
   }
   return s;
+}
+
+// Inner Jacobi: share/device_code_nosort.hpp:4-222 (SORT false),
+// share/device_code_cdsort_KISS.hpp:4-260 and share/device_code_cdsort.hpp:25-167
+// (SORT true): up to nswp level-0 sweeps by the N LANES threads of a workgroup,
+// half of them on R, half on W.  Returns, in every thread, the rotations.
+// on_r: one sweep on R by lane r of pivot pair y (level0_r, or another with
+// its counts and its steps' (c, t) and ACT_* in L).
+template <unsigned LANES, class Lds, class OnR>
+__device__ __forceinline__ void inner_sweeps_by(unsigned tid, Lds &L, unsigned s0steps, unsigned nswp,
+                                                bool cosines, unsigned &blk_s, unsigned &blk_b,
+                                                OnR on_r)
+{
+  constexpr unsigned NT = Lds::N * LANES;
+  const bool onR = tid < NT / 2u;  // this wave's matrix: R or W
+  const unsigned ht = tid & (NT / 2u - 1u);
+  const unsigned y = ht / LANES, r = ht & (LANES - 1u);
+  blk_s = blk_b = 0u;
+  for (unsigned swp = 0u; swp < nswp; ++swp) {
+    unsigned my_s = 0u, my_b = 0u;
+    bool swapped = false;
+    if (!onR)
+      level0_w<LANES>(L, y, r, s0steps, cosines && swp == 0u);
+    else
+      on_r(y, r, my_s, my_b, swapped);
+    // every lane of a pair's group holds its counts
+    if (onR && r == 0u && my_s) {
+      atomicAdd(&L.cs[swp & 1u], my_s);
+      atomicAdd(&L.cb[swp & 1u], my_b);
+    }
+    if (onR && swapped)
+      L.swp = 1;
+    __syncthreads();
+    const unsigned swp_s = L.cs[swp & 1u];
+    // (the other parity was read before this sweep's steps)
+    if (tid == 0u)
+      L.cs[(swp + 1u) & 1u] = 0u;
+    if (tid == 64u)
+      L.cb[(swp + 1u) & 1u] = 0u;
+    if (!swp_s)
+      break;
+    blk_s += swp_s;
+    blk_b += L.cb[swp & 1u];
+  }
+}
+
+template <bool SORT, unsigned LANES, class Lds>
+__device__ __forceinline__ void inner_sweeps(unsigned tid, Lds &L, const PairSigns &sg, unsigned s0steps,
+                                             unsigned nswp, bool cosines, unsigned &blk_s, unsigned &blk_b)
+{
+  inner_sweeps_by<LANES>(tid, L, s0steps, nswp, cosines, blk_s, blk_b,
+                         [&](unsigned y, unsigned r, unsigned &my_s, unsigned &my_b, bool &swapped) {
+                           if (sg.hyp)
+                             level0_r<SORT, LANES, true>(L, y, r, s0steps, sg.def, sg.npos, my_s, my_b, swapped);
+                           else
+                             level0_r<SORT, LANES, false>(L, y, r, s0steps, sg.def, sg.npos, my_s, my_b, swapped);
+                         });
 }
 
 // The visit's LDS before its Gram: level-0 table (16 bytes a thread), W = I,
@@ -285,7 +343,6 @@ __device__ __forceinline__ bool visit_core(unsigned tid, unsigned pi, PairLds &L
                                            RunCtl *__restrict__ ctl, VisitRec *__restrict__ rec,
                                            uint8_t plan, unsigned s0steps, unsigned nswp)
 {
-  constexpr unsigned NT = 32u * LANES;
   __syncthreads();
   // Cholesky, share/device_code_common_Cholesky.hpp:58-158 (USE_RSQRT):
   // column k scaled by rsqrt(A(k,k)), diagonal sqrt(A(k,k)), then
@@ -322,41 +379,8 @@ __device__ __forceinline__ bool visit_core(unsigned tid, unsigned pi, PairLds &L
     return false;
   }
 
-  // Inner Jacobi: share/device_code_nosort.hpp:4-222 (SORT false),
-  // share/device_code_cdsort_KISS.hpp:4-260 and share/device_code_cdsort.hpp:25-167
-  // (SORT true).
-  const bool onR = tid < NT / 2u;  // this wave's matrix: R or W
-  const unsigned ht = tid & (NT / 2u - 1u);
-  const unsigned y = ht / LANES, r = ht & (LANES - 1u);
-  unsigned blk_s = 0u, blk_b = 0u;
-  for (unsigned swp = 0u; swp < nswp; ++swp) {
-    unsigned my_s = 0u, my_b = 0u;
-    bool swapped = false;
-    if (!onR)
-      level0_w<LANES>(L, y, r, s0steps, swp == 0u);
-    else if (sg.hyp)
-      level0_r<SORT, LANES, true>(L, y, r, s0steps, sg.def, sg.npos, my_s, my_b, swapped);
-    else
-      level0_r<SORT, LANES, false>(L, y, r, s0steps, sg.def, sg.npos, my_s, my_b, swapped);
-    // every lane of a pair's group holds its counts
-    if (onR && r == 0u && my_s) {
-      atomicAdd(&L.cs[swp & 1u], my_s);
-      atomicAdd(&L.cb[swp & 1u], my_b);
-    }
-    if (onR && swapped)
-      L.swp = 1;
-    __syncthreads();
-    const unsigned swp_s = L.cs[swp & 1u];
-    // (the other parity was read before this sweep's steps)
-    if (tid == 0u)
-      L.cs[(swp + 1u) & 1u] = 0u;
-    if (tid == 64u)
-      L.cb[(swp + 1u) & 1u] = 0u;
-    if (!swp_s)
-      break;
-    blk_s += swp_s;
-    blk_b += L.cb[swp & 1u];
-  }
+  unsigned blk_s, blk_b;
+  inner_sweeps<SORT, LANES>(tid, L, sg, s0steps, nswp, true, blk_s, blk_b);
 
   // the block update is left out exactly when W is the identity (no rotation,
   // no swap)

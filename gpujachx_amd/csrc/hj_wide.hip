@@ -10,12 +10,10 @@
 //     16-row slabs, the waves added in order, the chunks in order by the
 //     visit;
 //   - Cholesky (share/device_code_common_Cholesky.hpp:58-158, USE_RSQRT) at
-//     64 pivots, one row per lane, the pivots on one wave and the column
-//     updates on the others;
-//   - level-0: 32 pivot pairs a step, 16 lanes a pair, lane r holding rows
-//     r + 16i (i < 4) of both columns of R and W; dot products by the xor
-//     butterfly 32,16 in the lane, 8,4,2,1 across lanes; the convergence
-//     test at tolerance sqrt(64) 2^-53;
+//     64 pivots, 32 at a time;
+//   - level-0: 32 pivot pairs a step, 8 lanes a pair, dot products by the xor
+//     butterfly 32,16,8 in the lane, 4,2,1 across lanes; the convergence test
+//     at tolerance sqrt(64) 2^-53;
 //   - update: out(r, j) = MFMA chain over k = 0..63.
 // With the learned pair-skip a step's plan marks skipped pairs: no Gram, no
 // visit (its record keeps the last executed visit), no update.
@@ -24,6 +22,7 @@
 #include "hj_device.hpp"
 #include "hj_fused.hpp"
 #include "hj_util.hpp"
+#include "hj_visit.hpp"
 
 namespace hj {
 
@@ -31,7 +30,7 @@ namespace {
 
 constexpr unsigned WTILES = 10u;             // tiles of a 64-column pair's lower triangle
 constexpr unsigned WPART = WTILES * 256u;    // doubles per Gram partial
-constexpr unsigned LDRW = 65u;               // padded column of R and W in LDS
+constexpr unsigned LDRW = 72u;               // column of R and W in LDS: of eight lanes a pivot pair, two neighbouring pairs in different banks
 constexpr double WTOL = 0x1p-50;             // sqrt(64) * 2^-53
 #define RW(A, r, c) (A)[(c) * LDRW + (r)]
 
@@ -139,113 +138,208 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   }
 }
 
-// Sum of the 64 rows of one pivot pair held by 16 lanes, lane r holding
-// rows r + 16i as v[i]: the xor butterfly 32,16 inside the lane, 8 (a
-// rotation by 8 inside the 16-lane DPP row), 4,2,1 across lanes.
-__device__ __forceinline__ double lane_xor8(double v) { return dpp_mov<0x128>(v); }
+constexpr unsigned VT = 512u;  // threads of a visit: half on R, half on W, 8 lanes a pivot pair
 
-__device__ __forceinline__ double sum16x4(const double *v)
-{
-  double s = (v[0] + v[2]) + (v[1] + v[3]);
-  s = s + lane_xor8(s);
-  s = s + lane_xor4(s);
-  s = s + lane_xor2(s);
-  s = s + lane_xor1(s);
-  return s;
-}
-
-constexpr unsigned VT = 512u;  // threads of a visit: 32 pivot pairs x 16 lanes
-
-// In-place 64x64 Cholesky by the workgroup's eight waves, in LDS (lane x
-// of every wave standing for row x of the lower triangle):
-// share/device_code_common_Cholesky.hpp:58-158 (USE_RSQRT).  Per pivot k,
-// wave 0 scales column k (rsqrt(A(k,k)) below the diagonal, sqrt(A(k,k)) on
-// it), copies it to col and forms the next pivot A(k+1,k+1) - L(k+1,k)^2;
-// after a barrier it computes that pivot's rsqrt and sqrt while waves 1-7
-// apply A(x,j) = fma(-A(x,k), A(j,k), A(x,j)) to the columns j > k in
-// batches of 8 (a batch's loads, then its fmas, then its stores; rows above
-// j produce values never read).  Then R = L^T, zeros below the diagonal.
-__device__ __forceinline__ void chol64_block(double *A_, double *col_, unsigned tid)
-{
-  lds_f64 *const A = (lds_f64 *)A_;
-  lds_f64 *const col = (lds_f64 *)col_;
-  const unsigned x = tid & 63u, w = tid >> 6;
-  double akk = 0.0, rk = 0.0, dk = 0.0;
-  if (w == 0u) {
-    akk = readlane_d(A[x], 0);
-    rk = dev_rsqrt(akk);
-    dk = sqrt(akk);
-  }
-  for (unsigned k = 0u; k < 64u; ++k) {
-    const unsigned k1 = k + 1u;
-    if (w == 0u) {
-      double v = A[k * LDRW + x];
-      v = (x > k) ? v * rk : ((x == k) ? dk : v);
-      A[k * LDRW + x] = v;
-      col[x] = v;
-      if (k1 < 64u) {
-        const double lk = readlane_d(v, k1);
-        const double d1 = readlane_d(A[k1 * LDRW + x], k1);
-        akk = __fma_rn(-lk, lk, d1);
-      }
-    }
-    __syncthreads();
-    if (k1 < 64u) {
-      if (w == 0u) {
-        rk = dev_rsqrt(akk);
-        dk = sqrt(akk);
-      }
-      else {
-        const double v = col[x];
-        for (unsigned jb = (k1 & ~7u) + 8u * (w - 1u); jb < 64u; jb += 8u * (VT / 64u - 1u)) {
-          double av[8], cv[8];
-#pragma unroll
-          for (unsigned i = 0u; i < 8u; ++i) {
-            av[i] = A[(jb + i) * LDRW + x];
-            cv[i] = col[jb + i];
-          }
-#pragma unroll
-          for (unsigned i = 0u; i < 8u; ++i)
-            if (jb + i >= k1) av[i] = __fma_rn(-v, cv[i], av[i]);
-#pragma unroll
-          for (unsigned i = 0u; i < 8u; ++i)
-            A[(jb + i) * LDRW + x] = av[i];
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // R(r, c) = L(c, r) for r <= c: all reads, a barrier, all writes
-  double t[4096u / VT];
-#pragma unroll
-  for (unsigned i = 0u; i < 4096u / VT; ++i) {
-    const unsigned e = tid + VT * i, r = e & 63u, c = e >> 6;
-    t[i] = (r <= c) ? A[r * LDRW + c] : 0.0;
-  }
-  __syncthreads();
-#pragma unroll
-  for (unsigned i = 0u; i < 4096u / VT; ++i) {
-    const unsigned e = tid + VT * i, r = e & 63u, c = e >> 6;
-    A[c * LDRW + r] = t[i];
-  }
-}
-
+// LDS of a 64-column pair visit
 constexpr unsigned S0W_BYTES = 64u * 32u * 2u;  // level-0 table of order 64 (<= 64 steps)
 
 struct PairLdsW {
+  static constexpr unsigned N = 64u, LD = LDRW;  // order and leading dimension of R and W
+  static constexpr double TOL = WTOL;            // of the convergence test
   double R[64u * LDRW];
   double W[64u * LDRW];
+  double A22[32u * L0LD];  // the Cholesky's trailing block
   double col[64];
-  unsigned cnt_s[32], cnt_b[32];
-  float cmax[32];
+  double diag[64];         // the Gram's diagonal
+  double rot[2][32][4];    // per step parity and pivot pair: c, t, |Apq|, |p| |q|
+  unsigned act[2][32];     // ... what happens to its columns (ACT_*)
+  unsigned cs[2], cb[2];   // rotations of an inner sweep, by its parity
+  unsigned cmax;           // bits of the largest cosine of the first inner sweep
   float bnorm[2];
   int swp;
-  uint8_t S0[S0W_BYTES];
+  __attribute__((aligned(16))) uint8_t S0[S0W_BYTES];
 };
+
+// The first 32 columns of the Cholesky factor of the 64x64 Gram in A (lower
+// triangle, A[c * LDRW + r] = A(r, c)) by one wave, lane x on row x:
+// share/device_code_common_Cholesky.hpp:58-158 (USE_RSQRT) for k < 32, j < 32.
+// On return A holds the first 32 rows of R = L^T (R(k, x) at A[x * LDRW + k])
+// and zeros below them; the columns from 32 on are untouched.
+//
+// panel_any takes any input, column by column in LDS.
+__device__ __forceinline__ void panel_any(lds_f64 *A, lds_f64 *col, unsigned x)
+{
+#pragma unroll 1
+  for (unsigned k = 0u; k < 32u; ++k) {
+    const double akk = A[k * LDRW + k], v = A[k * LDRW + x];
+    const double rk = dev_rsqrt_any(akk), dk = sqrt(akk);
+    const double w = (x == k) ? dk : v * rk;
+    wave_lds_sync();
+    if (x >= k) A[k * LDRW + x] = w;
+    col[x] = w;
+    wave_lds_sync();
+#pragma unroll 1
+    for (unsigned j = k + 1u; j < 32u; ++j)
+      if (x >= j) A[j * LDRW + x] = __fma_rn(-w, col[j], A[j * LDRW + x]);
+    wave_lds_sync();
+  }
+#pragma unroll 1
+  for (unsigned c = 0u; c < 32u; ++c) {
+    const double v = A[c * LDRW + x];
+    wave_lds_sync();
+    if (x > c) {
+      A[x * LDRW + c] = v;
+      A[c * LDRW + x] = 0.0;
+    }
+    wave_lds_sync();
+  }
+}
+
+// chol32_wave's scheme on 64 rows: the panel in registers, the next pivot's
+// rsqrt (the chain of the pivots) beside the column's updates, the diagonal's
+// square roots in one instruction sequence at the end.
+__device__ __forceinline__ void panel_wave(double *A_, double *col_, unsigned x)
+{
+  lds_f64 *const A = (lds_f64 *)A_;
+  lds_f64 *const col = (lds_f64 *)col_;
+  double b[32];
+#pragma unroll
+  for (unsigned c = 0u; c < 32u; ++c)
+    b[c] = (c <= x) ? A[c * LDRW + x] : 0.0;
+  double akk = readlane_d(b[0], 0);
+  bool sure;
+  double rk = rsqrt_bracket(akk, sure);
+  unsigned long long bad = __ballot(!(sure && rsqrt_plain_range(akk)));
+#pragma unroll
+  for (unsigned k = 0u; k < 32u; ++k) {
+    const unsigned k1 = k + 1u;
+    const double u = pin(b[k] * rk);
+    col[x] = u;
+    b[k] = pin((x > k) ? u : b[k]);
+    if (k1 == 32u)
+      break;
+    const double lk = readlane_d(u, k1);
+    const double d1 = readlane_d(b[k1], k1);
+    akk = __fma_rn(-lk, lk, d1);
+    wave_lds_sync();
+    double cv[32];
+#pragma unroll
+    for (unsigned j = k1; j < 32u; ++j)
+      cv[j] = col[j];
+    // the column's reads are issued here, all of them, and used after the
+    // pivot's chain has started
+    __builtin_amdgcn_sched_barrier(0);
+    rk = rsqrt_bracket(akk, sure);
+    bad |= __ballot(!(sure && rsqrt_plain_range(akk)));
+#pragma unroll
+    for (unsigned j = k1; j < 32u; ++j)
+      b[j] = __fma_rn(-u, cv[j], b[j]);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+s"(bad));
+#pragma unroll
+    for (unsigned j = k1; j < 32u; ++j)
+      asm volatile("" : "+v"(b[j]));
+    wave_lds_sync();
+  }
+  if (bad) {
+    panel_any(A, col, x);
+    return;
+  }
+  // (above the diagonal: entries of other columns' lower triangle stay)
+#pragma unroll
+  for (unsigned c = 0u; c < 32u; ++c)
+    if (c <= x) A[x * LDRW + c] = b[c];
+#pragma unroll
+  for (unsigned c = 0u; c < 32u; ++c)
+    if (c < x) A[c * LDRW + x] = 0.0;
+  wave_lds_sync();
+  const double d = sqrt(A[x * LDRW + x]);
+  wave_lds_sync();
+  if (x < 32u) A[x * LDRW + x] = d;
+}
+
+// In-place 64x64 Cholesky by the workgroup, R = L^T with zeros below: the
+// first 32 columns (one wave), the trailing block's update by them (a chain
+// over k = 0..31 in order on FP64 MFMA, one wave a tile), its Cholesky (one
+// wave, chol32_wave), while the others set W to the identity.  Every entry
+// takes the same operations in the same order as column by column.  Ends
+// synchronized.
+__device__ __forceinline__ void chol64_block(PairLdsW &L, unsigned tid)
+{
+  lds_f64 *const A = (lds_f64 *)L.R;
+  lds_f64 *const B = (lds_f64 *)L.A22;
+  const unsigned l = tid & 63u, w = tid >> 6;
+  if (w == 0u) {
+    panel_wave(L.R, L.col, l);
+  }
+  else if (tid < 66u) {
+    // squared Frobenius norms of the two blocks, for the visit record
+    double sn = 0.0;
+    for (unsigned k = 0u; k < 32u; ++k)
+      sn = sn + L.diag[32u * (tid - 64u) + k];
+    L.bnorm[tid - 64u] = (float)log2(sn);
+  }
+  __syncthreads();
+  if (w < 3u) {
+    // tile (ti, tj) of the trailing block: 00, 10, 11
+    const unsigned i0 = w ? 16u : 0u, j0 = (w == 2u) ? 16u : 0u;
+    const lds_f64 *const X = A + (32u + i0 + (l & 15u)) * LDRW + (l >> 4);
+    const lds_f64 *const Y = A + (32u + j0 + (l & 15u)) * LDRW + (l >> 4);
+    const lds_f64 *const C = A + (32u + j0 + (l & 15u)) * LDRW + 32u + i0 + (l >> 4);
+    d4 acc;
+#pragma unroll
+    for (unsigned r = 0u; r < 4u; ++r)
+      acc[r] = C[4u * r];
+#pragma unroll
+    for (unsigned u = 0u; u < 8u; ++u)
+      acc = mfma(-X[4u * u], Y[4u * u], acc);
+#pragma unroll
+    for (unsigned r = 0u; r < 4u; ++r)
+      B[(j0 + (l & 15u)) * L0LD + i0 + 4u * r + (l >> 4)] = acc[r];
+  }
+  __syncthreads();
+  if (w == 0u) {
+    (void)chol32_wave<L0LD>(L.A22, L.col, l, false);
+  }
+  else {
+    for (unsigned e = tid - 64u; e < 4096u; e += VT - 64u)
+      RW(L.W, e & 63u, e >> 6) = ((e & 63u) == (e >> 6)) ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  for (unsigned e = tid; e < 1024u; e += VT)
+    RW(L.R, 32u + (e & 31u), 32u + (e >> 5)) = L.A22[(e >> 5) * L0LD + (e & 31u)];
+  __syncthreads();
+}
+
+// J of a pair's 64 columns (see PairSigns)
+__device__ __forceinline__ PairSigns pair_signs32(int definite, unsigned nplus, unsigned iBlk,
+                                                  unsigned jBlk)
+{
+  PairSigns s = {definite, 0u, false};
+  if (!definite) {
+    const unsigned ifc0 = iBlk * 32u, ifc1 = jBlk * 32u;
+    if (nplus <= ifc0) { s.npos = 0u; s.def = -1; }
+    else if (nplus <= ifc0 + 32u) { s.npos = nplus - ifc0; s.def = 0; }
+    else if (nplus <= ifc1) { s.npos = 32u; s.def = 0; }
+    else if (nplus <= ifc1 + 32u) { s.npos = 32u + (nplus - ifc1); s.def = 0; }
+    else { s.npos = 64u; s.def = +1; }
+    s.hyp = (s.def == 0);
+  }
+  return s;
+}
 
 // One 64-column block pair per workgroup of 512 threads: chunk partials ->
 // R (lower), Cholesky, level-0 sweeps on R accumulating W, counters, W and
-// the update flag out.  The arithmetic of pair_visit at 64 columns.
+// the update flag out.  The visit of 32 columns (hj_visit.hpp) at 64: four
+// waves keep R, eight lanes a pivot pair, four apply the same rotations to W
+// one step behind.  A level-0 step is bound by its instructions (a wave of
+// either kind on every SIMD) and by LDS, which moves R and W once in and once
+// out: 1024 cycles at 128 bytes each, so the columns' leading dimension keeps
+// the groups of a wave off each other's banks (LDRW = 65: two- to fourfold
+// conflicts).  Measured, 4608 x 2048: partials 4 us, Cholesky 14 us, a level-0
+// sweep 73 us (89 us at LDRW = 65); 92 us a launch, 126 us with eight waves of
+// 16 lanes a pair that each kept R and W, and a Cholesky of 64 pivots with two
+// barriers each.
 template <bool SORT>
 __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pairs,
                                                 const double *__restrict__ part, unsigned nchunk,
@@ -269,161 +363,44 @@ __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pai
     }
     return;
   }
-  double *const R = L.R;
-  double *const W = L.W;
-  const unsigned iBlk = pairs[2u * pi], jBlk = pairs[2u * pi + 1u];
-  // local J structure, share/device_code_nosort_accumV.hpp:53-76
-  bool hyp = false;
-  int def = definite;
-  unsigned npos = 0u;
-  if (!definite) {
-    const unsigned ifc0 = iBlk * 32u, ifc1 = jBlk * 32u;
-    if (nplus <= ifc0) { npos = 0u; def = -1; }
-    else if (nplus <= ifc0 + 32u) { npos = nplus - ifc0; def = 0; }
-    else if (nplus <= ifc1) { npos = 32u; def = 0; }
-    else if (nplus <= ifc1 + 32u) { npos = 32u + (nplus - ifc1); def = 0; }
-    else { npos = 64u; def = +1; }
-    hyp = (def == 0);
-  }
-  if (tid == 0u)
-    L.swp = 0;
-  for (unsigned e = tid; e < 2u * 32u * s0steps; e += VT)
-    L.S0[e] = strat0[e];
+  const PairSigns sg = pair_signs32(definite, nplus, pairs[2u * pi], pairs[2u * pi + 1u]);
   {
     const double *const pp = part + (size_t)pi * nchunk * WPART;
-    // two entries a thread at a time, all their chunk loads in flight
-    // together; the chunks summed in chunk order
-#pragma unroll 1
-    for (unsigned q = 0u; q < WPART / VT; ++q) {
-      double v[1][MAX_GRAM_CHUNKS];
+    // a thread's entries with all their chunk loads in flight together; the
+    // chunks summed in chunk order
+    constexpr unsigned NE = WPART / VT;
+    double v[NE][MAX_GRAM_CHUNKS];
 #pragma unroll
-      for (unsigned h = 0u; h < 1u; ++h)
+    for (unsigned q = 0u; q < NE; ++q)
 #pragma unroll
-        for (unsigned c = 0u; c < MAX_GRAM_CHUNKS; ++c)
-          if (c < nchunk) v[h][c] = pp[(size_t)c * WPART + tid + VT * (q + h)];
+      for (unsigned c = 0u; c < MAX_GRAM_CHUNKS; ++c)
+        if (c < nchunk) v[q][c] = pp[(size_t)c * WPART + tid + VT * q];
+    for (unsigned e = tid; e < 2u * 32u * s0steps; e += VT)
+      L.S0[e] = strat0[e];
+    if (tid == 0u) {
+      L.swp = 0;
+      L.cmax = 0u;
+      L.cs[0] = L.cb[0] = 0u;
+    }
 #pragma unroll
-      for (unsigned h = 0u; h < 1u; ++h) {
-        const unsigned e = tid + VT * (q + h);
-        double s = v[h][0];
+    for (unsigned q = 0u; q < NE; ++q) {
+      const unsigned e = tid + VT * q;
+      double s = v[q][0];
 #pragma unroll
-        for (unsigned c = 1u; c < MAX_GRAM_CHUNKS; ++c)
-          if (c < nchunk) s = s + v[h][c];
-        const unsigned tt = e >> 8, ti = tile_i(tt), tj = tt - ti * (ti + 1u) / 2u;
-        const unsigned l = (e >> 2) & 63u, r = e & 3u;
-        RW(R, 16u * ti + 4u * r + (l >> 4), 16u * tj + (l & 15u)) = s;
-      }
+      for (unsigned c = 1u; c < MAX_GRAM_CHUNKS; ++c)
+        if (c < nchunk) s = s + v[q][c];
+      const unsigned tt = e >> 8, ti = tile_i(tt), tj = tt - ti * (ti + 1u) / 2u;
+      const unsigned l = (e >> 2) & 63u, r = e & 3u;
+      const unsigned row = 16u * ti + 4u * r + (l >> 4), col = 16u * tj + (l & 15u);
+      RW(L.R, row, col) = s;
+      if (row == col) L.diag[row] = s;
     }
   }
-  for (unsigned e = tid; e < 4096u; e += VT)
-    RW(W, e & 63u, e >> 6) = ((e & 63u) == (e >> 6)) ? 1.0 : 0.0;
   __syncthreads();
-  if (rec && tid < 2u) {
-    // squared Frobenius norms of the two blocks, for the visit record
-    double sn = 0.0;
-    for (unsigned k = 0u; k < 32u; ++k)
-      sn = sn + RW(R, 32u * tid + k, 32u * tid + k);
-    L.bnorm[tid] = (float)log2(sn);
-  }
-  __syncthreads();
-  chol64_block(R, L.col, tid);
-  __syncthreads();
+  chol64_block(L, tid);
 
-  const unsigned y = tid >> 4, r = tid & 15u;
-  unsigned blk_s = 0u, blk_b = 0u;
-  bool swapped = false;
-  double my_cos = 0.0;  // max |Apq| / sqrt(Dp Dq) of the slot's pivots, first inner sweep
-  for (unsigned swp = 0u; swp < nswp; ++swp) {
-    unsigned my_s = 0u, my_b = 0u;
-    for (unsigned step = 0u; step < s0steps; ++step) {
-      const unsigned p = L.S0[(step * 32u + y) * 2u], q = L.S0[(step * 32u + y) * 2u + 1u];
-      double Gp[4], Gq[4], Vp[4], Vq[4], t0[4], t1[4], t2[4];
-#pragma unroll
-      for (unsigned i = 0u; i < 4u; ++i) {
-        Gp[i] = RW(R, r + 16u * i, p);
-        Gq[i] = RW(R, r + 16u * i, q);
-        Vp[i] = RW(W, r + 16u * i, p);
-        Vq[i] = RW(W, r + 16u * i, q);
-      }
-#pragma unroll
-      for (unsigned i = 0u; i < 4u; ++i) {
-        t0[i] = __fma_rn(Gp[i], Gp[i], 0.0);
-        t1[i] = __fma_rn(Gq[i], Gq[i], 0.0);
-        t2[i] = __fma_rn(Gp[i], Gq[i], 0.0);
-      }
-      double Dp = sum16x4(t0), Dq = sum16x4(t1);
-      const double Apq = sum16x4(t2);
-      const double Dp_ = sqrt(Dp), Dq_ = sqrt(Dq), Apq_ = fabs(Apq), Dpq_ = Dp_ * Dq_;
-      const int transf_s = !(Apq_ < (Dpq_ * WTOL));
-      if (rec && swp == 0u && Dpq_ > 0.0)
-        my_cos = fmax(my_cos, Apq_ / Dpq_);
-      int pdef = def;
-      if (hyp) {
-        if ((p < npos) && (q < npos)) pdef = +1;
-        else if ((p >= npos) && (q >= npos)) pdef = -1;
-        else pdef = 0;
-      }
-      bool trig;
-      if (!SORT) trig = !hyp || pdef;
-      else trig = (pdef != 0);
-      double c, t;
-      const int rot_b = dev_rot(trig, Apq, Dp, Dq, c, t);
-      int transf_b = 0;
-      if (transf_s) {
-        transf_b = rot_b;
-        const double t_ = trig ? -t : t;
-        if (SORT && trig) {
-          Dp = __fma_rn(t, Apq, Dp);
-          Dq = __fma_rn(t_, Apq, Dq);
-        }
-        bool keep = true;
-        if (SORT)
-          keep = (!pdef) || ((pdef > 0) && (Dp >= Dq)) || ((pdef < 0) && (Dp <= Dq));
-        const unsigned P = keep ? p : q, Q = keep ? q : p;
-#pragma unroll
-        for (unsigned i = 0u; i < 4u; ++i) {
-          const double rp = __fma_rn(t_, Gq[i], Gp[i]), rq = __fma_rn(t, Gp[i], Gq[i]);
-          const double wp = __fma_rn(t_, Vq[i], Vp[i]), wq = __fma_rn(t, Vp[i], Vq[i]);
-          RW(R, r + 16u * i, P) = c * rp;
-          RW(R, r + 16u * i, Q) = c * rq;
-          RW(W, r + 16u * i, P) = c * wp;
-          RW(W, r + 16u * i, Q) = c * wq;
-        }
-      }
-      else if (SORT && (((pdef > 0) && (Dp < Dq)) || ((pdef < 0) && (Dq < Dp)))) {
-#pragma unroll
-        for (unsigned i = 0u; i < 4u; ++i) {
-          RW(R, r + 16u * i, p) = Gq[i];
-          RW(R, r + 16u * i, q) = Gp[i];
-          RW(W, r + 16u * i, p) = Vq[i];
-          RW(W, r + 16u * i, q) = Vp[i];
-        }
-        swapped = true;
-      }
-      my_s += (unsigned)transf_s;
-      my_b += (unsigned)transf_b;
-      __syncthreads();
-    }
-    if (r == 0u) {
-      L.cnt_s[y] = my_s;
-      L.cnt_b[y] = my_b;
-    }
-    __syncthreads();
-    unsigned swp_s = 0u, swp_b = 0u;
-    for (unsigned i = 0u; i < 32u; ++i) {
-      swp_s += L.cnt_s[i];
-      swp_b += L.cnt_b[i];
-    }
-    __syncthreads();
-    if (!swp_s)
-      break;
-    blk_s += swp_s;
-    blk_b += swp_b;
-  }
-  if (swapped)
-    L.swp = 1;
-  if (r == 0u)
-    L.cmax[y] = (float)my_cos;
-  __syncthreads();
+  unsigned blk_s, blk_b;
+  inner_sweeps<SORT, VT / 64u>(tid, L, sg, s0steps, nswp, rec != nullptr, blk_s, blk_b);
   if (tid == 0u) {
     // convergence counter, share/device_code_nosort.hpp:94-103
     if (blk_s) {
@@ -436,13 +413,10 @@ __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pai
     if (rec) {
       // the record in the units of a 32-column pair's inner sweep (496 pivot
       // pairs): this pair's counts scaled from its 2016
-      float cm = 0.0f;
-      for (unsigned i = 0u; i < 32u; ++i)
-        cm = fmaxf(cm, L.cmax[i]);
       VisitRec v;
       v.rot_s = (min(blk_s, 2016u) * 496u + 1008u) / 2016u;
       v.rot_b = (min(blk_b, 2016u) * 496u + 1008u) / 2016u;
-      v.maxcos = cm;
+      v.maxcos = __uint_as_float(L.cmax);
       v.l2ni = L.bnorm[0];
       v.l2nj = L.bnorm[1];
       v.sweep = ctl->sweep;
@@ -453,7 +427,7 @@ __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pai
   }
   double *const wo = Wout + (size_t)pi * 4096u;
   for (unsigned e = tid; e < 4096u; e += VT)
-    wo[e] = RW(W, e & 63u, e >> 6);
+    wo[e] = RW(L.W, e & 63u, e >> 6);
 }
 
 // Block update M[:, pair] <- M[:, pair] W of the pairs of one step: a
