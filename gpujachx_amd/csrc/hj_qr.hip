@@ -1,43 +1,32 @@
 // hj_qr.hip -- the QR factorization of a block-pair visit and Drmac's sorted
 // level-0 (the reference's build options USE_QR and USE_DRMAC,
-// share/device_code_common.hpp:78-85,140-144), one wave per block pair.
+// share/device_code_common.hpp:78-85,140-144), one workgroup per block pair.
 //
-// Layout.  A 64-lane wave owns one pair.  Its LDS holds two 32x32 blocks,
-// R (the running triangular factor) and P (the panel being reduced; W once
-// the factorization is done), column-major with leading dimension 33: the
-// L0A layout of the Cholesky path, so that path's wave_level0 runs on them
-// unchanged.  Lanes form 16 quads; lane r of quad q holds rows r, r+4, ...,
-// r+28 of whatever column the quad works on, so a 32-row reduction is the
-// butterfly 16,8,4,2,1 with levels 16, 8, 4 inside the lane and 2, 1 by
-// quad DPP (sum4x8) -- the bits of the reference's 32-lane dSum32.  A single
-// wave needs no workgroup barrier: its LDS accesses complete in program
-// order, and wave_lds_sync() only keeps the compiler from moving them from
-// one phase into the next.
-//
-// The visit:
-//  * factorization by 32-row panels in order (dFactorize,
-//    share/device_code_common_QR.hpp:68-92): Householder QR of the first
-//    panel into R; for each further panel, its Householder QR into P, then
-//    R <- R of [R; P] by a wavefront of Givens rotations (dPeelOff, :4-66).
-//    A panel's global loads are issued before the previous panel's
-//    reduction, so they arrive while it runs.
-//      Householder step k (dQR32, share/device_code_common_Kepler.hpp:326-371):
-//      every quad forms the overflow-safe norm of column k itself (no
-//      broadcast), then quad q reflects columns k+1+q and k+17+q.
-//      Givens step k: lanes 0..31 each form the rotation of one row x >= k
-//      (with row x-k of P) into LDS; quad q then rotates columns k+q and
-//      k+16+q.
+// The visit, of eight waves with up to 16 panels of 32 rows in LDS (32x32,
+// column-major with leading dimension 33; beyond 512 rows, 15 more at a time):
+//  * the panels' Householder QR (dQR32,
+//    share/device_code_common_Kepler.hpp:326-371), each by a wave of its own:
+//    the panels do not depend on each other (householder32);
+//  * the panels' factors into the first's, in order (dPeelOff,
+//    share/device_code_common_QR.hpp:4-92), by a wavefront of Givens rotations:
+//    32 dependent rotations a panel, all that is serial here (merge_panel);
 //  * level-0: Drmac's sweeps for sorted definite blocks when asked
-//    (share/device_code_cdsort_Drmac.hpp:4-316), quad q taking pivot pair q
-//    of each step; otherwise the Cholesky path's wave_level0.
+//    (share/device_code_cdsort_Drmac.hpp:4-316; drmac_r), otherwise the
+//    Cholesky path's, four waves on R and four on W (hj_visit.hpp);
 //  * counters, the update flag and W to HBM; the block update is k_update's.
+// Reductions over 32 rows are the butterfly 16, 8, 4, 2, 1 of the reference's
+// dSum32, the first level or levels inside a lane.
 // This path is latency-bound; like the reference's, it is an accuracy option
-// for extremely graded column pairs, not a fast path.
+// for extremely graded column pairs, not a fast path.  Measured, 512 x 256
+// (16 panels a pair): Householder 70 us (two panels a wave), merges 150 us
+// (480 steps of 312 ns), level-0 32 us; 262 us a launch, where one wave a
+// pair, doing all of it in turn, took 1466 us.
 #include <climits>
 #include <cfloat>
 
 #include "hj_device.hpp"
 #include "hj_kernels.hpp"
+#include "hj_visit.hpp"
 
 namespace hj {
 namespace {
@@ -237,213 +226,352 @@ __device__ __forceinline__ void givens(double f, double g, double &c, double &s,
   const double af = fabs(f), ag = fabs(g);
   const bool fbig = af >= ag;
   const double big = fbig ? af : ag, small = fbig ? ag : af;
-  if (small == 0.0) {
-    r = big;
-    c = fbig ? copysign(1.0, f) : 0.0;
-    s = fbig ? 0.0 : copysign(1.0, g);
-    return;
-  }
+  const bool one = small == 0.0;  // one of the two is zero
   const double q = small / big;
-  r = big * sqrt(__fma_rn(q, q, 1.0));
-  c = f / r;
-  s = g / r;
+  r = one ? big : pin(big * sqrt(__fma_rn(q, q, 1.0)));
+  // (the quotients are issued side by side, also where they are not used)
+  const double cq = pin(f / r), sq = pin(g / r);
+  c = one ? (fbig ? copysign(1.0, f) : 0.0) : cq;
+  s = one ? (fbig ? 0.0 : copysign(1.0, g)) : sq;
 }
 
-// Householder QR of the 32x32 block A in place: for k = 0..30 the reflector
-// I - tau v v^T with v_k = 1, v_x = A(x,k) / (alpha + beta) below the
+// Sum of the 32 rows of a column held by 16 lanes, lane r holding rows row_of(r)
+// and row_of(r) + 16 as a, b: the butterfly 16, 8, 4, 2, 1.
+__device__ __forceinline__ double sum16x2(double a, double b)
+{
+  double s = a + b;
+  s = s + dpp_mov<0x128>(s);
+  s = s + dpp_mov<0x141>(s);
+  s = s + dpp_mov<0x4E>(s);
+  return s + dpp_mov<0xB1>(s);
+}
+
+// Whether x adds to a plain sum of squares (quad_ssq's middle band)
+__device__ __forceinline__ unsigned ssq_plain(double x)
+{
+  const double a = fabs(x);
+  const bool zero = x == 0.0, above = a >= SSQ_SMALL, below = a <= SSQ_BIG;
+  return (unsigned)zero | ((unsigned)above & (unsigned)below);
+}
+
+// ||A(k0:31, c)||_2 by quads (all of the wave's with the same column, or each
+// with its own): the norm of a column with entries outside the middle band
+__device__ __noinline__ double column_nrm2(const lds_f64 *A, unsigned c, unsigned k0, unsigned r4)
+{
+  double v[8];
+#pragma unroll
+  for (unsigned j = 0u; j < 8u; ++j) {
+    const unsigned x = r4 + 4u * j;
+    v[j] = (x >= k0) ? A[c * L0LD + x] : 0.0;
+  }
+  return quad_nrm2(v);
+}
+
+// Householder QR of the 32x32 block A in place by one wave: for k = 0..30 the
+// reflector I - tau v v^T with v_k = 1, v_x = A(x,k) / (alpha + beta) below the
 // diagonal, beta = sign(alpha) ||A(k:31,k)||, applied to columns k+1..31 as
 // A(:,c) += (-(tau v^T A(:,c))) v; column k becomes (-beta, 0, ..., 0).
-__device__ void householder32(double *A, unsigned q, unsigned r)
+// A step is bound by the instructions it issues: 16 lanes hold a column (two
+// rows each), so that the norm and the divisions, which every group does for
+// itself, are few, and four columns a group are updated side by side.
+__device__ void householder32(double *A_, unsigned l)
 {
+  lds_f64 *const A = (lds_f64 *)A_;
+  const unsigned g = l >> 4, x0 = row_of(l & 15u), x1 = x0 + 16u;
 #pragma unroll 1
   for (unsigned k = 0u; k < 31u; ++k) {
-    double v[8];
-#pragma unroll
-    for (unsigned j = 0u; j < 8u; ++j) {
-      const unsigned x = r + 4u * j;
-      const double a = L0A(A, x, k);
-      v[j] = (x >= k) ? a : 0.0;
-    }
-    const double nrm = quad_nrm2(v);
+    const double a0 = A[k * L0LD + x0], a1 = A[k * L0LD + x1];
+    const double alpha = A[k * L0LD + k];
+    double v0 = (x0 >= k) ? a0 : 0.0, v1 = (x1 >= k) ? a1 : 0.0;
+    double nrm = sqrt(sum16x2(v0 * v0, v1 * v1));
+    if (__ballot((ssq_plain(v0) & ssq_plain(v1)) == 0u) != 0ull)
+      nrm = column_nrm2(A, k, k, l & 3u);
     if (!(nrm > 0.0))
-      continue;  // the same in every lane: every quad holds column k
-    const double alpha = L0A(A, k, k);
+      continue;  // the same in every lane: every group holds column k
     // column k has been read by every lane before any lane writes it
     wave_lds_sync();
-    const double beta = copysign(nrm, alpha), ab = alpha + beta, tau = ab / beta;
+    const double beta = copysign(nrm, alpha), ab = alpha + beta;
+    // (the three quotients side by side)
+    const double tau = pin(ab / beta);
+    v0 = pin(v0 / ab);
+    v1 = pin(v1 / ab);
+    v0 = (x0 == k) ? 1.0 : ((x0 > k) ? v0 : 0.0);
+    v1 = (x1 == k) ? 1.0 : ((x1 > k) ? v1 : 0.0);
+#pragma unroll 1
+    for (unsigned c = k + 1u + g; c < 32u; c += 16u) {
+      double b0[4], b1[4], t[4];
 #pragma unroll
-    for (unsigned j = 0u; j < 8u; ++j) {
-      const unsigned x = r + 4u * j;
-      v[j] = (x == k) ? 1.0 : ((x > k) ? v[j] / ab : 0.0);
-    }
-    for (unsigned c = k + 1u + q; c < 32u; c += 16u) {
-      double a[8], pr[8];
-#pragma unroll
-      for (unsigned j = 0u; j < 8u; ++j) {
-        a[j] = L0A(A, r + 4u * j, c);
-        pr[j] = v[j] * a[j];
+      for (unsigned i = 0u; i < 4u; ++i) {
+        // (a column past the last: the last again, not stored)
+        const lds_f64 *const p = A + min(c + 4u * i, 31u) * L0LD;
+        b0[i] = p[x0];
+        b1[i] = p[x1];
       }
-      const double tdp = -(tau * sum4x8(pr));
 #pragma unroll
-      for (unsigned j = 0u; j < 8u; ++j)
-        L0A(A, r + 4u * j, c) = __fma_rn(tdp, v[j], a[j]);
-    }
-    if (q == 15u) {
+      for (unsigned i = 0u; i < 4u; ++i)
+        t[i] = v0 * b0[i] + v1 * b1[i];
 #pragma unroll
-      for (unsigned j = 0u; j < 8u; ++j) {
-        const unsigned x = r + 4u * j;
-        if (x >= k) L0A(A, x, k) = (x == k) ? -beta : 0.0;
+      for (unsigned i = 0u; i < 4u; ++i) t[i] = t[i] + dpp_mov<0x128>(t[i]);
+#pragma unroll
+      for (unsigned i = 0u; i < 4u; ++i) t[i] = t[i] + dpp_mov<0x141>(t[i]);
+#pragma unroll
+      for (unsigned i = 0u; i < 4u; ++i) t[i] = t[i] + dpp_mov<0x4E>(t[i]);
+#pragma unroll
+      for (unsigned i = 0u; i < 4u; ++i) t[i] = t[i] + dpp_mov<0xB1>(t[i]);
+#pragma unroll
+      for (unsigned i = 0u; i < 4u; ++i) {
+        const double tdp = -(tau * t[i]);
+        b0[i] = __fma_rn(tdp, v0, b0[i]);
+        b1[i] = __fma_rn(tdp, v1, b1[i]);
       }
+#pragma unroll
+      for (unsigned i = 0u; i < 4u; ++i) {
+        if (c + 4u * i < 32u) {
+          A[(c + 4u * i) * L0LD + x0] = b0[i];
+          A[(c + 4u * i) * L0LD + x1] = b1[i];
+        }
+      }
+    }
+    if (g == 3u) {
+      if (x0 >= k) A[k * L0LD + x0] = (x0 == k) ? -beta : 0.0;
+      if (x1 >= k) A[k * L0LD + x1] = (x1 == k) ? -beta : 0.0;
     }
     wave_lds_sync();
   }
 }
 
-// R0 <- the R factor of [R0; R1] for upper triangular R0, R1: at step k,
-// row x >= k of R0 meets row x-k of R1 in the rotation that zeroes R1(x-k, x)
-// against R0(x, x), applied to columns x..31 (products and sums rounded
-// separately).  gv: 96 doubles of LDS for the step's c, s, r.
-__device__ void merge_rows(double *R0, double *R1, double *gv, unsigned l, unsigned q, unsigned r)
+constexpr unsigned QR_WAVES = 8u;
+constexpr unsigned QR_NT = 64u * QR_WAVES;
+constexpr unsigned QR_LANES = QR_NT / 32u;  // lanes a pivot pair of level-0, R's and W's
+constexpr unsigned QR_PANELS = 16u;         // panels in LDS at once, the running factor among them
+constexpr unsigned QR_PANEL = 32u * L0LD;
+
+// LDS of a visit: the panels (the first is the running factor R, the second
+// becomes W), what inner_sweeps_by shares (see PairLds), the rotations of a
+// merge step by its parity
+struct QrLds {
+  static constexpr unsigned N = 32u, LD = L0LD;
+  static constexpr double TOL = MYTOL;
+  double R[QR_PANEL];
+  double W[QR_PANEL];
+  double panels[(QR_PANELS - 2u) * QR_PANEL];
+  double rot[2][16][4];
+  double gv[2][32][2];
+  unsigned act[2][16];
+  unsigned cs[2], cb[2];
+  unsigned cmax;
+  int swp;
+  __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
+};
+static_assert(offsetof(QrLds, W) == sizeof(double) * QR_PANEL &&
+                  offsetof(QrLds, panels) == sizeof(double) * 2u * QR_PANEL,
+              "the panels adjoin");
+
+// x of the lane before (lane 0: 0)
+__device__ __forceinline__ double lane_before(double x)
 {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// The R factor of [R; P1; P2; ...] for upper triangular panels, one after the
+// other, by the workgroup.  With the next panel P, at step k = 0..31 every row
+// x >= k of R meets row x-k of P in the rotation that zeroes P(x-k, x) against
+// R(x, x), applied to columns x..31 (products and sums rounded separately).
+// The chain is one rotation a step (a division, a root, a division) and what
+// brings the next step's operands: wave 0 keeps the diagonal and the two
+// diagonals above it in registers, lane x column x: step k's rotation, the
+// entries beside the diagonal by it (the lane before's: the next rotation's
+// P entry), and the second diagonal's by step k-1's, while the other waves
+// apply step k-1's to the entries further right, a thread an entry of R, which
+// stays in its register over all panels.  A barrier a step.
+struct Merge {
+  unsigned l, t;       // lane of wave 0's, thread of the others (wave 0: >= MERGE_ENTRIES)
+  unsigned x, col;     // the thread's entry of R
+  double A0, A1, A2;   // wave 0: R(x, x), R(x-1, x), R(x-2, x)
+  double a;            // others: R(x, col)
+};
+constexpr unsigned MERGE_ENTRIES = 29u * 30u / 2u;  // entries with col >= x + 3
+static_assert(MERGE_ENTRIES <= QR_NT - 64u, "a thread an entry");
+
+__device__ __forceinline__ void merge_begin(Merge &M, const QrLds &L, unsigned tid)
+{
+  const lds_f64 *const R = (const lds_f64 *)L.R;
+  M.l = min(tid, 64u);
+  M.t = tid < 64u ? MERGE_ENTRIES : tid - 64u;
+  // entries by column 3, 4, ..., column c with rows 0 .. c-3
+  unsigned c = 3u, off = 0u;
+  while (c < 31u && off + (c - 2u) <= M.t) {
+    off += c - 2u;
+    ++c;
+  }
+  M.col = tid < 64u ? (tid & 31u) : c;
+  M.x = tid < 64u ? (tid & 31u) : min(M.t - off, 31u);
+  // (read by every thread: a branch around the ones it does not use would
+  // keep them in memory)
+  M.A0 = R[M.x * L0LD + M.x];
+  M.A1 = R[M.x * L0LD + (M.x >= 1u ? M.x - 1u : 0u)];
+  M.A2 = R[M.x * L0LD + (M.x >= 2u ? M.x - 2u : 0u)];
+  M.a = R[M.col * L0LD + M.x];
+}
+
+__device__ __forceinline__ void merge_end(const Merge &M, QrLds &L)
+{
+  lds_f64 *const R = (lds_f64 *)L.R;
+  if (M.l < 32u) {
+    R[M.x * L0LD + M.x] = M.A0;
+    if (M.x >= 1u) R[M.x * L0LD + M.x - 1u] = M.A1;
+    if (M.x >= 2u) R[M.x * L0LD + M.x - 2u] = M.A2;
+  }
+  else if (M.t < MERGE_ENTRIES)
+    R[M.col * L0LD + M.x] = M.a;
+  __syncthreads();
+}
+
+// all threads of the workgroup; P synchronized
+__device__ __forceinline__ void merge_panel(Merge &M, QrLds &L, double *P_)
+{
+  lds_f64 *const P = (lds_f64 *)P_;
+  lds_f64 *const gv = (lds_f64 *)&L.gv[0][0][0];
+  if (M.l < 64u) {
+    const lds_f64 *const pc = P + M.x * L0LD;
+    double g = pc[M.x], c2 = 0.0, s2 = 0.0;
 #pragma unroll 1
-  for (unsigned k = 0u; k < 32u; ++k) {
-    if ((l < 32u) && (l >= k)) {
-      double c, s, rr;
-      givens(L0A(R0, l, l), L0A(R1, l - k, l), c, s, rr);
-      gv[l] = c;
-      gv[32u + l] = s;
-      gv[64u + l] = rr;
-    }
-    wave_lds_sync();
-    for (unsigned col = k + q; col < 32u; col += 16u) {
-#pragma unroll
-      for (unsigned j = 0u; j < 8u; ++j) {
-        const unsigned x = r + 4u * j;
-        if ((x < k) || (x > col)) continue;
-        if (x < col) {
-          const double c = gv[x], s = gv[32u + x];
-          const double a = L0A(R0, x, col), b = L0A(R1, x - k, col);
-          const double ca = c * a, sb = s * b, cb = c * b, sa = s * a;
-          L0A(R0, x, col) = ca + sb;
-          L0A(R1, x - k, col) = cb - sa;
-        }
-        else {
-          L0A(R0, x, col) = gv[64u + x];
-          L0A(R1, x - k, col) = 0.0;
-        }
+    for (unsigned k = 0u; k < 32u; ++k) {
+      const bool next = M.x > k;  // this lane rotates at step k+1
+      double b = pc[next ? M.x - k - 1u : 0u];
+      double c, s, r;
+      givens(M.A0, g, c, s, r);
+      if (M.x >= k) M.A0 = r;
+      if (M.l < 32u) {
+        gv[64u * (k & 1u) + 2u * M.x] = c;
+        gv[64u * (k & 1u) + 2u * M.x + 1u] = s;
       }
+      if (k) {
+        // the second diagonal's entry by step k-1's rotation of row x-2
+        const double ca = c2 * M.A2, sb = s2 * b, cb = c2 * b, sa = s2 * M.A2;
+        M.A2 = next ? ca + sb : M.A2;
+        b = cb - sa;
+      }
+      // the entry beside the diagonal by this step's rotation of row x-1
+      const double c1 = lane_before(c), s1 = lane_before(s);
+      const double ca = c1 * M.A1, sb = s1 * b, cb = c1 * b, sa = s1 * M.A1;
+      M.A1 = next ? ca + sb : M.A1;
+      g = cb - sa;
+      c2 = lane_before(c1);
+      s2 = lane_before(s1);
+      __syncthreads();
     }
-    wave_lds_sync();
+  }
+  else {
+    __syncthreads();
+#pragma unroll 1
+    for (unsigned k = 0u; k < 31u; ++k) {
+      if (M.t < MERGE_ENTRIES && M.x >= k) {
+        lds_f64 *const p = P + M.col * L0LD + M.x - k;
+        const double c = gv[64u * (k & 1u) + 2u * M.x], s = gv[64u * (k & 1u) + 2u * M.x + 1u];
+        const double b = *p;
+        const double ca = c * M.a, sb = s * b, cb = c * b, sa = s * M.a;
+        M.a = ca + sb;
+        *p = cb - sa;
+      }
+      __syncthreads();
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Drmac's sorted definite level-0 (posd for definite >= 0: the larger norm
-// first; negd: the smaller first), share/device_code_cdsort_Drmac.hpp:4-316.
-// The cosine of the pivot columns and their norms are formed overflow-safe;
-// the rotation comes from cot(2 phi) = (nq/np - np/nq) / (2 cos), and where
-// that exceeds COT_LIMIT the smaller column is made orthogonal to the larger
-// one directly.  Quad q takes pivot pair q of a step.
-__device__ void drmac_level0(double *R, double *W, const uint8_t *S0, unsigned s0steps,
-                             unsigned nswp, int definite, unsigned q, unsigned r,
-                             unsigned &out_s, unsigned &out_b)
+// One of Drmac's sorted definite level-0 sweeps on R (posd for definite >= 0:
+// the larger norm first; negd: the smaller first),
+// share/device_code_cdsort_Drmac.hpp:4-316: level0_r with other rotations.
+// The cosine of the pivot columns and their norms are formed overflow-safe
+// (wave by wave, by the plain sums where those are in range); the rotation
+// comes from cot(2 phi) = (nq/np - np/nq) / (2 cos), and where that exceeds
+// COT_LIMIT the smaller column is made orthogonal to the larger one directly.
+// W's columns take c = 1 and t = -+cos there.
+__device__ __forceinline__ void drmac_r(QrLds &L, unsigned y, unsigned r, unsigned s0steps,
+                                        int definite, unsigned &my_s, unsigned &my_b)
 {
+  constexpr unsigned LD = L0LD;
   const bool pos = (definite >= 0);
-  unsigned blk_s = 0u, blk_b = 0u;
-  for (unsigned swp = 0u; swp < nswp; ++swp) {
-    unsigned my_s = 0u, my_b = 0u;
-    for (unsigned step = 0u; step < s0steps; ++step) {
-      const unsigned p = S0[(step * 16u + q) * 2u], o = S0[(step * 16u + q) * 2u + 1u];
-      double Gp[8], Go[8], Vp[8], Vo[8];
-#pragma unroll
-      for (unsigned j = 0u; j < 8u; ++j) {
-        Gp[j] = L0A(R, r + 4u * j, p);
-        Go[j] = L0A(R, r + 4u * j, o);
-        Vp[j] = L0A(W, r + 4u * j, p);
-        Vo[j] = L0A(W, r + 4u * j, o);
-      }
-      const double Ap = quad_nrm2(Gp), Ao = quad_nrm2(Go);
-      const double cs = quad_cos(Ap, Ao, Gp, Go);
-      const int rot = (fabs(cs) >= MYTOL);
-      int big = 0;
-      if (rot) {
-        const double o_p = Ao / Ap, p_o = Ap / Ao;
-        const double ct2 = (o_p - p_o) / scalbn(cs, 1);
-        if (ct2 <= COT_LIMIT) {
-          const double act = fabs(ct2);
-          double c, t;
-          if (act < SQRT_HEPS) {
-            t = copysign(1.0 / (act + 1.0), ct2);
-            c = dev_rsqrt(__fma_rn(t, t, 1.0));
-            big = 1;
-          }
-          else if (act >= SQRT_2_HEPS) {
-            t = copysign(1.0 / scalbn(act, 1), ct2);
-            c = 1.0;
-          }
-          else {
-            t = copysign(1.0 / (act + sqrt(__fma_rn(act, act, 1.0))), ct2);
-            c = dev_rsqrt(__fma_rn(t, t, 1.0));
-            big = (c < 1.0);
-          }
-          const double tc = t * cs;
-          // the norms after the rotation decide which column goes first
-          const double Ap2 = Ap * sqrt(__fma_rn(-tc, o_p, 1.0));
-          const double Ao2 = Ao * sqrt(__fma_rn(tc, p_o, 1.0));
-          const bool keep = pos ? (Ap2 >= Ao2) : (Ap2 <= Ao2);
-          const unsigned P1 = keep ? p : o, P2 = keep ? o : p;
-#pragma unroll
-          for (unsigned j = 0u; j < 8u; ++j) {
-            const double rp = __fma_rn(-t, Go[j], Gp[j]), ro = __fma_rn(t, Gp[j], Go[j]);
-            const double wp = __fma_rn(-t, Vo[j], Vp[j]), wo = __fma_rn(t, Vp[j], Vo[j]);
-            L0A(R, r + 4u * j, P1) = big ? c * rp : rp;
-            L0A(R, r + 4u * j, P2) = big ? c * ro : ro;
-            L0A(W, r + 4u * j, P1) = big ? c * wp : wp;
-            L0A(W, r + 4u * j, P2) = big ? c * wo : wo;
-          }
-        }
-        else if (pos ? (Ap >= Ao) : (Ap <= Ao)) {
-          // column o loses its component along p; p stays first
-#pragma unroll
-          for (unsigned j = 0u; j < 8u; ++j) {
-            L0A(R, r + 4u * j, o) = Ao * __fma_rn(-cs, Gp[j] / Ap, Go[j] / Ao);
-            L0A(W, r + 4u * j, p) = __fma_rn(cs, Vo[j], Vp[j]);
-            L0A(W, r + 4u * j, o) = __fma_rn(-cs, Vp[j], Vo[j]);
-          }
-        }
-        else {
-          // column p loses its component along o, and the two change places
-#pragma unroll
-          for (unsigned j = 0u; j < 8u; ++j) {
-            L0A(R, r + 4u * j, o) = Ap * __fma_rn(-cs, Go[j] / Ao, Gp[j] / Ap);
-            L0A(R, r + 4u * j, p) = Go[j];
-            L0A(W, r + 4u * j, o) = __fma_rn(-cs, Vo[j], Vp[j]);
-            L0A(W, r + 4u * j, p) = __fma_rn(cs, Vp[j], Vo[j]);
-          }
-        }
-      }
-      else if (pos ? (Ap < Ao) : (Ao < Ap)) {
+  lds_f64 *const R = (lds_f64 *)L.R;
+  lds_f64 *const M = R + row_of(r);
+  const uint16_t *const S0 = reinterpret_cast<const uint16_t *>(L.S0) + y;
+#pragma unroll 1
+  for (unsigned step = 0u; step < s0steps; ++step) {
+    const unsigned pq = S0[16u * step], p = pq & 255u, q = pq >> 8;
+    lds_f64 *const ap = M + p * LD, *const aq = M + q * LD;
+    const double Gp[2] = {ap[0], ap[16]}, Gq[2] = {aq[0], aq[16]};
+    double Dp, Dq, cs;
+    dots3<16u>(Gp, Gq, Dp, Dq, cs);
+    double Ap = sqrt(Dp), Aq = sqrt(Dq);
+    {
+      const double nx = fmax(Ap, Aq), ny = fmin(Ap, Aq), nn = nx * ny;
+      const bool fits = nn < DBL_MAX, above = nn > PROD_SMALL;
+      cs = (cs / ny) / nx;
+      const unsigned plain = ssq_plain(Gp[0]) & ssq_plain(Gp[1]) & ssq_plain(Gq[0]) & ssq_plain(Gq[1]) &
+                         (unsigned)((ny >= 1.0) ? fits : above);
+      if (__ballot(plain == 0u) != 0ull) {
+        double vp[8], vq[8];
 #pragma unroll
         for (unsigned j = 0u; j < 8u; ++j) {
-          L0A(R, r + 4u * j, p) = Go[j];
-          L0A(R, r + 4u * j, o) = Gp[j];
-          L0A(W, r + 4u * j, p) = Vo[j];
-          L0A(W, r + 4u * j, o) = Vp[j];
+          vp[j] = R[p * LD + (r & 3u) + 4u * j];
+          vq[j] = R[q * LD + (r & 3u) + 4u * j];
+        }
+        Ap = column_nrm2(R, p, 0u, r & 3u);
+        Aq = column_nrm2(R, q, 0u, r & 3u);
+        cs = quad_cos(Ap, Aq, vp, vq);
+      }
+    }
+    const bool rot = (fabs(cs) >= MYTOL);
+    const double q_p = Aq / Ap, p_q = Ap / Aq;
+    const double ct2 = (q_p - p_q) / (2.0 * cs), act = fabs(ct2);
+    const bool ortho = rot & !(ct2 <= COT_LIMIT);
+    const bool small = act < SQRT_HEPS, large = act >= SQRT_2_HEPS;
+    const double sq = pin(sqrt(__fma_rn(act, act, 1.0)));
+    const double cot = large ? 2.0 * act : act + (small ? 1.0 : sq);
+    double t = copysign(1.0 / cot, ct2);
+    const double cr = rsqrt_near1(__fma_rn(t, t, 1.0));
+    const bool big = small | (!large & (cr < 1.0));
+    double c = big ? cr : 1.0;
+    const double tc = t * cs;
+    // the norms after the rotation decide which column goes first
+    const double Ap2 = Ap * sqrt(__fma_rn(-tc, q_p, 1.0));
+    const double Aq2 = Aq * sqrt(__fma_rn(tc, p_q, 1.0));
+    bool cross = rot ? !(pos ? (Ap2 >= Aq2) : (Ap2 <= Aq2)) : (pos ? (Ap < Aq) : (Aq < Ap));
+    // (a wave of nothing but rotations and swaps: no branch)
+    if (__ballot(ortho) == 0ull) {
+      apply_pair<16u, 2u, false>(ap, aq, Gp, Gq, rot, cross, true, c, t);
+    }
+    else {
+      if (ortho) {
+        // the smaller column loses its component along the larger, which
+        // stays or comes first
+        cross = !(pos ? (Ap >= Aq) : (Ap <= Aq));
+        c = 1.0;
+        t = cross ? cs : -cs;
+#pragma unroll
+        for (unsigned i = 0u; i < 2u; ++i) {
+          const double up = Gp[i] / Ap, uq = Gq[i] / Aq;
+          aq[16u * i] = cross ? Ap * __fma_rn(-cs, uq, up) : Aq * __fma_rn(-cs, up, uq);
+          if (cross) ap[16u * i] = Gq[i];
         }
       }
-      my_s += (unsigned)rot;
-      my_b += (unsigned)big;
-      wave_lds_sync();
+      else
+        apply_pair<16u, 2u, false>(ap, aq, Gp, Gq, rot, cross, true, c, t);
     }
-    // the four lanes of a quad hold its counts
-    const unsigned swp_s = wave_sum_u(my_s) >> 2, swp_b = wave_sum_u(my_b) >> 2;
-    if (!swp_s)
-      break;
-    blk_s += swp_s;
-    blk_b += swp_b;
+    if (r == 0u) {
+      double *const o = L.rot[step & 1u][y];
+      o[0] = c;
+      o[1] = t;
+      o[2] = o[3] = 0.0;
+      L.act[step & 1u][y] = (rot ? ACT_ROT : 0u) | (cross ? ACT_CROSS : 0u) | ACT_TRIG;
+    }
+    my_s += rot ? 1u : 0u;
+    my_b += (rot & !ortho & big) ? 1u : 0u;
+    __syncthreads();
   }
-  out_s = blk_s;
-  out_b = blk_b;
 }
 
 // ---------------------------------------------------------------------------
@@ -474,79 +602,88 @@ __device__ __forceinline__ void pair_signs(int definite, unsigned nplus, unsigne
   }
 }
 
-// One block pair per 64-lane workgroup.
+// One block pair per workgroup.
 template <bool SORT, bool DRMAC>
-__global__ __launch_bounds__(64) void k_pair_qr(const double *__restrict__ G, unsigned ldG,
-                                                unsigned nrow, const uint16_t *__restrict__ pairs,
-                                                double *__restrict__ Wout,
-                                                unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
-                                                const uint8_t *__restrict__ strat0, unsigned s0steps,
-                                                unsigned nswp, int definite, unsigned nplus)
+__global__ __launch_bounds__(QR_NT) void k_pair_qr(const double *__restrict__ G, unsigned ldG,
+                                                   unsigned nrow, const uint16_t *__restrict__ pairs,
+                                                   double *__restrict__ Wout,
+                                                   unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
+                                                   const uint8_t *__restrict__ strat0, unsigned s0steps,
+                                                   unsigned nswp, int definite, unsigned nplus)
 {
-  __shared__ double R[32u * L0LD];
-  __shared__ double P[32u * L0LD];
-  __shared__ double gv[96];
-  __shared__ __attribute__((aligned(16))) uint8_t S0[STRAT0_TAB_BYTES];
-  const unsigned l = threadIdx.x, q = l >> 2, r = l & 3u;
+  __shared__ QrLds L;
+  const unsigned tid = threadIdx.x, l = tid & 63u, w = tid >> 6;
   const unsigned pi = blockIdx.x;
   const unsigned bi = pairs[2u * pi], bj = pairs[2u * pi + 1u];
-  static_assert(STRAT0_TAB_BYTES == 64u * sizeof(uint4), "one 16-byte piece per lane");
-  reinterpret_cast<uint4 *>(S0)[l] = reinterpret_cast<const uint4 *>(strat0)[l];
+  static_assert(STRAT0_TAB_BYTES == 64u * sizeof(uint4), "one 16-byte piece per lane of a wave");
+  if (tid < 64u)
+    reinterpret_cast<uint4 *>(L.S0)[l] = reinterpret_cast<const uint4 *>(strat0)[l];
+  if (tid == 0u) {
+    L.swp = 0;
+    L.cmax = 0u;
+    L.cs[0] = L.cb[0] = 0u;
+  }
 
-  int def;
-  bool hyp;
-  unsigned npos;
-  pair_signs(definite, nplus, bi, bj, def, hyp, npos);
+  PairSigns sg;
+  pair_signs(definite, nplus, bi, bj, sg.def, sg.hyp, sg.npos);
 
   // panel loads: lane l takes row l % 32 of the pair's columns 2i + l / 32
   // (i < 8 in block bi, i >= 8 in block bj)
   const unsigned row = l & 31u, half = l >> 5;
   const double *const c0 = G + (size_t)(16u * bi + half) * ldG + row;
   const double *const c1 = G + (size_t)(16u * bj + half) * ldG + row;
-  auto load_panel = [&](double (&v)[16], unsigned i0) {
+  const unsigned npan = nrow / 32u;
+  Merge M;
+  // panels at .. at + n - 1 in slots s0 .. s0 + n - 1 (slot 0: the running
+  // factor), wave w those of slots w and w + 8
+  for (unsigned at = 0u, s0 = 0u; at < npan; s0 = 1u) {
+    const unsigned n = min(npan - at, QR_PANELS - s0);
+    double v[2][16];
 #pragma unroll
-    for (unsigned i = 0u; i < 16u; ++i)
-      v[i] = ((i < 8u) ? c0 : c1)[(size_t)(2u * (i & 7u)) * ldG + i0];
-  };
-  double pf[16];
-  load_panel(pf, 0u);
+    for (unsigned h = 0u; h < 2u; ++h) {
+      const unsigned sl = w + QR_WAVES * h;
+      if (sl >= s0 && sl < s0 + n) {
 #pragma unroll
-  for (unsigned i = 0u; i < 16u; ++i) L0A(R, row, 2u * i + half) = pf[i];
-  if (nrow > 32u)
-    load_panel(pf, 32u);
-  wave_lds_sync();
-  householder32(R, q, r);
-#pragma unroll 1
-  for (unsigned i0 = 32u; i0 < nrow; i0 += 32u) {
+        for (unsigned i = 0u; i < 16u; ++i)
+          v[h][i] = ((i < 8u) ? c0 : c1)[(size_t)(2u * (i & 7u)) * ldG + 32u * (at + sl - s0)];
+      }
+    }
 #pragma unroll
-    for (unsigned i = 0u; i < 16u; ++i) L0A(P, row, 2u * i + half) = pf[i];
-    if (i0 + 32u < nrow)
-      load_panel(pf, i0 + 32u);
+    for (unsigned h = 0u; h < 2u; ++h) {
+      const unsigned sl = w + QR_WAVES * h;
+      if (sl >= s0 && sl < s0 + n) {
+#pragma unroll
+        for (unsigned i = 0u; i < 16u; ++i)
+          L0A(L.R + sl * QR_PANEL, row, 2u * i + half) = v[h][i];
+      }
+    }
     wave_lds_sync();
-    householder32(P, q, r);
-    merge_rows(R, P, gv, l, q, r);
+#pragma unroll 1
+    for (unsigned sl = w; sl < s0 + n; sl += QR_WAVES)
+      if (sl >= s0) householder32(L.R + sl * QR_PANEL, l);
+    __syncthreads();
+    if (!s0) merge_begin(M, L, tid);
+#pragma unroll 1
+    for (unsigned sl = 1u; sl < s0 + n; ++sl)
+      merge_panel(M, L, L.R + sl * QR_PANEL);
+    at += n;
   }
+  merge_end(M, L);
   // W = I
-#pragma unroll
-  for (unsigned i = 0u; i < 16u; ++i) {
-    const unsigned c = 2u * i + half;
-    L0A(P, row, c) = (row == c) ? 1.0 : 0.0;
-  }
-  wave_lds_sync();
+  for (unsigned e = tid; e < 1024u; e += QR_NT)
+    L0A(L.W, e & 31u, e >> 5) = ((e & 31u) == (e >> 5)) ? 1.0 : 0.0;
+  __syncthreads();
 
-  unsigned blk_s = 0u, blk_b = 0u;
-  if (DRMAC && SORT && !hyp) {
-    drmac_level0(R, P, S0, s0steps, nswp, def, q, r, blk_s, blk_b);
-  }
-  else {
-    double unused_cos;
-    bool unused_swap;
-    wave_level0<SORT, false>(R, P, S0, s0steps, nswp, def, hyp, npos, l, blk_s, blk_b, unused_swap,
-                             unused_cos);
-  }
-  wave_lds_sync();
+  unsigned blk_s, blk_b;
+  if (DRMAC && SORT && !sg.hyp)
+    inner_sweeps_by<QR_LANES>(tid, L, s0steps, nswp, false, blk_s, blk_b,
+                              [&](unsigned y, unsigned r, unsigned &my_s, unsigned &my_b, bool &) {
+                                drmac_r(L, y, r, s0steps, sg.def, my_s, my_b);
+                              });
+  else
+    inner_sweeps<SORT, QR_LANES>(tid, L, sg, s0steps, nswp, false, blk_s, blk_b);
 
-  if (l == 0u) {
+  if (tid == 0u) {
     // the run's counter: big rotations in the high word, all in the low one;
     // without a big rotation only the low word is added to, with no carry
     // out of it (share/device_code_nosort.hpp:94-103)
@@ -557,11 +694,8 @@ __global__ __launch_bounds__(64) void k_pair_qr(const double *__restrict__ G, un
     flags[pi] = SORT ? 1u : (blk_s ? 1u : 0u);
   }
   double *const wo = Wout + (size_t)pi * 1024u;
-#pragma unroll
-  for (unsigned i = 0u; i < 16u; ++i) {
-    const unsigned c = 2u * i + half;
-    wo[c * 32u + row] = L0A(P, row, c);
-  }
+  for (unsigned e = tid; e < 1024u; e += QR_NT)
+    wo[e] = L0A(L.W, e & 31u, e >> 5);
 }
 
 }  // namespace
@@ -572,13 +706,13 @@ void launch_pair_qr(hipStream_t s, bool sort, bool drmac, const double *G, unsig
                     int definite, unsigned nplus)
 {
   if (sort && drmac)
-    hipLaunchKernelGGL((k_pair_qr<true, true>), dim3(np), dim3(64), 0, s, G, ldG, nrow, pairs, W,
+    hipLaunchKernelGGL((k_pair_qr<true, true>), dim3(np), dim3(QR_NT), 0, s, G, ldG, nrow, pairs, W,
                        flags, ctl, strat0, s0steps, nswp, definite, nplus);
   else if (sort)
-    hipLaunchKernelGGL((k_pair_qr<true, false>), dim3(np), dim3(64), 0, s, G, ldG, nrow, pairs, W,
+    hipLaunchKernelGGL((k_pair_qr<true, false>), dim3(np), dim3(QR_NT), 0, s, G, ldG, nrow, pairs, W,
                        flags, ctl, strat0, s0steps, nswp, definite, nplus);
   else
-    hipLaunchKernelGGL((k_pair_qr<false, false>), dim3(np), dim3(64), 0, s, G, ldG, nrow, pairs, W,
+    hipLaunchKernelGGL((k_pair_qr<false, false>), dim3(np), dim3(QR_NT), 0, s, G, ldG, nrow, pairs, W,
                        flags, ctl, strat0, s0steps, nswp, definite, nplus);
 }
 
