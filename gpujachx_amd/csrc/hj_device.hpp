@@ -270,6 +270,16 @@ __device__ __forceinline__ void dots3(const double *p, const double *q, double &
   level3<0xB1>(Dp, Dq, Apq);
 }
 
+// Whether |Apq| < sqrt(Dp) sqrt(Dq) tol is certain, as rounded, from the
+// squares alone: they say so by 2^-40, far more than the roundings of either
+// side, and none of them is near the ends of the exponent range.  (NaN: not.)
+__device__ __forceinline__ bool surely_orthogonal(double Apq, double Dp, double Dq, double tol)
+{
+  const double b = (Dp * Dq) * (tol * tol * (1.0 - 0x1p-40));
+  const bool less = Apq * Apq < b, above = b > 0x1p-960, below = b < 0x1p+1000;
+  return less & above & below;
+}
+
 // dev_rot for a pivot pair whose lanes (a multiple of four, from a multiple of
 // four on) all hold the same Apq, Dp, Dq: also sqrt(Dp) sqrt(Dq).  The three
 // square roots -- of zeta^2 +- 1, Dp and Dq -- are one instruction sequence,

@@ -34,6 +34,7 @@ struct PairLds {
 constexpr unsigned ACT_ROT = 1u;    // rotated
 constexpr unsigned ACT_CROSS = 2u;  // the results change places (with ACT_ROT or alone)
 constexpr unsigned ACT_TRIG = 4u;   // the rotation is trigonometric
+constexpr unsigned ACT_NORMS = 8u;  // no rotation: |p|^2 and |q|^2 in place of c and t
 
 // The columns of M (R or W) of a pivot pair after the step: lane l of the
 // pair's group holds rows row + LANES i as P[i], Q[i]; ap, aq: the first of
@@ -84,6 +85,7 @@ __device__ __forceinline__ void level0_r(Lds &L, unsigned y, unsigned r, unsigne
   const uint64_t neg0 = (!HYP && def < 0) ? 0x8000000000000000ull : 0ull;
   unsigned pq = S0[0];
   unsigned p = pq & 255u, q = pq >> 8, op = p * LD, oq = q * LD;
+  bool calm = false;
 #pragma unroll 1
   for (unsigned step = 0u; step < s0steps; ++step) {
     lds_f64 *const ap = M + op, *const aq = M + oq;
@@ -104,10 +106,33 @@ __device__ __forceinline__ void level0_r(Lds &L, unsigned y, unsigned r, unsigne
     }
     double Dp, Dq, Apq;
     dots3<LANES, ROWS>(Gp, Gq, Dp, Dq, Apq);
+    const double Apq_ = fabs(Apq);
+    // No pair of the wave rotates: at most swaps.  Asked only after a step
+    // without a rotation: the test would be in the chain of a step with one
+    // (40 of its 1490 cycles), and visits are calm or busy as a whole.
+    if (calm && __ballot(!surely_orthogonal(Apq, Dp, Dq, Lds::TOL)) == 0ull) {
+      const bool cross = SORT & inorder & (u2d(d2u(Dp) ^ neg) < u2d(d2u(Dq) ^ neg));
+      if (SORT && __ballot(cross) != 0ull) {
+        swapped = swapped | cross;
+        apply_pair<LANES, ROWS, HYP>(ap, aq, Gp, Gq, false, cross, trig, 1.0, 0.0);
+      }
+      if (r == 0u) {
+        double *const o = L.rot[step & 1u][y];
+        o[0] = Dp;
+        o[1] = Dq;
+        o[2] = Apq_;
+        L.act[step & 1u][y] = (cross ? ACT_CROSS : 0u) | ACT_NORMS;
+      }
+      p = pq & 255u;
+      q = pq >> 8;
+      op = pinu(p * LD);
+      oq = pinu(q * LD);
+      __syncthreads();
+      continue;
+    }
     // the rotation on every lane; only a transforming pair uses it
     double c, t, Dpq_;
     const bool big = rot_quad<HYP>(trig, Apq, Dp, Dq, r, c, t, Dpq_);
-    const double Apq_ = fabs(Apq);
     const bool transf = !(Apq_ < (Dpq_ * Lds::TOL));
     bool cross = false;
     if (SORT) {
@@ -130,6 +155,7 @@ __device__ __forceinline__ void level0_r(Lds &L, unsigned y, unsigned r, unsigne
     }
     my_s += transf ? 1u : 0u;
     my_b += (transf & big) ? 1u : 0u;
+    calm = __ballot(transf) == 0ull;
     p = pq & 255u;
     q = pq >> 8;
     op = pinu(p * LD);
@@ -154,20 +180,23 @@ __device__ __forceinline__ void level0_w(Lds &L, unsigned y, unsigned r, unsigne
     const unsigned pq = S0[PAIRS * step];
     const unsigned op = pinu((pq & 255u) * LD), oq = pinu((pq >> 8) * LD);
     __syncthreads();
-    lds_f64 *const ap = M + op, *const aq = M + oq;
-    double P[ROWS], Q[ROWS];
-#pragma unroll
-    for (unsigned i = 0u; i < ROWS; ++i) {
-      P[i] = ap[LANES * i];
-      Q[i] = aq[LANES * i];
-    }
     const double *const o = L.rot[step & 1u][y];
     const unsigned act = L.act[step & 1u][y];
-    const double cn = o[2], cd = o[3];
-    apply_pair<LANES, ROWS, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
-                            (act & ACT_TRIG) != 0u, o[0], o[1]);
-    if (cosines)
+    if (__ballot((act & (ACT_ROT | ACT_CROSS)) != 0u) != 0ull) {
+      lds_f64 *const ap = M + op, *const aq = M + oq;
+      double P[ROWS], Q[ROWS];
+#pragma unroll
+      for (unsigned i = 0u; i < ROWS; ++i) {
+        P[i] = ap[LANES * i];
+        Q[i] = aq[LANES * i];
+      }
+      apply_pair<LANES, ROWS, true>(ap, aq, P, Q, (act & ACT_ROT) != 0u, (act & ACT_CROSS) != 0u,
+                                    (act & ACT_TRIG) != 0u, o[0], o[1]);
+    }
+    if (cosines) {
+      const double cn = o[2], cd = (act & ACT_NORMS) ? sqrt(o[0]) * sqrt(o[1]) : o[3];
       my_cos = fmax(my_cos, (cd > 0.0) ? cn / cd : 0.0);
+    }
   }
   // (a nonnegative float's bits order as the float does)
   if (cosines && r == 0u)
