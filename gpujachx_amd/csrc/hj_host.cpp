@@ -911,8 +911,10 @@ static void level2_wide(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   uint8_t *d_s0 = nullptr;
   uint16_t *d_s1 = nullptr;
   HIP_CALL(hipMalloc(&d_part, sizeof(double) * (size_t)np * nchunk * wide_part_doubles()));
-  HIP_CALL(hipMalloc(&d_W, sizeof(double) * (size_t)np * 4096u));
-  HIP_CALL(hipMalloc(&d_flags, sizeof(unsigned) * np));
+  // W and the flags by step parity: V's update by a step's rides in the next
+  // step's visits' launch
+  HIP_CALL(hipMalloc(&d_W, sizeof(double) * (size_t)np * 4096u * 2u));
+  HIP_CALL(hipMalloc(&d_flags, sizeof(unsigned) * np * 2u));
   // the learned pair-skip at this width: the model and run-level policy of
   // the 16-column form, the records in its units
   const size_t nkeys = (size_t)np * steps;
@@ -969,19 +971,35 @@ static void level2_wide(unsigned routine, unsigned nrow, unsigned ncol, unsigned
     if (learned)
       launch_plan(s, d_rec, (unsigned)nkeys, d_s1, nplus, log2n1, max_rot, d_ctl, d_model, true,
                   d_plan, 32u);
+    VItems vlate;  // V's items of the step before (none when profiling)
     for (unsigned st = 0u; st < steps; ++st) {
       const uint16_t *const pairs = d_s1 + (size_t)st * np * 2u;
       const uint8_t *const plan = learned ? d_plan + (size_t)st * np : nullptr;
       hipEvent_t *const ev = g_profile ? evs.data() + (size_t)4u * st : nullptr;
+      double *const W = d_W + (size_t)(st & 1u) * np * 4096u;
+      unsigned *const flags = d_flags + (size_t)(st & 1u) * np;
       if (ev) HIP_CALL(hipEventRecord(ev[0], s));
       launch_gram_w(s, dG, lddG, pairs, np, nchunk, CH, d_part, plan);
       if (ev) HIP_CALL(hipEventRecord(ev[1], s));
-      launch_pair_w(s, cdsort, pairs, np, d_part, nchunk, d_W, d_flags, d_ctl, d_s0, t0.steps,
-                    nswp, definite, nplus, plan, learned ? d_rec + (size_t)st * np : nullptr);
+      launch_pair_w(s, cdsort, pairs, np, d_part, nchunk, W, flags, d_ctl, d_s0, t0.steps,
+                    nswp, definite, nplus, plan, learned ? d_rec + (size_t)st * np : nullptr, vlate);
       if (ev) HIP_CALL(hipEventRecord(ev[2], s));
-      launch_update_w(s, dG, lddG, nrow, pairs, np, d_W, d_flags);
-      if (V)
-        launch_update_w(s, V, lddV, ncol, pairs, np, d_W, d_flags);
+      launch_update_w(s, dG, lddG, nrow, pairs, np, W, flags);
+      if (V && (ev || st + 1u == steps)) {
+        launch_update_w(s, V, lddV, ncol, pairs, np, W, flags);
+        vlate = VItems();
+      }
+      else if (V) {
+        vlate.V = V;
+        vlate.ld = lddV;
+        vlate.nrow = ncol;
+        vlate.ch = 256u;
+        vlate.nch = (ncol + 255u) / 256u;
+        vlate.n = np * vlate.nch;
+        vlate.pairs = pairs;
+        vlate.W = W;
+        vlate.flags = flags;
+      }
       if (ev) HIP_CALL(hipEventRecord(ev[3], s));
     }
     HIP_CALL(hipMemcpyAsync(h_ctl, d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));

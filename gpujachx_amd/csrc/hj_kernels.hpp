@@ -190,18 +190,18 @@ void launch_initV(hipStream_t s, double *V, unsigned ifc, unsigned nRank, unsign
 
 // The wide-block form (hj_wide.hip): blocks of 32 columns, 64-column pairs;
 // Gram partials of wide_part_doubles() doubles per (pair, row chunk), W of
-// 64x64 per pair, the update in wide_update_chunks(nrow) workgroups a pair.
+// 64x64 per pair.
 unsigned wide_part_doubles();
-unsigned wide_update_chunks(unsigned nrow);
 // plan (null: every visit runs): the step's plans, skipped pairs get no Gram
-// and no visit; rec (null: none): the visits' records
+// and no visit; rec (null: none): the visits' records; v: the update of V by
+// the W of the step before, workgroups of v.ch rows, in the same launch
 void launch_gram_w(hipStream_t s, const double *G, unsigned ldG, const uint16_t *pairs,
                    unsigned np, unsigned nchunk, unsigned CH, double *part, const uint8_t *plan);
 void launch_pair_w(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np,
                    const double *part, unsigned nchunk, double *W, unsigned *flags,
                    RunCtl *ctl, const uint8_t *strat0, unsigned s0steps,
                    unsigned nswp, int definite, unsigned nplus, const uint8_t *plan,
-                   VisitRec *rec);
+                   VisitRec *rec, const VItems &v = VItems());
 void launch_update_w(hipStream_t s, double *M, unsigned ldM, unsigned nrow,
                      const uint16_t *pairs, unsigned np, const double *W,
                      const unsigned *flags);

@@ -138,6 +138,110 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   }
 }
 
+// The same partials where the sub-chunks are too few for a wave each to fill the
+// chip: four waves a sub-chunk, each with two or three of the ten tiles' chains
+// (the two diagonal 32x32 quarters and the rows of the other one), reading
+// 32-row panels of the pair's columns into LDS, the next one's loads in flight.
+// Workgroup (pair, chunk), NW sub-chunks.  A wave issues 64 cycles of FP64 MFMA
+// a tile and four rows; 4608 x 2048, whose 576-row chunks hold one sub-chunk
+// each (256 in all), 187 us a step with all ten tiles on a wave, 159 now.
+constexpr unsigned GTW_LD = 34u;  // padded panel column: operands in 32 different banks
+
+template <unsigned W>
+__device__ __forceinline__ void gram_w_tiles_panel(const lds_f64 *p, d4 *acc)
+{
+  // tile rows / columns of wave W's chains
+  constexpr unsigned TI[4][3] = {{0u, 1u, 1u}, {2u, 3u, 3u}, {2u, 2u, 0u}, {3u, 3u, 0u}};
+  constexpr unsigned TJ[4][3] = {{0u, 0u, 1u}, {2u, 2u, 3u}, {0u, 1u, 0u}, {0u, 1u, 0u}};
+  constexpr unsigned NTILE = W < 2u ? 3u : 2u;
+#pragma unroll
+  for (unsigned r = 0u; r < 32u; r += 4u)
+#pragma unroll
+    for (unsigned t = 0u; t < NTILE; ++t)
+      acc[t] = mfma(p[16u * GTW_LD * TI[W][t] + r], p[16u * GTW_LD * TJ[W][t] + r], acc[t]);
+}
+
+template <unsigned NW>
+__global__ __launch_bounds__(256u * NW) void k_gram_w_tiles(const double *__restrict__ G, unsigned ldG,
+                                                            const uint16_t *__restrict__ pairs,
+                                                            unsigned nchunk, unsigned CH,
+                                                            double *__restrict__ part,
+                                                            const uint8_t *__restrict__ plan)
+{
+  __shared__ union {
+    double P[NW][2][64u * GTW_LD];
+    d4 red[NW][WTILES][64];
+  } S;
+  const unsigned tid = threadIdx.x, l = tid & 63u, sub = tid >> 8, w = (tid >> 6) & 3u;
+  const unsigned pi = blockIdx.x / nchunk, c = blockIdx.x - pi * nchunk;
+  if (plan && plan[pi] == PLAN_SKIP)
+    return;  // a skipped visit needs no Gram
+  const unsigned a = pairs[2u * pi], b = pairs[2u * pi + 1u];
+  const unsigned SUB = CH / NW;
+  // wave w reads columns 2w + l/32 + 8k of the pair, row l % 32 of a panel
+  const size_t r0 = (size_t)c * CH + (size_t)sub * SUB + (l & 31u);
+  const unsigned cw = 2u * w + (l >> 5);
+  const double *const ga = G + (size_t)(32u * a + cw) * ldG + r0;
+  const double *const gb = G + (size_t)(32u * b + cw) * ldG + r0;
+  const size_t cs = (size_t)8u * ldG;
+  double x[8];
+#pragma unroll
+  for (unsigned k = 0u; k < 4u; ++k) {
+    x[k] = ga[k * cs];
+    x[4u + k] = gb[k * cs];
+  }
+  d4 acc[3];
+#pragma unroll
+  for (unsigned t = 0u; t < 3u; ++t)
+    acc[t] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (unsigned g = 0u, h = 0u; g < SUB; g += 32u, h ^= 1u) {
+    lds_f64 *const p = (lds_f64 *)S.P[sub][h];
+#pragma unroll
+    for (unsigned k = 0u; k < 8u; ++k)
+      p[(cw + 8u * k) * GTW_LD + (l & 31u)] = x[k];
+    if (g + 32u < SUB) {
+#pragma unroll
+      for (unsigned k = 0u; k < 4u; ++k) {
+        x[k] = ga[k * cs + g + 32u];
+        x[4u + k] = gb[k * cs + g + 32u];
+      }
+    }
+    // (two buffers: a wave writes this one again only after the next
+    // panel's barrier, when every wave has left it)
+    __syncthreads();
+    const lds_f64 *const o = p + (l & 15u) * GTW_LD + (l >> 4);
+    if (w == 0u) gram_w_tiles_panel<0u>(o, acc);
+    else if (w == 1u) gram_w_tiles_panel<1u>(o, acc);
+    else if (w == 2u) gram_w_tiles_panel<2u>(o, acc);
+    else gram_w_tiles_panel<3u>(o, acc);
+  }
+  // tile numbers of the wave's chains: i (i + 1) / 2 + j
+  const unsigned t0 = (w == 0u) ? 0u : (w == 1u) ? 5u : (w == 2u) ? 3u : 6u;
+  const unsigned t1 = (w == 0u) ? 1u : (w == 1u) ? 8u : (w == 2u) ? 4u : 7u;
+  const unsigned t2 = (w == 0u) ? 2u : 9u;
+  double *const o = part + (size_t)blockIdx.x * WPART + 4u * l;
+  if (NW == 1u) {
+    *reinterpret_cast<d4 *>(o + 256u * t0) = acc[0];
+    *reinterpret_cast<d4 *>(o + 256u * t1) = acc[1];
+    if (w < 2u) *reinterpret_cast<d4 *>(o + 256u * t2) = acc[2];
+    return;
+  }
+  // the sub-chunks' tiles added in order
+  __syncthreads();
+  S.red[sub][t0][l] = acc[0];
+  S.red[sub][t1][l] = acc[1];
+  if (w < 2u) S.red[sub][t2][l] = acc[2];
+  __syncthreads();
+  for (unsigned t = tid >> 6; t < WTILES; t += 4u * NW) {
+    d4 v = S.red[0][t][l];
+#pragma unroll
+    for (unsigned u = 1u; u < NW; ++u)
+      v = v + S.red[u][t][l];
+    *reinterpret_cast<d4 *>(o + 256u * t) = v;
+  }
+}
+
 constexpr unsigned VT = 512u;  // threads of a visit: half on R, half on W, 8 lanes a pivot pair
 
 // LDS of a 64-column pair visit
@@ -328,6 +432,85 @@ __device__ __forceinline__ PairSigns pair_signs32(int definite, unsigned nplus, 
   return s;
 }
 
+// Block update M[:, pair] <- M[:, pair] W of one pair's rows [rbeg, rend) by the
+// NT threads of a workgroup: W in LDS (Wl, row-major, padded), each
+// wave 16-row slabs of the chunk with the next slab's loads in flight.  Per
+// slab the MFMA chains run over k = 0..63 in order: A = W^T (lane l:
+// W(4u + l/16, 16h + l%16)), B = the slab's transpose (lane l:
+// M(row + l%16, column 4u + l/16)); lane l, register q of tile h holds
+// output column 16h + 4q + l/16 of row row + l%16.
+constexpr unsigned LDWW = 65u;
+
+template <unsigned NT>
+__device__ __forceinline__ void update_w_rows(double *Wl_, double *__restrict__ M, unsigned ldM,
+                                              unsigned rbeg, unsigned rend, unsigned a, unsigned b,
+                                              const double *__restrict__ Wp, unsigned tid)
+{
+  lds_f64 *const Wl = (lds_f64 *)Wl_;
+  const unsigned l = tid & 63u, w = tid >> 6;
+  constexpr unsigned STEP = NT / 4u;  // rows of all waves' slabs
+  for (unsigned e = tid; e < 4096u; e += NT)
+    Wl[(e & 63u) * LDWW + (e >> 6)] = Wp[e];  // Wl[k * LDWW + j] = W(k, j), at 64 j + k of Wp
+  __syncthreads();
+  // column 4u + l/16 of the pair: block a for u < 8, block b after
+  double *const ca = M + (size_t)(32u * a + (l >> 4)) * ldM + (l & 15u);
+  double *const cb = M + (size_t)(32u * b + (l >> 4)) * ldM + (l & 15u);
+  const lds_f64 *const wl = Wl + (l >> 4) * LDWW + (l & 15u);
+  unsigned row = rbeg + 16u * w;
+  double xn[16];
+  if (row < rend) {
+#pragma unroll
+    for (unsigned u = 0u; u < 8u; ++u) {
+      xn[u] = ca[(size_t)(4u * u) * ldM + row];
+      xn[8u + u] = cb[(size_t)(4u * u) * ldM + row];
+    }
+  }
+  for (; row < rend; row += STEP) {
+    double x[16];
+#pragma unroll
+    for (unsigned u = 0u; u < 16u; ++u)
+      x[u] = xn[u];
+    if (row + STEP < rend) {
+#pragma unroll
+      for (unsigned u = 0u; u < 8u; ++u) {
+        xn[u] = ca[(size_t)(4u * u) * ldM + row + STEP];
+        xn[8u + u] = cb[(size_t)(4u * u) * ldM + row + STEP];
+      }
+    }
+    d4 acc[4];
+#pragma unroll
+    for (unsigned h = 0u; h < 4u; ++h)
+      acc[h] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (unsigned u = 0u; u < 16u; ++u) {
+      const lds_f64 *const wr = wl + 4u * u * LDWW;
+#pragma unroll
+      for (unsigned h = 0u; h < 4u; ++h)
+        acc[h] = mfma(wr[16u * h], x[u], acc[h]);
+    }
+#pragma unroll
+    for (unsigned h = 0u; h < 4u; ++h)
+#pragma unroll
+      for (unsigned q = 0u; q < 4u; ++q)
+        ((h < 2u) ? ca : cb)[(size_t)(16u * (h & 1u) + 4u * q) * ldM + row] = acc[h][q];
+  }
+}
+
+// The pairs of one step, a workgroup per (pair, chunk of rows).  Pairs whose W is
+// the identity (flag 0) are left alone.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_update_w(
+    double *__restrict__ M, unsigned ldM, unsigned nrow, const uint16_t *__restrict__ pairs,
+    const double *__restrict__ Wbuf, const unsigned *__restrict__ flags, unsigned nchunk, unsigned rows)
+{
+  __shared__ double Wl[64u * LDWW];
+  const unsigned pi = blockIdx.x / nchunk, c = blockIdx.x - pi * nchunk;
+  if (!flags[pi])
+    return;
+  const unsigned rbeg = c * rows;
+  update_w_rows<256u>(Wl, M, ldM, rbeg, min(rbeg + rows, nrow), pairs[2u * pi], pairs[2u * pi + 1u],
+                      Wbuf + (size_t)pi * 4096u, threadIdx.x);
+}
+
 // One 64-column block pair per workgroup of 512 threads: chunk partials ->
 // R (lower), Cholesky, level-0 sweeps on R accumulating W, counters, W and
 // the update flag out.  The visit of 32 columns (hj_visit.hpp) at 64: four
@@ -349,10 +532,21 @@ __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pai
                                                 const uint8_t *__restrict__ strat0,
                                                 unsigned s0steps, unsigned nswp, int definite,
                                                 unsigned nplus, const uint8_t *__restrict__ plan,
-                                                VisitRec *__restrict__ rec)
+                                                VisitRec *__restrict__ rec, unsigned np, VItems V)
 {
   __shared__ PairLdsW L;
   const unsigned tid = threadIdx.x, pi = blockIdx.x;
+  if (pi >= np) {
+    // V by the W of the step before, on the CUs that no visit takes
+    static_assert(64u * LDWW <= 64u * LDRW, "W fits R");
+    const unsigned v = (pi - np) / V.nch, c = pi - np - v * V.nch;
+    if (!V.flags[v])
+      return;
+    const unsigned r0 = c * V.ch;
+    update_w_rows<VT>(L.R, V.V, V.ld, r0, min(r0 + V.ch, V.nrow), V.pairs[2u * v], V.pairs[2u * v + 1u],
+                      V.W + (size_t)v * 4096u, tid);
+    return;
+  }
   unsigned long long *const cvg = &ctl->cvg;
   if (plan && plan[pi] == PLAN_SKIP) {
     // skipped visit: no update, the record keeps the last executed visit
@@ -430,85 +624,43 @@ __global__ __launch_bounds__(512) void k_pair_w(const uint16_t *__restrict__ pai
     wo[e] = RW(L.W, e & 63u, e >> 6);
 }
 
-// Block update M[:, pair] <- M[:, pair] W of the pairs of one step: a
-// workgroup per (pair, 512-row chunk), W in LDS (row-major, padded), each
-// wave 16-row slabs of the chunk with the next slab's loads in flight.  Per
-// slab the MFMA chains run over k = 0..63 in order: A = W^T (lane l:
-// W(4u + l/16, 16h + l%16)), B = the slab's transpose (lane l:
-// M(row + l%16, column 4u + l/16)); lane l, register q of tile h holds
-// output column 16h + 4q + l/16 of row row + l%16.  Pairs whose W is the
-// identity (flag 0) are left alone.
-constexpr unsigned UPW_ROWS = 512u;
-constexpr unsigned LDWW = 65u;
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_update_w(
-    double *__restrict__ M, unsigned ldM, unsigned nrow, const uint16_t *__restrict__ pairs,
-    const double *__restrict__ Wbuf, const unsigned *__restrict__ flags, unsigned nchunk)
-{
-  __shared__ double Wl[64u * LDWW];
-  const unsigned pi = blockIdx.x / nchunk, c = blockIdx.x - pi * nchunk;
-  if (!flags[pi])
-    return;
-  const unsigned l = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  const unsigned a = pairs[2u * pi], b = pairs[2u * pi + 1u];
-  const double *const Wp = Wbuf + (size_t)pi * 4096u;  // W(k, j) at 64 j + k
-  for (unsigned e = threadIdx.x; e < 4096u; e += blockDim.x)
-    Wl[(e & 63u) * LDWW + (e >> 6)] = Wp[e];  // Wl[k * LDWW + j] = W(k, j)
-  __syncthreads();
-  const unsigned rbeg = c * UPW_ROWS, rend = min(rbeg + UPW_ROWS, nrow);
-  // column 4u + l/16 of the pair: block a for u < 8, block b after
-  double *const ca = M + (size_t)(32u * a + (l >> 4)) * ldM + (l & 15u);
-  double *const cb = M + (size_t)(32u * b + (l >> 4)) * ldM + (l & 15u);
-  const double *const wl = Wl + (l >> 4) * LDWW + (l & 15u);
-  unsigned row = rbeg + 16u * w;
-  double xn[16];
-  if (row < rend) {
-#pragma unroll
-    for (unsigned u = 0u; u < 8u; ++u) {
-      xn[u] = ca[(size_t)(4u * u) * ldM + row];
-      xn[8u + u] = cb[(size_t)(4u * u) * ldM + row];
-    }
-  }
-  for (; row < rend; row += 64u) {
-    double x[16];
-#pragma unroll
-    for (unsigned u = 0u; u < 16u; ++u)
-      x[u] = xn[u];
-    if (row + 64u < rend) {
-#pragma unroll
-      for (unsigned u = 0u; u < 8u; ++u) {
-        xn[u] = ca[(size_t)(4u * u) * ldM + row + 64u];
-        xn[8u + u] = cb[(size_t)(4u * u) * ldM + row + 64u];
-      }
-    }
-    d4 acc[4];
-#pragma unroll
-    for (unsigned h = 0u; h < 4u; ++h)
-      acc[h] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (unsigned u = 0u; u < 16u; ++u) {
-      const double *const wr = wl + 4u * u * LDWW;
-#pragma unroll
-      for (unsigned h = 0u; h < 4u; ++h)
-        acc[h] = mfma(wr[16u * h], x[u], acc[h]);
-    }
-#pragma unroll
-    for (unsigned h = 0u; h < 4u; ++h)
-#pragma unroll
-      for (unsigned q = 0u; q < 4u; ++q)
-        ((h < 2u) ? ca : cb)[(size_t)(16u * (h & 1u) + 4u * q) * ldM + row] = acc[h][q];
-  }
-}
-
 }  // namespace
 
 unsigned wide_part_doubles() { return WPART; }
-unsigned wide_update_chunks(unsigned nrow) { return (nrow + UPW_ROWS - 1u) / UPW_ROWS; }
+
+namespace {
+
+// Sub-chunks of a step up to which k_gram_w_tiles takes its Gram: one a SIMD.
+// Beyond, a wave each fills the chip.  Measured, us a step with k_gram_w /
+// k_gram_w_tiles: 1088 x 512 (16 sub-chunks) 200 / 145, 4608 x 2048 (256) 187
+// / 159, 6144 x 2048 (1024) 174 / 164, 4096 x 2048 (2048) 148 / 153, 8192 x
+// 4096 (4096) 273 / 283.
+constexpr unsigned GRAM_W_TILES_MAX = 1024u;
+
+// Rows a workgroup of k_update_w: two workgroups a CU (each brings W's 32 KB
+// with it), at most 512 rows.  Measured, us a step at one / two / four a CU:
+// 4608 x 2048 170 / 158 / 158, 4096 x 2048 153 / 146 / 148, 6144 x 4096 234 /
+// 234 / 245.
+unsigned update_w_rows_per_wg(unsigned nrow, unsigned np)
+{
+  unsigned rows = 512u;
+  while (rows > 64u && np * ((nrow + rows - 1u) / rows) < 512u)
+    rows /= 2u;
+  return rows;
+}
+
+}  // namespace
 
 void launch_gram_w(hipStream_t s, const double *G, unsigned ldG, const uint16_t *pairs,
                    unsigned np, unsigned nchunk, unsigned CH, double *part, const uint8_t *plan)
 {
   const unsigned nw = gram_waves(CH);
+  if (np * nchunk * nw <= GRAM_W_TILES_MAX) {
+    const auto k = (nw == 1u) ? k_gram_w_tiles<1u> : (nw == 2u) ? k_gram_w_tiles<2u> : k_gram_w_tiles<4u>;
+    hipLaunchKernelGGL(k, dim3(np * nchunk), dim3(256u * nw), 0, s, G, ldG, pairs, nchunk, CH, part,
+                       plan);
+    return;
+  }
   hipLaunchKernelGGL(k_gram_w, dim3(np * nchunk), dim3(64u * nw), 0, s, G, ldG, pairs, nchunk, CH,
                      part, plan);
 }
@@ -517,23 +669,20 @@ void launch_pair_w(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np,
                    const double *part, unsigned nchunk, double *W, unsigned *flags,
                    RunCtl *ctl, const uint8_t *strat0, unsigned s0steps,
                    unsigned nswp, int definite, unsigned nplus, const uint8_t *plan,
-                   VisitRec *rec)
+                   VisitRec *rec, const VItems &v)
 {
-  if (sort)
-    hipLaunchKernelGGL(k_pair_w<true>, dim3(np), dim3(VT), 0, s, pairs, part, nchunk, W, flags,
-                       ctl, strat0, s0steps, nswp, definite, nplus, plan, rec);
-  else
-    hipLaunchKernelGGL(k_pair_w<false>, dim3(np), dim3(VT), 0, s, pairs, part, nchunk, W, flags,
-                       ctl, strat0, s0steps, nswp, definite, nplus, plan, rec);
+  const auto k = sort ? k_pair_w<true> : k_pair_w<false>;
+  hipLaunchKernelGGL(k, dim3(np + v.n), dim3(VT), 0, s, pairs, part, nchunk, W, flags, ctl, strat0,
+                     s0steps, nswp, definite, nplus, plan, rec, np, v);
 }
 
 void launch_update_w(hipStream_t s, double *M, unsigned ldM, unsigned nrow,
                      const uint16_t *pairs, unsigned np, const double *W,
                      const unsigned *flags)
 {
-  const unsigned nch = wide_update_chunks(nrow);
+  const unsigned rows = update_w_rows_per_wg(nrow, np), nch = (nrow + rows - 1u) / rows;
   hipLaunchKernelGGL(k_update_w, dim3(np * nch), dim3(256), 0, s, M, ldM, nrow, pairs, W, flags,
-                     nch);
+                     nch, rows);
 }
 
 }  // namespace hj

@@ -37,3 +37,15 @@ def test_signs_and_row_counts(nplus, alg, m, n):
     rng = np.random.default_rng(m + nplus)
     rg, ro = _both(alg, rng.standard_normal((m, n)) * 10.0 ** rng.uniform(-3, 3, n), nplus)
     assert_same(rg, ro)
+
+
+# the Gram's tiles on waves of their own (1, 2 and 4 sub-chunks a chunk), one
+# wave a sub-chunk beyond 1024 of them, updates of 64 .. 512 rows a workgroup, V
+# beside the next visits over an odd number of steps
+@pytest.mark.parametrize("m,n,fam", [(576, 192, "mmstep"), (2048, 128, "cycwor"), (4096, 128, "rowcyc"),
+                                     (1024, 960, "mmstep"), (8192, 64, "cycwor"), (4096, 1024, "cycwor")])
+def test_launches_of_a_step(m, n, fam):
+    rng = np.random.default_rng(n)
+    G = rng.standard_normal((m, n)) * 10.0 ** rng.uniform(-1, 1, n)
+    rg, ro = _both(11, G, n // 3, fam=fam)
+    assert_same(rg, ro)
