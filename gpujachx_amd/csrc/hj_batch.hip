@@ -18,7 +18,9 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <functional>
 #include <numeric>
+#include <queue>
 #include <string>
 #include <vector>
 
@@ -34,11 +36,8 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 namespace hj {
 namespace {
 
-constexpr unsigned BLDR = L0LD;                       // padded leading dimension (the level-0 layout)
-// doubles per wave: R and W (the fused pass: the W of both pairs, LDW rows),
-// and the 16x16 transpose buffer of the fused pass's stores
-constexpr unsigned WAVE_LDS = 2u * 32u * BLDR + 16u * LDT;
-static_assert(BLDR == LDW, "the fused pass keeps its W copies in the R / W regions");
+constexpr unsigned BLDR = 36u;  // leading dimension of R and W in LDS (see wave_level0)
+constexpr unsigned WAVE_LDS = 2u * 32u * BLDR;  // doubles per wave
 constexpr unsigned BATCH_MAX_WAVES = 8u;
 // waves per SIMD the batch kernel is compiled for (register budget 512/n)
 #ifndef BATCH_WAVES_PER_SIMD
@@ -50,9 +49,7 @@ struct BProb {
   unsigned nrow, ncol, nplus, ldG, ldV, routine;
   unsigned s1off;  // first pair of this problem's strategy table in the pool
   unsigned steps, np;
-  unsigned qoff;  // first closed quad of this problem's table in the quad pool, or NO_QUADS
 };
-constexpr unsigned NO_QUADS = 0xFFFFFFFFu;
 
 struct BOut {
   unsigned sweeps, pad;
@@ -70,27 +67,48 @@ __device__ __forceinline__ d4 mfma64(double a, double b, d4 c)
 // Gram of the pair (columns 16 iBlk.., 16 jBlk..) over all nrow rows by one
 // wave: 16-row slabs in order, MFMA step j taking row 4j + k in k-slot k
 // (the order of the single-problem Gram with one chunk and one wave); result
-// into R (both 16x16 diagonal tiles and the lower off-diagonal tile).
+// into R (both 16x16 diagonal tiles and the lower off-diagonal tile).  A
+// 64-row panel is read 512 bytes of a column at a time, with the next panel's
+// loads in flight, and turned into operands through the wave's R and W
+// regions.  (Operands read from memory as they are wanted, 32 bytes of a
+// column a load, go to L2 four times: 110 us a pair of 1024 rows, 8 waves a
+// CU; 55 us now.)
+constexpr unsigned BGT_LD = 66u;  // padded panel column: operands in 32 different banks
+static_assert(32u * BGT_LD <= 2u * 32u * BLDR, "a panel fits R and W");
 __device__ void wave_gram(const double *__restrict__ G, unsigned ldG, unsigned nrow, unsigned iBlk,
                           unsigned jBlk, double *R, unsigned l)
 {
-  const unsigned r0 = l >> 4;
-  const double *const g0 = G + (size_t)(16u * iBlk + (l & 15u)) * ldG + r0;
-  const double *const g1 = G + (size_t)(16u * jBlk + (l & 15u)) * ldG + r0;
+  const double *const gi = G + (size_t)16u * iBlk * ldG + l, *const gj = G + (size_t)16u * jBlk * ldG + l;
+  lds_f64 *const p = (lds_f64 *)R + l;
+  const lds_f64 *const o = (const lds_f64 *)R + (l & 15u) * BGT_LD + (l >> 4);
   d4 a00 = {0.0, 0.0, 0.0, 0.0}, a10 = a00, a11 = a00;
-  for (unsigned g = 0u; g < nrow; g += 32u) {
-    double x0[8], x1[8];
+  double x[32];
 #pragma unroll
-    for (unsigned t = 0u; t < 8u; ++t) {
-      x0[t] = g0[g + 4u * t];
-      x1[t] = g1[g + 4u * t];
-    }
+  for (unsigned c = 0u; c < 16u; ++c) {
+    x[c] = gi[(size_t)c * ldG];
+    x[16u + c] = gj[(size_t)c * ldG];
+  }
+#pragma unroll 1
+  for (unsigned g = 0u; g < nrow; g += 64u) {
 #pragma unroll
-    for (unsigned t = 0u; t < 8u; ++t) {
-      a00 = mfma64(x0[t], x0[t], a00);
-      a10 = mfma64(x1[t], x0[t], a10);
-      a11 = mfma64(x1[t], x1[t], a11);
+    for (unsigned c = 0u; c < 32u; ++c)
+      p[c * BGT_LD] = x[c];
+    if (g + 64u < nrow) {
+#pragma unroll
+      for (unsigned c = 0u; c < 16u; ++c) {
+        x[c] = gi[(size_t)c * ldG + g + 64u];
+        x[16u + c] = gj[(size_t)c * ldG + g + 64u];
+      }
     }
+    wave_lds_sync();
+#pragma unroll
+    for (unsigned r = 0u; r < 64u; r += 4u) {
+      const double u = o[r], v = o[16u * BGT_LD + r];
+      a00 = mfma64(u, u, a00);
+      a10 = mfma64(v, u, a10);
+      a11 = mfma64(v, v, a11);
+    }
+    wave_lds_sync();
   }
   // lane l, register r holds element (4r + l/16, l%16) of each tile
 #pragma unroll
@@ -105,53 +123,59 @@ __device__ void wave_gram(const double *__restrict__ G, unsigned ldG, unsigned n
 // [M_i M_j] <- [M_i M_j] W over rows [0, nrow) by one wave, 16-row slabs
 // (the arithmetic of k_update: per element an fma chain over k = 0..31).
 __device__ void wave_update(double *__restrict__ M, unsigned ld, unsigned nrow, unsigned iBlk,
-                            unsigned jBlk, const double *W, unsigned l, unsigned wld)
+                            unsigned jBlk, const double *W, unsigned l)
 {
-  // W(k, j) at W[j * wld + k] (the LDS copy, wld = BLDR, or the scratch, 32)
   double a0[8], a1[8];
 #pragma unroll
   for (unsigned u = 0u; u < 8u; ++u) {
-    a0[u] = W[(l & 15u) * wld + 4u * u + (l >> 4)];
-    a1[u] = W[(16u + (l & 15u)) * wld + 4u * u + (l >> 4)];
+    a0[u] = W[(l & 15u) * BLDR + 4u * u + (l >> 4)];
+    a1[u] = W[(16u + (l & 15u)) * BLDR + 4u * u + (l >> 4)];
   }
-  double *cp[8];
+  // column 4u + l/16 of the pair: block i for u < 4, block j after; the output
+  // columns of register q are those of u = q and 4 + q
+  double *const ci = M + (size_t)(16u * iBlk + (l >> 4)) * ld + (l & 15u);
+  double *const cj = M + (size_t)(16u * jBlk + (l >> 4)) * ld + (l & 15u);
+  const size_t cs = (size_t)4u * ld;
+  // 32 rows an iteration (ncol is a multiple of 32, nrow of 64), the next ones
+  // in flight: a slab's MFMAs take half the time that its loads do
+  double nb[2][8];
 #pragma unroll
-  for (unsigned u = 0u; u < 8u; ++u) {
-    const unsigned cc = 4u * u + (l >> 4);
-    const unsigned gc = (cc < 16u) ? (16u * iBlk + cc) : (16u * jBlk + cc - 16u);
-    cp[u] = M + (size_t)gc * ld + (l & 15u);
-  }
-  double *op0[4], *op1[4];
+  for (unsigned h = 0u; h < 2u; ++h)
 #pragma unroll
-  for (unsigned q = 0u; q < 4u; ++q) {
-    const unsigned cc = 4u * q + (l >> 4);
-    op0[q] = M + (size_t)(16u * iBlk + cc) * ld + (l & 15u);
-    op1[q] = M + (size_t)(16u * jBlk + cc) * ld + (l & 15u);
-  }
-  double nb[8];
+    for (unsigned u = 0u; u < 4u; ++u) {
+      nb[h][u] = ci[u * cs + 16u * h];
+      nb[h][4u + u] = cj[u * cs + 16u * h];
+    }
+#pragma unroll 1
+  for (unsigned r = 0u; r < nrow; r += 32u) {
+    double b[2][8];
 #pragma unroll
-  for (unsigned u = 0u; u < 8u; ++u)
-    nb[u] = cp[u][0];
-  for (unsigned r = 0u; r < nrow; r += 16u) {
-    double b[8];
-#pragma unroll
-    for (unsigned u = 0u; u < 8u; ++u)
-      b[u] = nb[u];
-    if (r + 16u < nrow) {
+    for (unsigned h = 0u; h < 2u; ++h)
 #pragma unroll
       for (unsigned u = 0u; u < 8u; ++u)
-        nb[u] = cp[u][r + 16u];
-    }
-    d4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+        b[h][u] = nb[h][u];
+    if (r + 32u < nrow) {
 #pragma unroll
-    for (unsigned u = 0u; u < 8u; ++u) {
-      acc0 = mfma64(a0[u], b[u], acc0);
-      acc1 = mfma64(a1[u], b[u], acc1);
+      for (unsigned h = 0u; h < 2u; ++h)
+#pragma unroll
+        for (unsigned u = 0u; u < 4u; ++u) {
+          nb[h][u] = ci[u * cs + r + 32u + 16u * h];
+          nb[h][4u + u] = cj[u * cs + r + 32u + 16u * h];
+        }
     }
 #pragma unroll
-    for (unsigned q = 0u; q < 4u; ++q) {
-      op0[q][r] = acc0[q];
-      op1[q][r] = acc1[q];
+    for (unsigned h = 0u; h < 2u; ++h) {
+      d4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = acc0;
+#pragma unroll
+      for (unsigned u = 0u; u < 8u; ++u) {
+        acc0 = mfma64(a0[u], b[h][u], acc0);
+        acc1 = mfma64(a1[u], b[h][u], acc1);
+      }
+#pragma unroll
+      for (unsigned q = 0u; q < 4u; ++q) {
+        ci[q * cs + r + 16u * h] = acc0[q];
+        cj[q * cs + r + 16u * h] = acc1[q];
+      }
     }
   }
 }
@@ -197,15 +221,13 @@ __device__ __noinline__ void wave_visit(const BProb &P, unsigned iBlk, unsigned 
   // slot holding rows l%4 + 4k)
   unsigned blk_s = 0u, blk_b = 0u;
   bool swapped = false;
-  double cos_unused = 0.0;
-  wave_level0<SORT, false>(R, W, S0, s0steps, nswp, def, hyp, npos, l, blk_s, blk_b, swapped,
-                           cos_unused);
+  wave_level0<SORT, BLDR>(R, W, S0, s0steps, nswp, def, hyp, npos, l, blk_s, blk_b, swapped);
   out_s = blk_s;
   out_b = blk_b;
   out_upd = (blk_s != 0u) || swapped;
 }
 
-// One block pair by one wave: Gram, visit, update (the unfused step).
+// One block pair by one wave: Gram, visit, update.
 template <bool SORT>
 __device__ void wave_pair(const BProb &P, unsigned iBlk, unsigned jBlk, double *R, double *W,
                           const uint8_t *S0, unsigned s0steps, unsigned nswp, int definite,
@@ -216,71 +238,9 @@ __device__ void wave_pair(const BProb &P, unsigned iBlk, unsigned jBlk, double *
   bool upd = false;
   wave_visit<SORT>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, out_s, out_b, upd);
   if (upd) {
-    wave_update(P.G, P.ldG, P.nrow, iBlk, jBlk, W, l, BLDR);
+    wave_update(P.G, P.ldG, P.nrow, iBlk, jBlk, W, l);
     if (P.routine & HYPJAC_FULL_SVD)
-      wave_update(P.V, P.ldV, P.ncol, iBlk, jBlk, W, l, BLDR);
-  }
-}
-
-// Gram tiles of a pair (00, 10, 11; lane l, register r at l*4 + r, the MFMA
-// output layout) from the fused pass's scratch into R, as wave_gram leaves
-// them
-__device__ __forceinline__ void gram_to_R(const double *__restrict__ g, double *R, unsigned l)
-{
-#pragma unroll
-  for (unsigned r = 0u; r < 4u; ++r) {
-    const unsigned i = 4u * r + (l >> 4), j = l & 15u;
-    BR(R, i, j) = g[l * 4u + r];
-    BR(R, 16u + i, j) = g[256u + l * 4u + r];
-    BR(R, 16u + i, 16u + j) = g[512u + l * 4u + r];
-  }
-}
-
-// The fused transition of a closed quad by one wave over all rows: the
-// update of both pairs of step s (W0, W1 in LDS, W(k, j) at k*LDW + j) and
-// the Gram of both pairs of step s+1 from the updated values in registers,
-// in the single-wave Gram's order (16-row slabs ascending), to g0, g1.
-__device__ void wave_upgram(double *__restrict__ G, unsigned ldG, unsigned nrow, unsigned A0,
-                            unsigned B0, unsigned A1, unsigned B1, bool u0, bool u1, const Quad &Q,
-                            const double *W0, const double *W1, double *T, unsigned l,
-                            double *__restrict__ g0, double *__restrict__ g1)
-{
-  d4 z = {0.0, 0.0, 0.0, 0.0};
-  d4 g00 = z, g10 = z, g11 = z, h00 = z, h10 = z, h11 = z;
-  double xa[8], xb[8];
-  slab_load<true>(G, ldG, 0u, A0, B0, u0, l, xa);
-  slab_load<true>(G, ldG, 0u, A1, B1, u1, l, xb);
-  for (unsigned r = 0u; r < nrow; r += 16u) {
-    double ca[8], cb[8];
-#pragma unroll
-    for (unsigned u = 0u; u < 8u; ++u) {
-      ca[u] = xa[u];
-      cb[u] = xb[u];
-    }
-    if (r + 16u < nrow) {
-      slab_load<true>(G, ldG, r + 16u, A0, B0, u0, l, xa);
-      slab_load<true>(G, ldG, r + 16u, A1, B1, u1, l, xb);
-    }
-    d4 t0, t1, t2, t3;
-    slab_compute<true>(G, ldG, r, A0, B0, u0, W0, l, ca, t0, t1, T);
-    slab_compute<true>(G, ldG, r, A1, B1, u1, W1, l, cb, t2, t3, T);
-    {
-      const d4 X = sel4(Q.x0, t0, t1, t2, t3), Y = sel4(Q.y0, t0, t1, t2, t3);
-      gram_fp64_slab(X, Y, g00, g10, g11);
-    }
-    {
-      const d4 X = sel4(Q.x1, t0, t1, t2, t3), Y = sel4(Q.y1, t0, t1, t2, t3);
-      gram_fp64_slab(X, Y, h00, h10, h11);
-    }
-  }
-#pragma unroll
-  for (unsigned r = 0u; r < 4u; ++r) {
-    g0[l * 4u + r] = g00[r];
-    g0[256u + l * 4u + r] = g10[r];
-    g0[512u + l * 4u + r] = g11[r];
-    g1[l * 4u + r] = h00[r];
-    g1[256u + l * 4u + r] = h10[r];
-    g1[512u + l * 4u + r] = h11[r];
+      wave_update(P.V, P.ldV, P.ncol, iBlk, jBlk, W, l);
   }
 }
 
@@ -294,10 +254,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BATCH_WAVES
                                                unsigned *__restrict__ queue,
                                                const uint16_t *__restrict__ s1pool,
                                                const uint8_t *__restrict__ strat0, unsigned s0steps,
-                                               unsigned max_sweeps, BOut *__restrict__ out,
-                                               const Quad *__restrict__ qpool,
-                                               double *__restrict__ scr,
-                                               unsigned *__restrict__ sflags, unsigned np_max)
+                                               unsigned max_sweeps, BOut *__restrict__ out)
 {
   extern __shared__ double lds[];
   __shared__ uint8_t S0[1024];
@@ -306,12 +263,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BATCH_WAVES
   const unsigned l = threadIdx.x & 63u, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
   double *const R = lds + (size_t)wv * WAVE_LDS;
   double *const W = R + 32u * BLDR;
-  double *const T = W + 32u * BLDR;
-  // this workgroup's scratch of the fused steps: the Grams of the next
-  // step's pairs, the W and update flags of the running step's pairs
-  double *const sg = scr + (size_t)blockIdx.x * np_max * (768u + 1024u);
-  double *const sw = sg + (size_t)np_max * 768u;
-  unsigned *const sf = sflags + (size_t)blockIdx.x * np_max;
   for (unsigned e = threadIdx.x; e < s0steps * 32u; e += blockDim.x)
     S0[e] = strat0[e];
   for (;;) {
@@ -346,88 +297,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(BATCH_WAVES
       unsigned sw_s = 0u, sw_b = 0u;
       for (unsigned st = 0u; st < P.steps; ++st) {
         __syncthreads();
-        const bool fused = (P.qoff != NO_QUADS) && (st + 1u < P.steps);
-        if (!fused && (P.qoff == NO_QUADS || st == 0u)) {
-          // unfused step: each wave's pairs, Gram -> visit -> update
-          for (unsigned pi = wv; pi < P.np; pi += nw) {
-            const unsigned iBlk = tab[2u * (st * P.np + pi)], jBlk = tab[2u * (st * P.np + pi) + 1u];
-            unsigned s = 0u, b = 0u;
-            if (sort)
-              wave_pair<true>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b);
-            else
-              wave_pair<false>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b);
-            sw_s += s;
-            sw_b += b;
-          }
-          continue;
-        }
-        // fused steps: the visits (Gram of step 0 from G, later ones from
-        // the previous transition's pass), then one pass per closed quad
-        // updating both pairs and forming the next step's Grams; the last
-        // step of a sweep updates after each visit
         for (unsigned pi = wv; pi < P.np; pi += nw) {
           const unsigned iBlk = tab[2u * (st * P.np + pi)], jBlk = tab[2u * (st * P.np + pi) + 1u];
-          if (st == 0u)
-            wave_gram(P.G, P.ldG, P.nrow, iBlk, jBlk, R, l);
-          else
-            gram_to_R(sg + (size_t)pi * 768u, R, l);
-          wave_lds_sync();
           unsigned s = 0u, b = 0u;
-          bool upd = false;
           if (sort)
-            wave_visit<true>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b, upd);
+            wave_pair<true>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b);
           else
-            wave_visit<false>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b, upd);
+            wave_pair<false>(P, iBlk, jBlk, R, W, S0, s0steps, nswp, definite, l, s, b);
           sw_s += s;
           sw_b += b;
-          if (!fused) {
-            if (upd) {
-              wave_update(P.G, P.ldG, P.nrow, iBlk, jBlk, W, l, BLDR);
-              if (full)
-                wave_update(P.V, P.ldV, P.ncol, iBlk, jBlk, W, l, BLDR);
-            }
-          }
-          else {
-            double *const w = sw + (size_t)pi * 1024u;
-#pragma unroll
-            for (unsigned e = 0u; e < 16u; ++e) {
-              const unsigned k = l + 64u * e;
-              w[k] = BR(W, k & 31u, k >> 5);
-            }
-            if (l == 0u)
-              sf[pi] = upd ? 1u : 0u;
-          }
-          wave_lds_sync();
-        }
-        if (!fused)
-          continue;
-        __syncthreads();
-        const unsigned nq = P.np / 2u;
-        const Quad *const Qs = qpool + P.qoff + (size_t)st * nq;
-        for (unsigned qi = wv; qi < nq; qi += nw) {
-          const Quad Q = Qs[qi];
-          const unsigned A0 = tab[2u * (st * P.np + Q.p0)], B0 = tab[2u * (st * P.np + Q.p0) + 1u];
-          const unsigned A1 = tab[2u * (st * P.np + Q.p1)], B1 = tab[2u * (st * P.np + Q.p1) + 1u];
-          const bool u0 = sf[Q.p0] != 0u, u1 = sf[Q.p1] != 0u;
-          const double *const w0 = sw + (size_t)Q.p0 * 1024u;
-          const double *const w1 = sw + (size_t)Q.p1 * 1024u;
-          // W(k, j) of both pairs into this wave's R / W regions (k * LDW + j)
-#pragma unroll
-          for (unsigned e = 0u; e < 16u; ++e) {
-            const unsigned k = l + 64u * e;
-            R[(k & 31u) * LDW + (k >> 5)] = w0[k];
-            W[(k & 31u) * LDW + (k >> 5)] = w1[k];
-          }
-          wave_lds_sync();
-          wave_upgram(P.G, P.ldG, P.nrow, A0, B0, A1, B1, u0, u1, Q, R, W, T, l,
-                      sg + (size_t)Q.n0 * 768u, sg + (size_t)Q.n1 * 768u);
-          if (full) {
-            if (u0)
-              wave_update(P.V, P.ldV, P.ncol, A0, B0, w0, l, 32u);
-            if (u1)
-              wave_update(P.V, P.ldV, P.ncol, A1, B1, w1, l, 32u);
-          }
-          wave_lds_sync();
         }
       }
       if (l == 0u) {
@@ -497,10 +375,6 @@ struct Plan {
   BProb *d_probs = nullptr;
   unsigned *d_order = nullptr, *d_queue = nullptr;
   uint16_t *d_pool = nullptr;
-  Quad *d_quads = nullptr;       // closed quads of the fusable tables
-  double *d_scr = nullptr;       // per workgroup: Grams and W of the fused steps
-  unsigned *d_sflags = nullptr;  // per workgroup: update flags of the fused steps
-  unsigned np_max = 1u;
   uint8_t *d_s0 = nullptr;
   unsigned s0steps = 0u;
   BOut *d_out = nullptr;
@@ -512,6 +386,49 @@ struct Plan {
   size_t lds = 0u;
   double clock_mhz = 100.0;
 };
+
+constexpr unsigned DEFAULT_WAVES = 4u, DEFAULT_WG_PER_CU = 2u;
+
+// The shape of a batch whose caller left it to the library (the default
+// configuration): eight wave slots a CU as one workgroup of eight waves, two of
+// four or four of two, whichever ends first when the problems, in queue order,
+// go to the next free workgroup.  A wide workgroup brings the largest problems,
+// which end last, to their end; narrow ones waste no slots on small problems.
+// A problem's time: its steps times the rounds of pairs its waves take, a pair
+// costing 80 us and 8.5 (G) and 5 us (V) per 64 rows with eight waves of the CU
+// busy, half of that alone.  Measured, ms at 8 x 1 / 4 x 2 / 2 x 4: 384
+// problems of up to 512 columns with V 112 / 182 / 323, 1200 of them 189 / 235
+// / 351, 384 of up to 128 3.2 / 4.2 / 7.6, 2048 of up to 256 with V 54 / 52 /
+// 58, 4096 of up to 128 with V 28 / 21 / 20, 4096 of 64 12.7 / 8.1 / 5.4.
+void choose_shape(hj_batch_cfg &cfg, const std::vector<BProb> &probs,
+                  const std::vector<unsigned> &order, unsigned ncu)
+{
+  const unsigned shapes[][2] = {{4u, 2u}, {8u, 1u}, {2u, 4u}};
+  double best = 0.0;
+  for (const auto &sh : shapes) {
+    const unsigned w = sh[0], g = sh[1], slots = g * ncu;
+    const unsigned resident = std::min(g, (unsigned)((probs.size() + ncu - 1u) / ncu));
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
+    double end = 0.0;
+    for (unsigned pid : order) {
+      const BProb &b = probs[pid];
+      const double t = 80.0 + b.nrow / 64.0 * 8.5 + (b.V ? b.ncol / 64.0 * 5.0 : 0.0);
+      const double busy = std::min(1.0, std::min(b.np, w) * resident / 8.0);
+      double at = (double)b.steps * ((b.np + w - 1u) / w) * t * (0.5 + 0.5 * busy);
+      if (free_at.size() >= slots) {
+        at += free_at.top();
+        free_at.pop();
+      }
+      free_at.push(at);
+      end = std::max(end, at);
+    }
+    if (best == 0.0 || end < best) {
+      best = end;
+      cfg.waves = w;
+      cfg.wg_per_cu = g;
+    }
+  }
+}
 
 double cost_of(const hj_batch_desc &d)
 {
@@ -527,8 +444,8 @@ using namespace hj;
 extern "C" void hj_batch_default_cfg(hj_batch_cfg *cfg)
 {
   if (!cfg) return;
-  cfg->waves = 4u;
-  cfg->wg_per_cu = 2u;
+  cfg->waves = DEFAULT_WAVES;
+  cfg->wg_per_cu = DEFAULT_WG_PER_CU;
   cfg->strategy = HJ_BATCH_STRAT_CYCWOR;
   cfg->max_sweeps = HYPJAC_NSWEEP;
   cfg->longest_first = 1u;
@@ -573,10 +490,8 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   P->cfg = cfg;
   // strategy tables: one per distinct (family, n1)
   std::vector<uint16_t> pool;
-  std::vector<Quad> qpool;
   std::vector<std::pair<std::string, unsigned>> keys;
-  std::vector<unsigned> key_off, key_steps, key_qoff;
-  const bool nofuse = getenv("HJ_BATCH_NOFUSE") != nullptr;
+  std::vector<unsigned> key_off, key_steps;
   P->h_probs.resize(n);
   for (unsigned i = 0u; i < n; ++i) {
     const hj_batch_desc &d = probs[i];
@@ -593,15 +508,6 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
       keys.push_back({fam, n1});
       key_off.push_back((unsigned)(pool.size() / 2u));
       key_steps.push_back(t.steps);
-      // fused steps when every transition of the table has closed quads
-      std::vector<uint16_t> flat(t.tab.begin(), t.tab.end());
-      std::vector<Quad> q;
-      std::vector<char> closed;
-      bool all = !nofuse && closed_quads(flat.data(), t.steps, t.pairs, q, &closed);
-      for (unsigned st = 0u; all && st + 1u < t.steps; ++st)
-        all = closed[st] != 0;
-      key_qoff.push_back(all ? (unsigned)qpool.size() : NO_QUADS);
-      if (all) qpool.insert(qpool.end(), q.begin(), q.end());
       pool.insert(pool.end(), t.tab.begin(), t.tab.end());
     }
     BProb b;
@@ -617,8 +523,6 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
     b.s1off = key_off[k];
     b.steps = key_steps[k];
     b.np = n1 / 2u;
-    b.qoff = key_qoff[k];
-    P->np_max = std::max(P->np_max, b.np);
     P->h_probs[i] = b;
   }
   std::vector<unsigned> order(n);
@@ -643,15 +547,14 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   HIP_CALL(hipMemcpy(P->d_order, order.data(), sizeof(unsigned) * n, hipMemcpyHostToDevice));
   HIP_CALL(hipMemcpy(P->d_pool, pool.data(), sizeof(uint16_t) * pool.size(), hipMemcpyHostToDevice));
   HIP_CALL(hipMemcpy(P->d_s0, s0b.data(), 1024u, hipMemcpyHostToDevice));
-  HIP_CALL(hipMalloc(&P->d_quads, sizeof(Quad) * std::max<size_t>(qpool.size(), 1u)));
-  if (!qpool.empty())
-    HIP_CALL(hipMemcpy(P->d_quads, qpool.data(), sizeof(Quad) * qpool.size(), hipMemcpyHostToDevice));
   P->h_out.resize(n);
 
   int dev = 0;
   HIP_CALL(hipGetDevice(&dev));
   hipDeviceProp_t prop;
   HIP_CALL(hipGetDeviceProperties(&prop, dev));
+  if (cfg.waves == DEFAULT_WAVES && cfg.wg_per_cu == DEFAULT_WG_PER_CU)
+    choose_shape(cfg, P->h_probs, order, (unsigned)prop.multiProcessorCount);
   P->grid = cfg.wg_per_cu * (unsigned)prop.multiProcessorCount;
   P->lds = sizeof(double) * WAVE_LDS * cfg.waves;
   const size_t lds_max = std::max(prop.sharedMemPerBlock, prop.sharedMemPerBlockOptin);
@@ -664,8 +567,6 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   }
   HIP_CALL(hipFuncSetAttribute(reinterpret_cast<const void *>(k_batch),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->lds));
-  HIP_CALL(hipMalloc(&P->d_scr, sizeof(double) * (768u + 1024u) * P->np_max * P->grid));
-  HIP_CALL(hipMalloc(&P->d_sflags, sizeof(unsigned) * P->np_max * P->grid));
   int rate_khz = 0;
   if (hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && rate_khz > 0)
     P->clock_mhz = rate_khz / 1000.0;
@@ -678,7 +579,7 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, P->cap, P->d_queue);
   hipLaunchKernelGGL(k_batch, dim3(P->grid), dim3(64u * cfg.waves), P->lds, P->cap, P->d_probs,
                      P->d_order, n, P->d_queue, P->d_pool, P->d_s0, P->s0steps, cfg.max_sweeps,
-                     P->d_out, P->d_quads, P->d_scr, P->d_sflags, P->np_max);
+                     P->d_out);
   HIP_CALL(hipStreamEndCapture(P->cap, &graph));
   HIP_CALL(hipGraphInstantiate(&P->gexec, graph, nullptr, nullptr, 0));
   HIP_CALL(hipGraphDestroy(graph));
@@ -729,8 +630,7 @@ extern "C" void hj_batch_free(void *plan)
   if (P->gexec) HIP_CALL(hipGraphExecDestroy(P->gexec));
   if (P->cap) HIP_CALL(hipStreamDestroy(P->cap));
   for (void *p : {(void *)P->d_probs, (void *)P->d_order, (void *)P->d_queue, (void *)P->d_pool,
-                  (void *)P->d_s0, (void *)P->d_out, (void *)P->d_quads, (void *)P->d_scr,
-                  (void *)P->d_sflags})
+                  (void *)P->d_s0, (void *)P->d_out})
     if (p) HIP_CALL(hipFree(p));
   delete P;
 }

@@ -512,27 +512,27 @@ __device__ __forceinline__ unsigned wave_sum_u(unsigned v)
 // Level-0 sweeps of one block pair by one wave (the inner Jacobi of
 // share/device_code_nosort.hpp:4-222 for SORT false,
 // share/device_code_cdsort_KISS.hpp:4-260 and share/device_code_cdsort.hpp:25-167
-// for SORT true).  R: the Cholesky factor, W: the identity on entry, both in
-// the L0A layout.  Slot y = l/4 takes pivot pair y of a step, lane r = l%4 of
+// for SORT true).  R: the Cholesky factor, W: the identity on entry, column
+// c at c LD (LD = 36: of the 16 slots' columns, four rows each, those of
+// neighbouring pairs fall into different LDS banks; 33 made fourfold
+// conflicts).  Slot y = l/4 takes pivot pair y of a step, lane r = l%4 of
 // the slot holds rows r + 4k of the two columns; the pivot pairs of a step
 // touch disjoint columns, so one wave-level LDS sync per step suffices.
 // Returns the rotation counts of all its sweeps (the reference's counting:
 // a sweep without a rotation ends the loop and adds nothing) in every lane,
-// whether a pivot pair was swapped by the sort rule (W is the identity
-// exactly when nothing was rotated or swapped), and with COS the largest
-// |A_pq| / sqrt(A_pp A_qq) over the pivots of the first sweep.
-template <bool SORT, bool COS>
+// and whether a pivot pair was swapped by the sort rule (W is the identity
+// exactly when nothing was rotated or swapped).
+template <bool SORT, unsigned LD>
 __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_t *S0,
                                             unsigned s0steps, unsigned nswp, int def, bool hyp,
                                             unsigned npos, unsigned l, unsigned &out_s,
-                                            unsigned &out_b, bool &out_swap, double &out_cos)
+                                            unsigned &out_b, bool &out_swap)
 {
   lds_f64 *const R = (lds_f64 *)R_;
   lds_f64 *const W = (lds_f64 *)W_;
   const unsigned y = l >> 2, r = l & 3u;
   unsigned blk_s = 0u, blk_b = 0u;
   bool swapped = false;
-  double my_cos = 0.0;
   for (unsigned swp = 0u; swp < nswp; ++swp) {
     unsigned my_s = 0u, my_b = 0u;
     for (unsigned step = 0u; step < s0steps; ++step) {
@@ -540,8 +540,8 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
       double Gp[8], Gq[8];
 #pragma unroll
       for (unsigned k = 0u; k < 8u; ++k) {
-        Gp[k] = L0A(R, r + 4u * k, p);
-        Gq[k] = L0A(R, r + 4u * k, q);
+        Gp[k] = R[p * LD + r + 4u * k];
+        Gq[k] = R[q * LD + r + 4u * k];
       }
       double Dp, Dq, Apq;
       dots3<4u>(Gp, Gq, Dp, Dq, Apq);
@@ -559,18 +559,15 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
       const bool rot_b = rot_quad<true>(trig, Apq, Dp, Dq, l, c, t, Dpq_);
       const double Apq_ = fabs(Apq);
       const int transf_s = !(Apq_ < (Dpq_ * MYTOL));
-      if (COS && swp == 0u)
-        my_cos = fmax(my_cos, (Dpq_ > 0.0) ? (Apq_ / Dpq_) : 0.0);
       int transf_b = 0;
-      // W's columns p, q (the same lane reads and writes the same entries
-      // within a step, so they may be read this late)
-      double Vp[8], Vq[8];
-#pragma unroll
-      for (unsigned k = 0u; k < 8u; ++k) {
-        Vp[k] = L0A(W, r + 4u * k, p);
-        Vq[k] = L0A(W, r + 4u * k, q);
-      }
       if (transf_s) {
+        // (W's columns: the same lane reads and writes the same entries)
+        double Vp[8], Vq[8];
+#pragma unroll
+        for (unsigned k = 0u; k < 8u; ++k) {
+          Vp[k] = W[p * LD + r + 4u * k];
+          Vq[k] = W[q * LD + r + 4u * k];
+        }
         transf_b = rot_b ? 1 : 0;
         const double t_ = trig ? -t : t;
         if (SORT && trig) {
@@ -587,19 +584,25 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
           // c * x is x
           const double rp = __fma_rn(t_, Gq[k], Gp[k]), rq = __fma_rn(t, Gp[k], Gq[k]);
           const double wp = __fma_rn(t_, Vq[k], Vp[k]), wq = __fma_rn(t, Vp[k], Vq[k]);
-          L0A(R, r + 4u * k, PP) = c * rp;
-          L0A(R, r + 4u * k, QQ) = c * rq;
-          L0A(W, r + 4u * k, PP) = c * wp;
-          L0A(W, r + 4u * k, QQ) = c * wq;
+          R[PP * LD + r + 4u * k] = c * rp;
+          R[QQ * LD + r + 4u * k] = c * rq;
+          W[PP * LD + r + 4u * k] = c * wp;
+          W[QQ * LD + r + 4u * k] = c * wq;
         }
       }
       else if (SORT && (((pdef > 0) && (Dp < Dq)) || ((pdef < 0) && (Dq < Dp)))) {
+        double Vp[8], Vq[8];
 #pragma unroll
         for (unsigned k = 0u; k < 8u; ++k) {
-          L0A(R, r + 4u * k, p) = Gq[k];
-          L0A(R, r + 4u * k, q) = Gp[k];
-          L0A(W, r + 4u * k, p) = Vq[k];
-          L0A(W, r + 4u * k, q) = Vp[k];
+          Vp[k] = W[p * LD + r + 4u * k];
+          Vq[k] = W[q * LD + r + 4u * k];
+        }
+#pragma unroll
+        for (unsigned k = 0u; k < 8u; ++k) {
+          R[p * LD + r + 4u * k] = Gq[k];
+          R[q * LD + r + 4u * k] = Gp[k];
+          W[p * LD + r + 4u * k] = Vq[k];
+          W[q * LD + r + 4u * k] = Vp[k];
         }
         swapped = true;
       }
@@ -619,12 +622,6 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
   out_s = blk_s;
   out_b = blk_b;
   out_swap = __ballot(swapped) != 0ull;
-  if (COS) {
-#pragma unroll
-    for (int o = 32; o >= 4; o >>= 1)
-      my_cos = fmax(my_cos, __shfl_xor(my_cos, o, 64));
-  }
-  out_cos = my_cos;
 }
 
 }  // namespace hj

@@ -207,7 +207,9 @@ typedef struct hj_batch_desc {
 #define HJ_BATCH_STRAT_BRENTL 1u
 #define HJ_BATCH_STRAT_MMSTEP 2u
 
-/* Launch shape and schedule (hj_batch_autotune picks them). */
+/* Launch shape and schedule (hj_batch_autotune picks them).  The default
+ * shape (4 waves, 2 workgroups per CU) leaves the arrangement of those eight
+ * waves a CU to the plan; the results do not depend on it. */
 typedef struct hj_batch_cfg {
   unsigned waves;          /* waves per workgroup, 1..8 (one block pair each) */
   unsigned wg_per_cu;      /* workgroups per CU in the persistent grid */
