@@ -191,6 +191,8 @@ static void launch_zero_words(hipStream_t s, void *p, size_t n)
   HIP_CALL(hipGetLastError());
 }
 
+constexpr size_t RING_BYTES = 2u * sizeof(unsigned long long);
+
 // Device workspace of one level-2 run.
 struct Work {
   unsigned np = 0u, steps = 0u, s0steps = 0u, nchunk = 0u, CH = 0u, chG = 0u, chV = 0u;
@@ -200,6 +202,7 @@ struct Work {
   double *d_part = nullptr, *d_W = nullptr;
   unsigned *d_flags = nullptr;
   RunCtl *d_ctl = nullptr, *h_ctl = nullptr;
+  unsigned long long *h_ring = nullptr;  // counters of the last two sweeps queued ahead (pinned, behind h_ctl)
   VisitRec *d_rec = nullptr;   // [steps][np] last executed visit of each pair
   uint8_t *d_skip = nullptr;   // [steps][np] skip mask of the running sweep
   uint16_t *d_model = nullptr; // bf16 MLP parameters
@@ -269,8 +272,9 @@ struct Work {
     launch_zero_words(s, d_slab + up_end, (o_flags - up_end) / sizeof(unsigned));
     // (the host copy of the tables is pageable and goes out of scope)
     HIP_CALL(hipStreamSynchronize(s));
-    HIP_CALL(hipHostMalloc(&h_ctl, sizeof(RunCtl), hipHostMallocDefault));
+    HIP_CALL(hipHostMalloc(&h_ctl, align256(sizeof(RunCtl)) + RING_BYTES, hipHostMallocDefault));
     memset(h_ctl, 0, sizeof(RunCtl));
+    h_ring = reinterpret_cast<unsigned long long *>(reinterpret_cast<uint8_t *>(h_ctl) + align256(sizeof(RunCtl)));
   }
 
   // A transition s -> s+1 is fused when every pair of step s, with the pair
@@ -733,10 +737,19 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   }
   const bool eager = g_profile || (g_step_limit > 0) || getenv("HJ_NOGRAPH");
   hipGraphExec_t gexec = nullptr;
+  // Sweeps queued one ahead, kernel by kernel: the host launches sweep k + 1
+  // before it waits for sweep k's counter, so the device does not idle for the
+  // host's round trip and the next graph's start (45 us a sweep; a 64 x 64
+  // sweep's steps take 95 us), and no graph is built.  The sweep queued after
+  // the last one finds done set and leaves everything as it is, at 1.5 us a
+  // launch: for sweeps of whole-step launches only (at most 15 a sweep where a
+  // pair has 512 rows of G and V).
+  const bool ahead = !eager && !staged && !planned && !qr && step_fits(nrow, V ? ncol : 0u) && !g_trace_buf;
   // graph path: events around each sweep's graph launch, and the launches
   // of the sweep's dominant kind it holds (staged launches; else the steps'
-  // update-class launches)
-  hipEvent_t gev[2] = {nullptr, nullptr};
+  // update-class launches); sweeps queued ahead: one after the start of each,
+  // which hands over the counter of the one before, four in turn
+  hipEvent_t gev[4] = {nullptr, nullptr, nullptr, nullptr};
   unsigned long long graph_launches = 0ull;
   std::vector<hipEvent_t> evs;
   if (g_profile) {
@@ -744,12 +757,14 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
     for (auto &e : evs) HIP_CALL(hipEventCreate(&e));
   }
   auto sweep_head = [&](hipStream_t st) {
-    launch_sweep_begin(st, w.d_ctl);
+    launch_sweep_begin(st, w.d_ctl, ahead ? w.h_ring : nullptr);
     if (planned)
       launch_plan(st, w.d_rec, (unsigned)w.keys(), w.d_s1, nplus, log2n1, max_rot, w.d_ctl, w.d_model,
                   learned, w.d_skip);
   };
-  if (!eager) {
+  if (!eager)
+    for (unsigned i = 0u; i < (ahead ? 4u : 2u); ++i) HIP_CALL(hipEventCreate(&gev[i]));
+  if (!eager && !ahead) {
     // one sweep as a graph: start-of-sweep kernel (counters, no memset
     // node), the predictor, all steps, the control block to pinned memory
     hipGraph_t graph;
@@ -765,9 +780,8 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
     HIP_CALL(hipStreamEndCapture(s, &graph));
     HIP_CALL(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
     HIP_CALL(hipGraphDestroy(graph));
-    HIP_CALL(hipEventCreate(&gev[0]));
-    HIP_CALL(hipEventCreate(&gev[1]));
   }
+  unsigned queued = 0u;  // sweeps queued ahead
 
   long long swp_tim = 0;
   stopwatch_reset(swp_tim);
@@ -797,15 +811,29 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
         stop = true;
       HIP_CALL(hipMemcpyAsync(w.h_ctl, w.d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));
     }
+    else if (ahead) {
+      for (; queued < blk_swp + 2u; ++queued) {
+        sweep_head(s);
+        HIP_CALL(hipEventRecord(gev[queued & 3u], s));
+        if (queued < g_max_sweeps)
+          graph_launches = issue_sweep(s, w, cdsort, nswp, definite, nplus, dG, lddG, nrow, V, lddV,
+                                       ncol, nullptr, nullptr, false, false, nullptr);
+      }
+    }
     else {
       HIP_CALL(hipEventRecord(gev[0], s));
       HIP_CALL(hipGraphLaunch(gexec, s));
       HIP_CALL(hipEventRecord(gev[1], s));
     }
-    HIP_CALL(hipStreamSynchronize(s));
+    if (ahead) {
+      HIP_CALL(hipEventSynchronize(gev[(blk_swp + 1u) & 3u]));
+      w.h_ctl->cvg = *static_cast<volatile unsigned long long *>(w.h_ring + (blk_swp & 1u));
+    }
+    else
+      HIP_CALL(hipStreamSynchronize(s));
     if (!eager) {
       float ms = 0.0f;
-      HIP_CALL(hipEventElapsedTime(&ms, gev[0], gev[1]));
+      HIP_CALL(hipEventElapsedTime(&ms, gev[ahead ? blk_swp & 3u : 0u], gev[ahead ? (blk_swp + 1u) & 3u : 1u]));
       g_stats.kms[5] += ms;
       g_stats.kcnt[5] += graph_launches;
     }
@@ -864,14 +892,14 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
     if (!cvg_b && !skipped && !nsplit)
       break;
   }
+  *glbSwp = blk_swp;
+  launch_initD(s, dG, dD, 0u, nrow, ncol, nplus, lddG);
+  HIP_CALL(hipStreamSynchronize(s));
+  // (a sweep queued ahead may have been on its way until here)
   if (gexec) HIP_CALL(hipGraphExecDestroy(gexec));
   for (hipEvent_t e : gev)
     if (e) HIP_CALL(hipEventDestroy(e));
   for (auto &e : evs) HIP_CALL(hipEventDestroy(e));
-
-  *glbSwp = blk_swp;
-  launch_initD(s, dG, dD, 0u, nrow, ncol, nplus, lddG);
-  HIP_CALL(hipStreamSynchronize(s));
   HIP_CALL(hipStreamDestroy(s));
   w.release();
 }

@@ -930,11 +930,23 @@ __global__ __launch_bounds__(256) void k_initV(double *__restrict__ V, unsigned 
 // no big rotation certifies (every visit, FP64); otherwise skipping is on
 // when the form is and the previous sweep's big-rotation fraction reached
 // min_frac, the split Gram when the form is.
-__global__ void k_sweep_begin(RunCtl *ctl)
+__global__ void k_sweep_begin(RunCtl *ctl, unsigned long long *ring)
 {
   if (threadIdx.x == 0u) {
     const unsigned prev_b = (unsigned)(ctl->cvg >> 32);
     const bool first = (ctl->sweep == 0u);
+    if (ring) {
+      if (ctl->done)
+        return;
+      if (!first) {
+        __hip_atomic_store(&ring[(ctl->sweep - 1u) & 1u], ctl->cvg, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+        if (!prev_b) {
+          ctl->done = 1u;
+          return;
+        }
+      }
+    }
     const bool certify = !first && !prev_b && (ctl->skipped || ctl->split);
     const float frac = (float)prev_b / ctl->max_rot;
     ctl->skip_on = (ctl->learned && !first && !certify && frac >= ctl->min_frac) ? 1u : 0u;
@@ -1047,9 +1059,9 @@ void launch_initV(hipStream_t s, double *V, unsigned ifc, unsigned nRank, unsign
   hipLaunchKernelGGL(k_initV, dim3((unsigned)blocks), dim3(256), 0, s, V, ifc, nRank, ldV);
 }
 
-void launch_sweep_begin(hipStream_t s, RunCtl *ctl)
+void launch_sweep_begin(hipStream_t s, RunCtl *ctl, unsigned long long *ring)
 {
-  hipLaunchKernelGGL(k_sweep_begin, dim3(1), dim3(64), 0, s, ctl);
+  hipLaunchKernelGGL(k_sweep_begin, dim3(1), dim3(64), 0, s, ctl, ring);
 }
 
 void launch_dbg_scalar(hipStream_t s, int kind, int n, const double *a, const double *b,

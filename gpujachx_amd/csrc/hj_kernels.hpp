@@ -58,6 +58,7 @@ struct RunCtl {
   float min_skip_frac;          // ... and only if the model proposes at least this fraction of skips
   float max_rot;                // most big rotations a sweep can have (visits x 496)
   unsigned proposed;            // skips the model proposed for the running sweep
+  unsigned done;                // sweeps queued ahead: the one before ended the run, nothing is left to do
 };
 
 // waves sharing one Gram chunk of CH rows: each takes CH/nw rows, a multiple
@@ -205,7 +206,10 @@ void launch_pair_w(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np,
 void launch_update_w(hipStream_t s, double *M, unsigned ldM, unsigned nrow,
                      const uint16_t *pairs, unsigned np, const double *W,
                      const unsigned *flags);
-void launch_sweep_begin(hipStream_t s, RunCtl *ctl);
+// ring: sweeps are queued before the host has seen the one before, whose
+// counter goes to ring[(its number - 1) % 2] (pinned); a sweep after the last
+// does nothing (whole-step launches only)
+void launch_sweep_begin(hipStream_t s, RunCtl *ctl, unsigned long long *ring = nullptr);
 void launch_dbg_scalar(hipStream_t s, int kind, int n, const double *a, const double *b,
                        const double *c, double *oc, double *ot, int *ob);
 

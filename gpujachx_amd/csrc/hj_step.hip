@@ -139,6 +139,8 @@ __global__ __launch_bounds__(STEP_NT) void k_step(StepArgs A)
   const unsigned tid = threadIdx.x, pi = blockIdx.x, l = tid & 63u, w = tid >> 6;
   const unsigned iBlk = A.pairs[2u * pi], jBlk = A.pairs[2u * pi + 1u];
   const unsigned ld = A.nrow + 2u;
+  // (a sweep queued after the run's last one; a vector load)
+  const unsigned done = __hip_atomic_load(&A.ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // the pair's columns, four a wave, all loads in flight together (rows are a
   // multiple of 64)
   {
@@ -175,6 +177,8 @@ __global__ __launch_bounds__(STEP_NT) void k_step(StepArgs A)
       }
     }
   }
+  if (done)
+    return;
   __syncthreads();
   step_gram(L, ld, A.nsub, A.SUB, tid);
   visit_init<STEP_NT>(tid, L.pair, A.strat0);

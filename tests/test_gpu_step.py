@@ -64,3 +64,26 @@ def test_gram_tiles(m, n, limit):
                                            (640, 480, "BrentL", 31)])
 def test_v_rides_with_the_next_visits(m, n, fam, limit):
     both(11, m, n, n // 2, fam, limit)
+
+
+# sweeps queued one ahead (whole-step runs): ended by the cap or by convergence,
+# at every parity, twice in a row; the per-sweep counters are those of the oracle
+@pytest.mark.parametrize("cap", [1, 2, 3, 4, 30])
+@pytest.mark.parametrize("alg,m,n", [(11, 64, 32), (9, 128, 64), (2, 256, 96)])
+def test_sweeps_queued_ahead(cap, alg, m, n):
+    rng = np.random.default_rng(cap)
+    G = rng.standard_normal((m, n))
+    g.init_strats_builtin("cycwor", 32, "mmstep", n // 16)
+    s0, s1 = g.current_strats()
+    g.set_max_sweeps(cap)
+    o.set_max_sweeps(cap)
+    try:
+        ro = o.hypJacL2(alg, G, n, s0, s1)
+        for _ in range(2):
+            rg = g.hypJacL2(alg, G, n)
+            assert (rg.sweeps, rg.rot_s, rg.rot_b) == (ro["sweeps"], ro["rot_s"], ro["rot_b"])
+            np.testing.assert_array_equal(rg.D, ro["D"])
+            np.testing.assert_array_equal(rg.G, ro["G"])
+    finally:
+        g.set_max_sweeps(30)
+        o.set_max_sweeps(30)
