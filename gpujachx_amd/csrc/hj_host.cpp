@@ -214,6 +214,7 @@ struct Work {
   // the rest; transitions whose first-half quads need a pair of the previous
   // transition's second half
   bool stage_ok = false;
+  bool ahead = false;  // sweeps are queued one ahead (see level2_core)
   uint16_t *d_plist = nullptr;
   uint16_t *d_plist_run = nullptr;  // d_plist reordered per sweep (learned skip)
   uint16_t *d_qord = nullptr;       // per transition, the quads in item order (learned skip)
@@ -402,11 +403,23 @@ static VItems v_items(const Work &w, unsigned st, double *dV, unsigned lddV, uns
   return v;
 }
 
-// One level-1 step: Gram partials, pair kernels, block update.
+__global__ void k_thin_accum(RunCtl *ctl, unsigned long long *cvg)
+{
+  if (threadIdx.x == 0u) {
+    *cvg += ctl->cvg;
+    ctl->cvg = 0ull;
+  }
+}
+
+// One level-1 step: Gram partials, pair kernels, block update.  cvg (thin
+// layer): the caller's 8-byte device word, to which the step's rotation count
+// (added by the pair kernels to the workspace's control block) is added after
+// the step, by the update's launch where there is one (2048 x 1024: a step 60
+// us with a launch for it, 58 without).
 static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, unsigned nswp,
                        int definite, unsigned nplus, double *dG, unsigned lddG, unsigned nrow,
                        double *dV, unsigned lddV, unsigned ncol, hipEvent_t *ev, bool planned,
-                       bool split)
+                       bool split, unsigned long long *cvg = nullptr)
 {
   const size_t off = (size_t)step * w.np;
   const uint16_t *pairs = w.d_s1 + off * 2u;
@@ -418,12 +431,15 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
     launch_pair_qr(s, sort, g_fact == HJ_FACT_QR_DRMAC, dG, lddG, nrow, pairs, w.np, w.d_W,
                    w.d_flags, w.d_ctl, w.d_s0, w.s0steps, nswp, definite, nplus);
     if (ev) HIP_CALL(hipEventRecord(ev[2], s));
-    launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags);
+    launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags,
+                  w.d_ctl, cvg);
     if (ev) HIP_CALL(hipEventRecord(ev[3], s));
     return;
   }
   if (!ev && !skip && step_fits(nrow, dV ? ncol : 0u)) {
     issue_whole_step(s, w, step, sort, nswp, definite, nplus, dG, lddG, nrow, dV, lddV, ncol);
+    if (cvg)
+      hipLaunchKernelGGL(k_thin_accum, dim3(1), dim3(64), 0, s, w.d_ctl, cvg);
     return;
   }
   launch_gram(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, skip);
@@ -431,9 +447,10 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
     launch_gram_split(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, skip);
   if (ev) HIP_CALL(hipEventRecord(ev[1], s));
   launch_pair(s, sort, pairs, w.np, w.d_part, w.nchunk, w.d_W, w.d_flags, w.d_ctl, w.d_rec + off,
-              skip, split, w.d_s0, w.s0steps, nswp, definite, nplus);
+              skip, split, w.d_s0, w.s0steps, nswp, definite, nplus, VItems(), w.ahead);
   if (ev) HIP_CALL(hipEventRecord(ev[2], s));
-  launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags);
+  launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags,
+                w.d_ctl, cvg);
   if (ev) HIP_CALL(hipEventRecord(ev[3], s));
 }
 
@@ -743,7 +760,8 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   // sweep's steps take 95 us), and no graph is built.  The sweep queued after
   // the last one finds done set and leaves everything as it is, at 1.5 us a
   // launch: for sweeps of whole-step launches only (at most 15 a sweep where a
-  // pair has 512 rows of G and V).
+  // pair has 512 rows of G and V).  64 x 64 1.60 -> 1.40 ms, 256 x 256 9.04 -> 8.87;
+  // 512 x 256 with V, three launches a step, 3.30 -> 3.39.
   const bool ahead = !eager && !staged && !planned && !qr && step_fits(nrow, V ? ncol : 0u) && !g_trace_buf;
   // graph path: events around each sweep's graph launch, and the launches
   // of the sweep's dominant kind it holds (staged launches; else the steps'
@@ -1165,24 +1183,12 @@ struct Thin {
 };
 static Thin g_thin;
 
-// The rotation counter of the thin layer is the caller's 8-byte device
-// word: the step's count (added by the pair kernels to the workspace's
-// control block) is added to it after the step.
-__global__ void k_thin_accum(hj::RunCtl *ctl, unsigned long long *cvg)
-{
-  if (threadIdx.x == 0u) {
-    *cvg += ctl->cvg;
-    ctl->cvg = 0ull;
-  }
-}
-
 static void thin_step(unsigned step, bool sort, bool withV, int definite, unsigned nplus)
 {
   if (!g_thin.ready) HJ_DIE("initSymbols not called");
   if (step >= g_thin.w.steps) HJ_DIE("step out of range");
   issue_step(nullptr, g_thin.w, step, sort, g_thin.nSwp, definite, nplus, g_thin.G, g_thin.ldG,
-             g_thin.nRow, withV ? g_thin.V : nullptr, g_thin.ldV, g_thin.nCol, nullptr, false, false);
-  hipLaunchKernelGGL(k_thin_accum, dim3(1), dim3(64), 0, nullptr, g_thin.w.d_ctl, g_thin.cvg);
+             g_thin.nRow, withV ? g_thin.V : nullptr, g_thin.ldV, g_thin.nCol, nullptr, false, false, g_thin.cvg);
   HIP_CALL(hipGetLastError());
 }
 
@@ -1299,11 +1305,12 @@ constexpr size_t NOALLOC_BYTES = (size_t)8u << 20;
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 static void *g_scratch_ptr[NOALLOC_MAX_DEVICES];
+static unsigned long long *g_scratch_ring[NOALLOC_MAX_DEVICES];  // pinned (see level2_core)
 
 namespace {
 
-// the scratch array's device address on the current device
-unsigned char *scratch_here()
+// the scratch array's device address and the ring on the current device
+unsigned char *scratch_here(unsigned long long *&ring)
 {
   int dev = 0;
   HIP_CALL(hipGetDevice(&dev));
@@ -1314,6 +1321,9 @@ unsigned char *scratch_here()
     HIP_CALL(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     g_scratch_ptr[dev] = p;
   }
+  if (!g_scratch_ring[dev])
+    HIP_CALL(hipHostMalloc(&g_scratch_ring[dev], RING_BYTES, hipHostMallocDefault));
+  ring = g_scratch_ring[dev];
   return static_cast<unsigned char *>(g_scratch_ptr[dev]);
 }
 
@@ -1338,12 +1348,13 @@ struct ScratchPlan {
 
 // The sweeps of level2_core in the plain FP64 form, each level-1 step
 // launched as Gram, pair visits and block update on the caller's stream,
-// with the control block read back after every sweep.
+// with the control block read back after every sweep (or its counter through
+// the ring, the next sweep queued).
 static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsigned nplus,
                            double *dG, unsigned lddG, double *dV, unsigned lddV, double *dD,
                            unsigned *glbSwp, unsigned long long *glb_s,
                            unsigned long long *glb_b, hipStream_t s, unsigned char *base,
-                           const ScratchPlan &sp)
+                           const ScratchPlan &sp, unsigned long long *ring)
 {
   const bool cdsort = (routine & HYPJAC_CDSORT_1) != 0u;
   const bool full_svd = (routine & HYPJAC_FULL_SVD) != 0u;
@@ -1384,14 +1395,38 @@ static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsig
   long long swp_tim = 0;
   stopwatch_reset(swp_tim);
   unsigned blk_swp = 0u;
-  RunCtl h;
-  while (blk_swp < g_max_sweeps) {
-    launch_sweep_begin(s, w.d_ctl);
+  // Sweeps queued one ahead, as in level2_core; without a graph to lose also for
+  // short sweeps of three launches, whose last, empty one costs 6 to 10 us a
+  // step (512 x 128 with V 1.61 -> 1.53 ms).
+  const bool ahead = g_fact == HJ_FACT_CHOLESKY &&
+                     (step_fits(nrow, V ? ncol : 0u) || (w.steps <= 16u && nrow <= 2048u));
+  w.ahead = ahead;
+  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  if (ahead)
+    for (hipEvent_t &e : ev) HIP_CALL(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  unsigned queued = 0u;
+  auto steps = [&]() {
     for (unsigned st = 0u; st < w.steps; ++st)
       issue_step(s, w, st, cdsort, nswp, definite, nplus, dG, lddG, nrow, V, lddV, ncol, nullptr,
                  false, false);
-    HIP_CALL(hipMemcpyAsync(&h, w.d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));
-    HIP_CALL(hipStreamSynchronize(s));
+  };
+  RunCtl h;
+  while (blk_swp < g_max_sweeps) {
+    if (ahead) {
+      for (; queued < blk_swp + 2u; ++queued) {
+        launch_sweep_begin(s, w.d_ctl, ring);
+        HIP_CALL(hipEventRecord(ev[queued & 3u], s));
+        if (queued < g_max_sweeps) steps();
+      }
+      HIP_CALL(hipEventSynchronize(ev[(blk_swp + 1u) & 3u]));
+      h.cvg = *static_cast<volatile unsigned long long *>(ring + (blk_swp & 1u));
+    }
+    else {
+      launch_sweep_begin(s, w.d_ctl);
+      steps();
+      HIP_CALL(hipMemcpyAsync(&h, w.d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));
+      HIP_CALL(hipStreamSynchronize(s));
+    }
     ++blk_swp;
     const unsigned cvg_s = static_cast<unsigned>(h.cvg);
     const unsigned cvg_b = static_cast<unsigned>(h.cvg >> 32u);
@@ -1416,6 +1451,8 @@ static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsig
   *glbSwp = blk_swp;
   launch_initD(s, dG, dD, 0u, nrow, ncol, nplus, lddG);
   HIP_CALL(hipStreamSynchronize(s));
+  for (hipEvent_t e : ev)
+    if (e) HIP_CALL(hipEventDestroy(e));
   g_last_stage = 0;
 }
 
@@ -1441,10 +1478,11 @@ extern "C" int hypJacL2_dev_noalloc(unsigned routine, unsigned nrow, unsigned nc
                             "more than the %zu of the scratch array\n", ncol, sp.end, NOALLOC_BYTES);
     return HJ_ERR_SCRATCH;
   }
-  unsigned char *const base = scratch_here();
+  unsigned long long *ring = nullptr;
+  unsigned char *const base = scratch_here(ring);
   stopwatch_reset(t1);
   level2_noalloc(routine, nrow, ncol, nplus, dG, lddG, full_svd ? dV : nullptr, lddV, dD, glbSwp,
-                 glb_s, glb_b, static_cast<hipStream_t>(stream), base, sp);
+                 glb_s, glb_b, static_cast<hipStream_t>(stream), base, sp, ring);
   const long long tc = stopwatch_lap(t1);
   const long long tw = stopwatch_lap(t0);
   if (timing) {
@@ -1670,7 +1708,8 @@ extern "C" int configureGPUex(const int dev, const unsigned maxShMemB)
     (void)snprintf(msg, sizeof(msg), "HIP device %d is %s, not a gfx9 (CDNA) part", dev, p.gcnArchName);
     HJ_DIE(msg);
   }
-  (void)scratch_here();  // the allocation-free entry's array on this device
+  unsigned long long *ring = nullptr;
+  (void)scratch_here(ring);  // the allocation-free entry's array on this device
   return p.major * 10 + p.minor;
 }
 

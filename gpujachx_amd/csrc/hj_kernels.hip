@@ -471,9 +471,16 @@ __global__ __launch_bounds__(64) void k_update(double *__restrict__ G, unsigned 
                                                unsigned chV, unsigned nchV,
                                                const uint16_t *__restrict__ pairs,
                                                const double *__restrict__ Wbuf,
-                                               const unsigned *__restrict__ flags)
+                                               const unsigned *__restrict__ flags, RunCtl *ctl,
+                                               unsigned long long *cvg)
 {
   const unsigned l = threadIdx.x;
+  if (cvg && blockIdx.x == 0u && l == 0u) {
+    // a step of the thin layer: its rotations (the visits are complete) to the
+    // caller's counter
+    *cvg += ctl->cvg;
+    ctl->cvg = 0ull;
+  }
   const unsigned per = nchG + nchV;
   const unsigned pi = blockIdx.x / per, c = blockIdx.x - pi * per;
   if (!flags[pi])
@@ -507,12 +514,18 @@ __device__ __forceinline__ void v_item(const VItems &V, unsigned b, unsigned tid
               V.W + (size_t)pi * 1024u, tid & 63u);
 }
 
+// relaxed device-scope load (a vector load, coherent across the XCDs)
+__device__ __forceinline__ unsigned ld_relaxed(const unsigned *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Workgroups [0, np): the visits; then V's items of the step before (V.n of
 // them, none without V).
 // split_src: the partials of this launch's pairs came from k_gram followed by
 // k_gram_split (a standalone Gram launch), so split-planned pairs hold split
 // Grams
-template <bool SORT>
+template <bool SORT, bool AHEAD>
 __global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
     const uint16_t *__restrict__ pairs, const double *__restrict__ part, unsigned nchunk,
     double *__restrict__ Wout, unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
@@ -526,12 +539,14 @@ __global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
     v_item<PAIR_LANES / 2u>(V, pi - np, tid);
     return;
   }
+  // (sweeps queued ahead are kernels of their own: the load costs 1%)
+  const unsigned done = AHEAD ? ld_relaxed(&ctl->done) : 0u;
   const uint8_t plan = visit_plan(skip ? skip[pi] : PLAN_FP64, split_src != 0);
   if (plan == PLAN_SKIP)
     skip_visit(tid, pi, flags, ctl, rec);
   else
     pair_visit<SORT, PAIR_LANES>(tid, pi, L, pairs, part, nchunk, Wout, flags, ctl, rec, plan,
-                                 strat0, s0steps, nswp, definite, nplus);
+                                 strat0, s0steps, nswp, definite, nplus, done);
 }
 
 // ---------------------------------------------------------------------------
@@ -568,12 +583,6 @@ __device__ __forceinline__ void store_partial(double *o, unsigned l, bool split,
     o[256u + idx] = a10[r];
     o[512u + idx] = a11[r];
   }
-}
-
-// relaxed device-scope load (a vector load, coherent across the XCDs)
-__device__ __forceinline__ unsigned ld_relaxed(const unsigned *p)
-{
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // LDS of one fused workgroup: wave partials, W of both pairs, the waves'
@@ -1025,9 +1034,10 @@ void launch_gram_split(hipStream_t s, const double *G, unsigned ldG, const uint1
 void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, const double *part,
                  unsigned nchunk, double *W, unsigned *flags, RunCtl *ctl, VisitRec *rec,
                  const uint8_t *skip, bool split_src, const uint8_t *strat0, unsigned s0steps,
-                 unsigned nswp, int definite, unsigned nplus, const VItems &v)
+                 unsigned nswp, int definite, unsigned nplus, const VItems &v, bool ahead)
 {
-  const auto k = sort ? k_pair<true> : k_pair<false>;
+  const auto k = ahead ? (sort ? k_pair<true, true> : k_pair<false, true>)
+                       : (sort ? k_pair<true, false> : k_pair<false, false>);
   hipLaunchKernelGGL(k, dim3(np + (v.n + PAIR_LANES / 2u - 1u) / (PAIR_LANES / 2u)),
                      dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl, rec, skip,
                      split_src ? 1 : 0, strat0, s0steps, nswp, definite, nplus, np, v);
@@ -1035,12 +1045,13 @@ void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, c
 
 void launch_update(hipStream_t s, double *G, unsigned ldG, unsigned nrowG, unsigned chG,
                    double *V, unsigned ldV, unsigned nrowV, unsigned chV, const uint16_t *pairs,
-                   unsigned np, const double *W, const unsigned *flags)
+                   unsigned np, const double *W, const unsigned *flags,
+                   RunCtl *ctl, unsigned long long *cvg)
 {
   const unsigned nchG = (nrowG + chG - 1u) / chG;
   const unsigned nchV = V ? (nrowV + chV - 1u) / chV : 0u;
   hipLaunchKernelGGL(k_update, dim3(np * (nchG + nchV)), dim3(64), 0, s, G, ldG, nrowG, chG, nchG,
-                     V, ldV, nrowV, chV, nchV, pairs, W, flags);
+                     V, ldV, nrowV, chV, nchV, pairs, W, flags, ctl, cvg);
 }
 
 void launch_initD(hipStream_t s, double *G, double *D, unsigned ifc, unsigned nRow, unsigned nRank,

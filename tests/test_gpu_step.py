@@ -66,10 +66,10 @@ def test_v_rides_with_the_next_visits(m, n, fam, limit):
     both(11, m, n, n // 2, fam, limit)
 
 
-# sweeps queued one ahead (whole-step runs): ended by the cap or by convergence,
-# at every parity, twice in a row; the per-sweep counters are those of the oracle
+# sweeps queued one ahead (one launch a step, or three with and without V):
+# ended by the cap or by convergence, at every parity, twice in a row
 @pytest.mark.parametrize("cap", [1, 2, 3, 4, 30])
-@pytest.mark.parametrize("alg,m,n", [(11, 64, 32), (9, 128, 64), (2, 256, 96)])
+@pytest.mark.parametrize("alg,m,n", [(11, 64, 32), (9, 128, 64), (2, 256, 96), (11, 1024, 96), (9, 2048, 224)])
 def test_sweeps_queued_ahead(cap, alg, m, n):
     rng = np.random.default_rng(cap)
     G = rng.standard_normal((m, n))
@@ -84,6 +84,36 @@ def test_sweeps_queued_ahead(cap, alg, m, n):
             assert (rg.sweeps, rg.rot_s, rg.rot_b) == (ro["sweeps"], ro["rot_s"], ro["rot_b"])
             np.testing.assert_array_equal(rg.D, ro["D"])
             np.testing.assert_array_equal(rg.G, ro["G"])
+    finally:
+        g.set_max_sweeps(30)
+        o.set_max_sweeps(30)
+
+
+# the same without allocation (the ring of the scratch array is used again)
+@pytest.mark.parametrize("cap", [1, 2, 3, 30])
+@pytest.mark.parametrize("m,n", [(64, 32), (576, 64), (2048, 128)])
+def test_noalloc_sweeps_queued_ahead(cap, m, n):
+    import ctypes
+    import torch
+    rng = np.random.default_rng(cap)
+    G = np.asfortranarray(rng.standard_normal((m, n)))
+    g.init_strats_builtin("cycwor", 32, "mmstep", n // 16)
+    s0, s1 = g.current_strats()
+    g.set_max_sweeps(cap)
+    o.set_max_sweeps(cap)
+    try:
+        ro = o.hypJacL2(11, G, n, s0, s1)
+        for _ in range(2):
+            dG = torch.from_numpy(G.T.copy()).cuda()
+            dV, dD = torch.zeros(n, n, dtype=torch.float64, device="cuda"), torch.zeros(n, dtype=torch.float64, device="cuda")
+            sw, gs, gb = ctypes.c_uint(0), ctypes.c_ulonglong(0), ctypes.c_ulonglong(0)
+            rc = g.lib().hypJacL2_dev_noalloc(11, m, n, n, dG.data_ptr(), m, dV.data_ptr(), n, dD.data_ptr(),
+                                              ctypes.byref(sw), ctypes.byref(gs), ctypes.byref(gb), None,
+                                              torch.cuda.current_stream().cuda_stream)
+            assert rc == 0 and (sw.value, gs.value, gb.value) == (ro["sweeps"], ro["rot_s"], ro["rot_b"])
+            np.testing.assert_array_equal(dD.cpu().numpy(), ro["D"])
+            np.testing.assert_array_equal(dG.cpu().numpy().T, ro["G"])
+            np.testing.assert_array_equal(dV.cpu().numpy().T, ro["V"])
     finally:
         g.set_max_sweeps(30)
         o.set_max_sweeps(30)
