@@ -214,7 +214,6 @@ struct Work {
   // the rest; transitions whose first-half quads need a pair of the previous
   // transition's second half
   bool stage_ok = false;
-  bool ahead = false;  // sweeps are queued one ahead (see level2_core)
   uint16_t *d_plist = nullptr;
   uint16_t *d_plist_run = nullptr;  // d_plist reordered per sweep (learned skip)
   uint16_t *d_qord = nullptr;       // per transition, the quads in item order (learned skip)
@@ -447,7 +446,7 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
     launch_gram_split(s, dG, lddG, pairs, w.np, w.nchunk, w.CH, w.d_part, skip);
   if (ev) HIP_CALL(hipEventRecord(ev[1], s));
   launch_pair(s, sort, pairs, w.np, w.d_part, w.nchunk, w.d_W, w.d_flags, w.d_ctl, w.d_rec + off,
-              skip, split, w.d_s0, w.s0steps, nswp, definite, nplus, VItems(), w.ahead);
+              skip, split, w.d_s0, w.s0steps, nswp, definite, nplus);
   if (ev) HIP_CALL(hipEventRecord(ev[2], s));
   launch_update(s, dG, lddG, nrow, w.chG, dV, lddV, ncol, w.chV, pairs, w.np, w.d_W, w.d_flags,
                 w.d_ctl, cvg);
@@ -1305,12 +1304,11 @@ constexpr size_t NOALLOC_BYTES = (size_t)8u << 20;
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 static void *g_scratch_ptr[NOALLOC_MAX_DEVICES];
-static unsigned long long *g_scratch_ring[NOALLOC_MAX_DEVICES];  // pinned (see level2_core)
 
 namespace {
 
-// the scratch array's device address and the ring on the current device
-unsigned char *scratch_here(unsigned long long *&ring)
+// the scratch array's device address on the current device
+unsigned char *scratch_here()
 {
   int dev = 0;
   HIP_CALL(hipGetDevice(&dev));
@@ -1321,9 +1319,6 @@ unsigned char *scratch_here(unsigned long long *&ring)
     HIP_CALL(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     g_scratch_ptr[dev] = p;
   }
-  if (!g_scratch_ring[dev])
-    HIP_CALL(hipHostMalloc(&g_scratch_ring[dev], RING_BYTES, hipHostMallocDefault));
-  ring = g_scratch_ring[dev];
   return static_cast<unsigned char *>(g_scratch_ptr[dev]);
 }
 
@@ -1348,13 +1343,12 @@ struct ScratchPlan {
 
 // The sweeps of level2_core in the plain FP64 form, each level-1 step
 // launched as Gram, pair visits and block update on the caller's stream,
-// with the control block read back after every sweep (or its counter through
-// the ring, the next sweep queued).
+// with the control block read back after every sweep.
 static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsigned nplus,
                            double *dG, unsigned lddG, double *dV, unsigned lddV, double *dD,
                            unsigned *glbSwp, unsigned long long *glb_s,
                            unsigned long long *glb_b, hipStream_t s, unsigned char *base,
-                           const ScratchPlan &sp, unsigned long long *ring)
+                           const ScratchPlan &sp)
 {
   const bool cdsort = (routine & HYPJAC_CDSORT_1) != 0u;
   const bool full_svd = (routine & HYPJAC_FULL_SVD) != 0u;
@@ -1395,38 +1389,14 @@ static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsig
   long long swp_tim = 0;
   stopwatch_reset(swp_tim);
   unsigned blk_swp = 0u;
-  // Sweeps queued one ahead, as in level2_core; without a graph to lose also for
-  // short sweeps of three launches, whose last, empty one costs 6 to 10 us a
-  // step (512 x 128 with V 1.61 -> 1.53 ms).
-  const bool ahead = g_fact == HJ_FACT_CHOLESKY &&
-                     (step_fits(nrow, V ? ncol : 0u) || (w.steps <= 16u && nrow <= 2048u));
-  w.ahead = ahead;
-  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-  if (ahead)
-    for (hipEvent_t &e : ev) HIP_CALL(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  unsigned queued = 0u;
-  auto steps = [&]() {
+  RunCtl h;
+  while (blk_swp < g_max_sweeps) {
+    launch_sweep_begin(s, w.d_ctl);
     for (unsigned st = 0u; st < w.steps; ++st)
       issue_step(s, w, st, cdsort, nswp, definite, nplus, dG, lddG, nrow, V, lddV, ncol, nullptr,
                  false, false);
-  };
-  RunCtl h;
-  while (blk_swp < g_max_sweeps) {
-    if (ahead) {
-      for (; queued < blk_swp + 2u; ++queued) {
-        launch_sweep_begin(s, w.d_ctl, ring);
-        HIP_CALL(hipEventRecord(ev[queued & 3u], s));
-        if (queued < g_max_sweeps) steps();
-      }
-      HIP_CALL(hipEventSynchronize(ev[(blk_swp + 1u) & 3u]));
-      h.cvg = *static_cast<volatile unsigned long long *>(ring + (blk_swp & 1u));
-    }
-    else {
-      launch_sweep_begin(s, w.d_ctl);
-      steps();
-      HIP_CALL(hipMemcpyAsync(&h, w.d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));
-      HIP_CALL(hipStreamSynchronize(s));
-    }
+    HIP_CALL(hipMemcpyAsync(&h, w.d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, s));
+    HIP_CALL(hipStreamSynchronize(s));
     ++blk_swp;
     const unsigned cvg_s = static_cast<unsigned>(h.cvg);
     const unsigned cvg_b = static_cast<unsigned>(h.cvg >> 32u);
@@ -1451,8 +1421,6 @@ static void level2_noalloc(unsigned routine, unsigned nrow, unsigned ncol, unsig
   *glbSwp = blk_swp;
   launch_initD(s, dG, dD, 0u, nrow, ncol, nplus, lddG);
   HIP_CALL(hipStreamSynchronize(s));
-  for (hipEvent_t e : ev)
-    if (e) HIP_CALL(hipEventDestroy(e));
   g_last_stage = 0;
 }
 
@@ -1478,11 +1446,10 @@ extern "C" int hypJacL2_dev_noalloc(unsigned routine, unsigned nrow, unsigned nc
                             "more than the %zu of the scratch array\n", ncol, sp.end, NOALLOC_BYTES);
     return HJ_ERR_SCRATCH;
   }
-  unsigned long long *ring = nullptr;
-  unsigned char *const base = scratch_here(ring);
+  unsigned char *const base = scratch_here();
   stopwatch_reset(t1);
   level2_noalloc(routine, nrow, ncol, nplus, dG, lddG, full_svd ? dV : nullptr, lddV, dD, glbSwp,
-                 glb_s, glb_b, static_cast<hipStream_t>(stream), base, sp, ring);
+                 glb_s, glb_b, static_cast<hipStream_t>(stream), base, sp);
   const long long tc = stopwatch_lap(t1);
   const long long tw = stopwatch_lap(t0);
   if (timing) {
@@ -1708,8 +1675,7 @@ extern "C" int configureGPUex(const int dev, const unsigned maxShMemB)
     (void)snprintf(msg, sizeof(msg), "HIP device %d is %s, not a gfx9 (CDNA) part", dev, p.gcnArchName);
     HJ_DIE(msg);
   }
-  unsigned long long *ring = nullptr;
-  (void)scratch_here(ring);  // the allocation-free entry's array on this device
+  (void)scratch_here();  // the allocation-free entry's array on this device
   return p.major * 10 + p.minor;
 }
 

@@ -525,7 +525,7 @@ __device__ __forceinline__ unsigned ld_relaxed(const unsigned *p)
 // split_src: the partials of this launch's pairs came from k_gram followed by
 // k_gram_split (a standalone Gram launch), so split-planned pairs hold split
 // Grams
-template <bool SORT, bool AHEAD>
+template <bool SORT>
 __global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
     const uint16_t *__restrict__ pairs, const double *__restrict__ part, unsigned nchunk,
     double *__restrict__ Wout, unsigned *__restrict__ flags, RunCtl *__restrict__ ctl,
@@ -539,14 +539,12 @@ __global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
     v_item<PAIR_LANES / 2u>(V, pi - np, tid);
     return;
   }
-  // (sweeps queued ahead are kernels of their own: the load costs 1%)
-  const unsigned done = AHEAD ? ld_relaxed(&ctl->done) : 0u;
   const uint8_t plan = visit_plan(skip ? skip[pi] : PLAN_FP64, split_src != 0);
   if (plan == PLAN_SKIP)
     skip_visit(tid, pi, flags, ctl, rec);
   else
     pair_visit<SORT, PAIR_LANES>(tid, pi, L, pairs, part, nchunk, Wout, flags, ctl, rec, plan,
-                                 strat0, s0steps, nswp, definite, nplus, done);
+                                 strat0, s0steps, nswp, definite, nplus);
 }
 
 // ---------------------------------------------------------------------------
@@ -1034,10 +1032,9 @@ void launch_gram_split(hipStream_t s, const double *G, unsigned ldG, const uint1
 void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, const double *part,
                  unsigned nchunk, double *W, unsigned *flags, RunCtl *ctl, VisitRec *rec,
                  const uint8_t *skip, bool split_src, const uint8_t *strat0, unsigned s0steps,
-                 unsigned nswp, int definite, unsigned nplus, const VItems &v, bool ahead)
+                 unsigned nswp, int definite, unsigned nplus, const VItems &v)
 {
-  const auto k = ahead ? (sort ? k_pair<true, true> : k_pair<false, true>)
-                       : (sort ? k_pair<true, false> : k_pair<false, false>);
+  const auto k = sort ? k_pair<true> : k_pair<false>;
   hipLaunchKernelGGL(k, dim3(np + (v.n + PAIR_LANES / 2u - 1u) / (PAIR_LANES / 2u)),
                      dim3(32u * PAIR_LANES), 0, s, pairs, part, nchunk, W, flags, ctl, rec, skip,
                      split_src ? 1 : 0, strat0, s0steps, nswp, definite, nplus, np, v);

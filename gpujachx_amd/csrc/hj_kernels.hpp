@@ -177,13 +177,11 @@ void launch_gram_split(hipStream_t s, const double *G, unsigned ldG, const uint1
                        unsigned np, unsigned nchunk, unsigned CH, double *part, const uint8_t *plan);
 // split_src: the partials come from a standalone Gram launch, so pairs
 // planned split hold split Grams (else every pair is an FP64 visit); v: V's
-// items of an earlier step, in the same launch; ahead: sweeps are queued ahead,
-// no visit once RunCtl's done is set
+// items of an earlier step, in the same launch
 void launch_pair(hipStream_t s, bool sort, const uint16_t *pairs, unsigned np, const double *part,
                  unsigned nchunk, double *W, unsigned *flags, RunCtl *ctl, VisitRec *rec,
                  const uint8_t *skip, bool split_src, const uint8_t *strat0, unsigned s0steps,
-                 unsigned nswp, int definite, unsigned nplus, const VItems &v = VItems(),
-                 bool ahead = false);
+                 unsigned nswp, int definite, unsigned nplus, const VItems &v = VItems());
 // cvg: the caller's counter, to which ctl's goes (thin layer)
 void launch_update(hipStream_t s, double *G, unsigned ldG, unsigned nrowG, unsigned chG,
                    double *V, unsigned ldV, unsigned nrowV, unsigned chV, const uint16_t *pairs,
@@ -212,7 +210,7 @@ void launch_update_w(hipStream_t s, double *M, unsigned ldM, unsigned nrow,
                      const unsigned *flags);
 // ring: sweeps are queued before the host has seen the one before, whose
 // counter goes to ring[(its number - 1) % 2] (pinned); a sweep after the last
-// does nothing (k_step, or k_pair, whose update then finds every flag zero)
+// does nothing (k_step only)
 void launch_sweep_begin(hipStream_t s, RunCtl *ctl, unsigned long long *ring = nullptr);
 void launch_dbg_scalar(hipStream_t s, int kind, int n, const double *a, const double *b,
                        const double *c, double *oc, double *ot, int *ob);

@@ -465,15 +465,10 @@ __device__ __forceinline__ void pair_visit(unsigned tid, unsigned pi, PairLds &L
                                            RunCtl *__restrict__ ctl, VisitRec *__restrict__ rec,
                                            uint8_t plan, const uint8_t *__restrict__ strat0,
                                            unsigned s0steps, unsigned nswp, int definite,
-                                           unsigned nplus, unsigned done = 0u)
+                                           unsigned nplus)
 {
   constexpr unsigned NT = 32u * LANES;
   visit_load<NT>(tid, pi, L, part, nchunk, strat0);
-  if (done) {
-    // a sweep queued after the run's last one: no visit, no update
-    if (tid == 0u) flags[pi] = 0u;
-    return;
-  }
   const PairSigns sg = pair_signs16(definite, nplus, pairs[2u * pi], pairs[2u * pi + 1u]);
   // (W of a pair left alone is read by nothing)
   if (!visit_core<SORT, LANES>(tid, pi, L, sg, flags, ctl, rec, plan, s0steps, nswp))

@@ -66,8 +66,8 @@ def test_v_rides_with_the_next_visits(m, n, fam, limit):
     both(11, m, n, n // 2, fam, limit)
 
 
-# sweeps queued one ahead (one launch a step, or three with and without V):
-# ended by the cap or by convergence, at every parity, twice in a row
+# sweeps queued one ahead (one launch a step), or not (three): ended by the cap
+# or by convergence, at every parity, twice in a row
 @pytest.mark.parametrize("cap", [1, 2, 3, 4, 30])
 @pytest.mark.parametrize("alg,m,n", [(11, 64, 32), (9, 128, 64), (2, 256, 96), (11, 1024, 96), (9, 2048, 224)])
 def test_sweeps_queued_ahead(cap, alg, m, n):
@@ -89,10 +89,10 @@ def test_sweeps_queued_ahead(cap, alg, m, n):
         o.set_max_sweeps(30)
 
 
-# the same without allocation (the ring of the scratch array is used again)
+# the same without allocation (the scratch array is used again)
 @pytest.mark.parametrize("cap", [1, 2, 3, 30])
 @pytest.mark.parametrize("m,n", [(64, 32), (576, 64), (2048, 128)])
-def test_noalloc_sweeps_queued_ahead(cap, m, n):
+def test_noalloc_sweep_caps(cap, m, n):
     import ctypes
     import torch
     rng = np.random.default_rng(cap)
