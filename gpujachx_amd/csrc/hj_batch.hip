@@ -26,7 +26,6 @@
 
 #include "../../include/hypjac.h"
 #include "hj_device.hpp"
-#include "hj_fused.hpp"
 #include "hj_kernels.hpp"
 #include "hj_strat.hpp"
 #include "hj_util.hpp"
