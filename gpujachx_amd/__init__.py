@@ -149,6 +149,8 @@ def lib():
     L.hj_batch_run.restype = i
     L.hj_batch_results.argtypes = [vp, pu, pull, pull, pd, pd]
     L.hj_batch_results.restype = i
+    L.hj_batch_shape.argtypes = [vp, pu, pu]
+    L.hj_batch_shape.restype = i
     L.hj_batch_free.argtypes = [vp]
     L.hj_batch_free.restype = None
     L.hj_batch_autotune.argtypes = [pdesc, u, u, pcfg, pd]
@@ -352,7 +354,9 @@ def dbg_scalar(kind, a, b=None, c=None):
 class Batch:
     """A planned batch of independent (H)SVDs on device buffers (one
     persistent launch captured in a hipGraph).  `descs` is a list of
-    BatchDesc; run() executes it on `stream` (a hipStream_t handle or None)."""
+    BatchDesc; run() executes it on `stream` (a hipStream_t handle or None).
+    `cfg`: its launch shape and schedule; None: the defaults, in the shape that
+    the plan chooses by its problems (shape())."""
 
     def __init__(self, descs, cfg=None):
         L = lib()
@@ -360,7 +364,8 @@ class Batch:
         self._arr = (BatchDesc * self.n)(*descs)
         err = ctypes.c_int(0)
         self.cfg = cfg if cfg is not None else default_batch_cfg()
-        self._plan = L.hj_batch_plan(self._arr, self.n, ctypes.byref(self.cfg), ctypes.byref(err))
+        self._plan = L.hj_batch_plan(self._arr, self.n, ctypes.byref(cfg) if cfg is not None else None,
+                                     ctypes.byref(err))
         if not self._plan:
             raise ValueError("hj_batch_plan failed with %d" % err.value)
 
@@ -376,6 +381,12 @@ class Batch:
         lib().hj_batch_results(self._plan, sw, rs, rb, _pd(t0), _pd(t1))
         return {"sweeps": np.array(sw[:]), "rot_s": np.array(rs[:]), "rot_b": np.array(rb[:]),
                 "start_us": t0, "end_us": t1}
+
+    def shape(self):
+        """(waves per workgroup, workgroups per CU) of the plan."""
+        waves, wg = ctypes.c_uint(0), ctypes.c_uint(0)
+        lib().hj_batch_shape(self._plan, ctypes.byref(waves), ctypes.byref(wg))
+        return waves.value, wg.value
 
     def close(self):
         if self._plan:

@@ -386,10 +386,9 @@ struct Plan {
   double clock_mhz = 100.0;
 };
 
-constexpr unsigned DEFAULT_WAVES = 4u, DEFAULT_WG_PER_CU = 2u;
-
-// The shape of a batch whose caller left it to the library (the default
-// configuration): eight wave slots a CU as one workgroup of eight waves, two of
+// The shape of a batch whose caller left it to the library (no configuration; one
+// that is given runs as it is, the default's 4 x 2 too, which is what the
+// autotuner times): eight wave slots a CU as one workgroup of eight waves, two of
 // four or four of two, whichever ends first when the problems, in queue order,
 // go to the next free workgroup.  A wide workgroup brings the largest problems,
 // which end last, to their end; narrow ones waste no slots on small problems.
@@ -443,8 +442,8 @@ using namespace hj;
 extern "C" void hj_batch_default_cfg(hj_batch_cfg *cfg)
 {
   if (!cfg) return;
-  cfg->waves = DEFAULT_WAVES;
-  cfg->wg_per_cu = DEFAULT_WG_PER_CU;
+  cfg->waves = 4u;
+  cfg->wg_per_cu = 2u;
   cfg->strategy = HJ_BATCH_STRAT_CYCWOR;
   cfg->max_sweeps = HYPJAC_NSWEEP;
   cfg->longest_first = 1u;
@@ -486,7 +485,6 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   }
   Plan *P = new Plan;
   P->n = n;
-  P->cfg = cfg;
   // strategy tables: one per distinct (family, n1)
   std::vector<uint16_t> pool;
   std::vector<std::pair<std::string, unsigned>> keys;
@@ -552,8 +550,9 @@ extern "C" void *hj_batch_plan(const hj_batch_desc *probs, unsigned n, const hj_
   HIP_CALL(hipGetDevice(&dev));
   hipDeviceProp_t prop;
   HIP_CALL(hipGetDeviceProperties(&prop, dev));
-  if (cfg.waves == DEFAULT_WAVES && cfg.wg_per_cu == DEFAULT_WG_PER_CU)
+  if (!cfg_in)
     choose_shape(cfg, P->h_probs, order, (unsigned)prop.multiProcessorCount);
+  P->cfg = cfg;
   P->grid = cfg.wg_per_cu * (unsigned)prop.multiProcessorCount;
   P->lds = sizeof(double) * WAVE_LDS * cfg.waves;
   const size_t lds_max = std::max(prop.sharedMemPerBlock, prop.sharedMemPerBlockOptin);
@@ -619,6 +618,15 @@ extern "C" int hj_batch_results(void *plan, unsigned *sweeps, unsigned long long
     if (start_us) start_us[i] = (double)(o.t0 - tmin) / P->clock_mhz;
     if (end_us) end_us[i] = (double)(o.t1 - tmin) / P->clock_mhz;
   }
+  return 0;
+}
+
+extern "C" int hj_batch_shape(const void *plan, unsigned *waves, unsigned *wg_per_cu)
+{
+  const Plan *P = static_cast<const Plan *>(plan);
+  if (!P) return -1;
+  if (waves) *waves = P->cfg.waves;
+  if (wg_per_cu) *wg_per_cu = P->cfg.wg_per_cu;
   return 0;
 }
 

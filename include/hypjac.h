@@ -207,9 +207,10 @@ typedef struct hj_batch_desc {
 #define HJ_BATCH_STRAT_BRENTL 1u
 #define HJ_BATCH_STRAT_MMSTEP 2u
 
-/* Launch shape and schedule (hj_batch_autotune picks them).  The default
- * shape (4 waves, 2 workgroups per CU) leaves the arrangement of those eight
- * waves a CU to the plan; the results do not depend on it. */
+/* Launch shape and schedule (hj_batch_autotune picks them).  A plan runs the
+ * shape of the configuration it is given; without one (cfg NULL) the
+ * arrangement of eight waves a CU is the plan's choice, by its problems.  The
+ * results do not depend on it. */
 typedef struct hj_batch_cfg {
   unsigned waves;          /* waves per workgroup, 1..8 (one block pair each) */
   unsigned wg_per_cu;      /* workgroups per CU in the persistent grid */
@@ -218,6 +219,7 @@ typedef struct hj_batch_cfg {
   unsigned longest_first;  /* queue order: largest M*N^2 first (else input order) */
 } hj_batch_cfg;
 
+/* The default configuration: 4 waves, 2 workgroups per CU. */
 void hj_batch_default_cfg(hj_batch_cfg *cfg);
 /* Builds the plan of a batch: strategy tables, problem descriptors and the
  * batch captured as one hipGraph (queue reset + the persistent kernel).
@@ -232,6 +234,8 @@ int hj_batch_run(void *plan, void *stream);
 int hj_batch_results(void *plan, unsigned *sweeps, unsigned long long *rot_s,
                      unsigned long long *rot_b, double *start_us,
                      double *end_us);
+/* The launch shape that the plan runs (NULL outputs are skipped). */
+int hj_batch_shape(const void *plan, unsigned *waves, unsigned *wg_per_cu);
 void hj_batch_free(void *plan);
 /* Times every candidate launch shape and strategy on `sample` problems of
  * the batch (copies; the inputs are untouched); best->max_sweeps is kept. */
