@@ -232,7 +232,9 @@ struct Work {
     np = ncol / 32u;
     steps = STRAT1_STEPS;
     s0steps = STRAT0_STEPS;
-    nchunk = gram_nchunk(nrow, np);
+    // (the thin layer takes any multiple of 32 rows: those that 64 does not
+    // divide are one chunk)
+    nchunk = (nrow % 64u) ? 1u : gram_nchunk(nrow, np);
     CH = nrow / nchunk;
     chG = update_rows(nrow, withV ? ncol : 0u, np);
     chV = chG;
@@ -355,10 +357,12 @@ static void check_tables(unsigned ncol)
 // k_update: the pair fits its LDS, and its rows of G and V through one CU cost
 // less than two launches.  Measured, us a step (k_step against the three
 // launches): 64 x 64 39 / 44, 256 x 256 35 / 38, with V 37.3 / 37.7,
-// 384 x 256 37.5 / 39.7, 512 x 512 39.1 / 37.2, with V 44 / 37.5.
+// 384 x 256 37.5 / 39.7, 512 x 512 39.1 / 37.2, with V 44 / 37.5.  It loads 64
+// rows at a time (a row count of the thin layer that 64 does not divide takes the
+// launches).
 static bool step_fits(unsigned nrow, unsigned nrowV)
 {
-  return nrow + nrowV <= STEP_MAX_ROWS;
+  return nrow + nrowV <= STEP_MAX_ROWS && !(nrow % 64u);
 }
 
 // One level-1 step in one launch (plain form, Cholesky).

@@ -990,7 +990,8 @@ void launch_gram(hipStream_t s, const double *G, unsigned ldG, const uint16_t *p
                  unsigned nchunk, unsigned CH, double *part, const uint8_t *skip)
 {
   const unsigned nw = gram_waves(CH);
-  if (np * nchunk * nw <= GRAM_TILES_MAX) {
+  // (k_gram_tiles reads 64-row panels, k_gram 32 rows at a time)
+  if (np * nchunk * nw <= GRAM_TILES_MAX && !(CH % 64u)) {
     const auto k = (nw == 1u) ? k_gram_tiles<1u> : (nw == 2u) ? k_gram_tiles<2u> : k_gram_tiles<4u>;
     hipLaunchKernelGGL(k, dim3(np * nchunk), dim3(256u * nw), 0, s, G, ldG, pairs, nchunk, CH, part,
                        skip);
