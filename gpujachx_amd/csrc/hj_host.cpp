@@ -359,10 +359,11 @@ static void check_tables(unsigned ncol)
 // launches): 64 x 64 39 / 44, 256 x 256 35 / 38, with V 37.3 / 37.7,
 // 384 x 256 37.5 / 39.7, 512 x 512 39.1 / 37.2, with V 44 / 37.5.  It loads 64
 // rows at a time (a row count of the thin layer that 64 does not divide takes the
-// launches).
-static bool step_fits(unsigned nrow, unsigned nrowV)
+// launches) and gives a Gram chunk to one wave (512 rows of more than 256 pairs,
+// the thin layer's again, are chunks of two).
+static bool step_fits(const Work &w, unsigned nrow, unsigned nrowV)
 {
-  return nrow + nrowV <= STEP_MAX_ROWS && !(nrow % 64u);
+  return nrow + nrowV <= STEP_MAX_ROWS && !(nrow % 64u) && gram_waves(w.CH) == 1u;
 }
 
 // One level-1 step in one launch (plain form, Cholesky).
@@ -439,7 +440,7 @@ static void issue_step(hipStream_t s, const Work &w, unsigned step, bool sort, u
     if (ev) HIP_CALL(hipEventRecord(ev[3], s));
     return;
   }
-  if (!ev && !skip && step_fits(nrow, dV ? ncol : 0u)) {
+  if (!ev && !skip && step_fits(w, nrow, dV ? ncol : 0u)) {
     issue_whole_step(s, w, step, sort, nswp, definite, nplus, dG, lddG, nrow, dV, lddV, ncol);
     if (cvg)
       hipLaunchKernelGGL(k_thin_accum, dim3(1), dim3(64), 0, s, w.d_ctl, cvg);
@@ -491,7 +492,7 @@ static unsigned issue_sweep(hipStream_t s, const Work &w, bool sort, unsigned ns
 {
   bool have_gram = false;
   unsigned issued = 0u;
-  const bool whole = !evs && !planned && step_fits(nrow, dV ? ncol : 0u);
+  const bool whole = !evs && !planned && step_fits(w, nrow, dV ? ncol : 0u);
   VItems vlate;  // V's items of the step before (none when profiling)
   for (unsigned st = 0u; st < w.steps; ++st) {
     if (steps_left) {
@@ -765,7 +766,7 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   // launch: for sweeps of whole-step launches only (at most 15 a sweep where a
   // pair has 512 rows of G and V).  64 x 64 1.60 -> 1.40 ms, 256 x 256 9.04 -> 8.87;
   // 512 x 256 with V, three launches a step, 3.30 -> 3.39.
-  const bool ahead = !eager && !staged && !planned && !qr && step_fits(nrow, V ? ncol : 0u) && !g_trace_buf;
+  const bool ahead = !eager && !staged && !planned && !qr && step_fits(w, nrow, V ? ncol : 0u) && !g_trace_buf;
   // graph path: events around each sweep's graph launch, and the launches
   // of the sweep's dominant kind it holds (staged launches; else the steps'
   // update-class launches); sweeps queued ahead: one after the start of each,
