@@ -29,7 +29,7 @@ __device__ __forceinline__ double pin(double x)
 __device__ __forceinline__ uint64_t d2u(double x) { return (uint64_t)__double_as_longlong(x); }
 __device__ __forceinline__ double u2d(uint64_t u) { return __longlong_as_double((long long)u); }
 
-// m*(y+d)^2 - 1 with exact products; see dev_rsqrt.
+// m*(y+d)^2 - 1 with exact products; see rsqrt_core.
 __device__ __forceinline__ double rs_resid(double m, double y, double d)
 {
   const double h = y * y, l = __fma_rn(y, y, -h);
@@ -123,18 +123,6 @@ __device__ __forceinline__ double dev_rsqrt_any(double x)
   return special ? sp : normal;
 }
 
-// The same through rsqrt_bracket where every active lane's x allows it (a
-// wave-uniform branch): the general path is left for special, very large or
-// very small inputs and for values next to a midpoint.
-__device__ __forceinline__ double dev_rsqrt(double x)
-{
-  bool sure;
-  double y = rsqrt_bracket(x, sure);
-  if (__ballot(!(sure && rsqrt_plain_range(x))) != 0ull)
-    y = dev_rsqrt_any(x);
-  return y;
-}
-
 // Correctly rounded 1/sqrt(m) of a rotation's m = 1 +- t^2 (2^-26 < m <= 2,
 // or NaN): no scaling, no special values.
 __device__ __forceinline__ double rsqrt_near1(double m)
@@ -146,56 +134,7 @@ __device__ __forceinline__ double rsqrt_near1(double m)
   return y;
 }
 
-// 2x2 rotation of share/device_code_common_rotate.hpp:189-237 (USE_RSQRT),
-// trigonometric (trig) or hyperbolic, evaluated without divergent branches:
-// every path's operations are issued and the taken branch's results are
-// selected, so the values equal the branch formulas bit for bit.  The square
-// root and the reciprocal square root are skipped by a wave-uniform branch
-// when no active lane of the wave takes a branch that uses them (a nearly
-// converged wave: every pivot pair's |zeta| at or above sqrt(2/eps), c = 1).
-//   trig: zeta = (Dq-Dp)/(2Apq); |zeta| < sqrt(eps/2): t = 1/(|zeta|+1),
-//         |zeta| >= sqrt(2/eps): t = 1/(2|zeta|), c = 1, else
-//         t = 1/(|zeta| + sqrt(zeta^2+1)); c = rsqrt(1+t^2); big = c < 1.
-//   hyp:  zeta = -(Dq+Dp)/(2Apq); |zeta| >= sqrt(2/eps): t = 1/(2|zeta|),
-//         c = 1; |zeta| > 1: t = 1/(|zeta| + sqrt(zeta^2-1)),
-//         c = rsqrt(1-t^2), big = c > 1; else c = 2/sqrt(3), t = 1/2.
-__device__ __forceinline__ int dev_rot(bool trig, double Apq, double Dp, double Dq, double &c,
-                                       double &t)
-{
-  const double h = trig ? (Dq - Dp) : (Dq + Dp);
-  const double qz = pin(h / (2.0 * Apq));
-  const double ct2 = trig ? qz : -qz;
-  const double CT2 = fabs(ct2);
-  const bool large = CT2 >= SQRT_2_HEPS;
-  const bool small = trig && (CT2 < SQRT_HEPS);
-  const bool fix = !trig && !large && !(CT2 > 1.0);
-  double sq = 0.0;
-  if (__ballot(!large && !small && !fix) != 0ull)
-    sq = pin(sqrt(__fma_rn(CT2, CT2, trig ? 1.0 : -1.0)));
-  const double cot = large ? 2.0 * CT2 : (small ? CT2 + 1.0 : CT2 + sq);
-  const double rcot = pin(1.0 / cot);  // (a statement of its own: a pin inside ?: runs on one arm)
-  const double tt = fix ? TANH1_FIX : copysign(rcot, ct2);
-  double cr = 1.0;
-  if (__ballot(!large && !fix) != 0ull)
-    cr = pin(rsqrt_near1(__fma_rn(trig ? tt : -tt, tt, 1.0)));
-  c = large ? 1.0 : (fix ? COSHI_FIX : cr);
-  t = tt;
-  return large ? 0 : ((small || fix) ? 1 : (trig ? (cr < 1.0) : (cr > 1.0)));
-}
-
-__device__ __forceinline__ int dev_rot_t(double Apq, double Dp, double Dq, double &c, double &t)
-{
-  return dev_rot(true, Apq, Dp, Dq, c, t);
-}
-
-__device__ __forceinline__ int dev_rot_h(double Apq, double Dp, double Dq, double &c, double &t)
-{
-  return dev_rot(false, Apq, Dp, Dq, c, t);
-}
-
-// Lane exchanges inside groups of 8 lanes by DPP (no LDS traffic):
-// xor 1 and xor 2 are quad permutations, xor 4 is the half-row mirror
-// (lane i <- 7-i) followed by the quad reversal (i <- 3-i).
+// Lane exchanges by DPP (no LDS traffic): xor 1 and xor 2 are quad permutations.
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v)
 {
@@ -205,7 +144,6 @@ __device__ __forceinline__ double dpp_mov(double v)
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
   return __hiloint2double(hi, lo);
 }
-__device__ __forceinline__ double lane_xor4(double v) { return dpp_mov<0x1B>(dpp_mov<0x141>(v)); }
 __device__ __forceinline__ double lane_xor2(double v) { return dpp_mov<0x4E>(v); }
 __device__ __forceinline__ double lane_xor1(double v) { return dpp_mov<0xB1>(v); }
 
@@ -280,12 +218,24 @@ __device__ __forceinline__ bool surely_orthogonal(double Apq, double Dp, double 
   return less & above & below;
 }
 
-// dev_rot for a pivot pair whose lanes (a multiple of four, from a multiple of
-// four on) all hold the same Apq, Dp, Dq: also sqrt(Dp) sqrt(Dq).  The three
-// square roots -- of zeta^2 +- 1, Dp and Dq -- are one instruction sequence,
+// 2x2 rotation of share/device_code_common_rotate.hpp:189-237 (USE_RSQRT),
+// trigonometric (trig) or hyperbolic, for a pivot pair whose lanes (a multiple of
+// four, from a multiple of four on) all hold the same Apq, Dp, Dq; also
+// sqrt(Dp) sqrt(Dq).  HYP: trig is set per pair, else every pair is
+// trigonometric.  Returns whether the rotation is big.
+//   trig: zeta = (Dq-Dp)/(2Apq); |zeta| < sqrt(eps/2): t = 1/(|zeta|+1),
+//         |zeta| >= sqrt(2/eps): t = 1/(2|zeta|), c = 1, else
+//         t = 1/(|zeta| + sqrt(zeta^2+1)); c = rsqrt(1+t^2); big = c < 1.
+//   hyp:  zeta = -(Dq+Dp)/(2Apq); |zeta| >= sqrt(2/eps): t = 1/(2|zeta|),
+//         c = 1; |zeta| > 1: t = 1/(|zeta| + sqrt(zeta^2-1)),
+//         c = rsqrt(1-t^2), big = c > 1; else c = 2/sqrt(3), t = 1/2.
+// Evaluated without divergent branches: every path's operations are issued and
+// the taken branch's results are selected, so the values equal the branch
+// formulas bit for bit; the reciprocal root is skipped by a wave-uniform branch
+// where no lane takes a branch that uses it.  The three square roots -- of
+// zeta^2 +- 1, Dp and Dq -- are one instruction sequence,
 // on lanes 0, 1 and 2 of every quad, spread by DPP moves (the roots of the
-// norms are wanted late, by the convergence test).  HYP: trig is set per
-// pair, else every pair is trigonometric.  (Pinned values: operands of
+// norms are wanted late, by the convergence test).  (Pinned values: operands of
 // selects, which would otherwise become branches.)
 template <bool HYP>
 __device__ __forceinline__ bool rot_quad(bool trig, double Apq, double Dp, double Dq, unsigned l,
@@ -490,8 +440,7 @@ __device__ __forceinline__ bool chol32_wave(double *A_, double *col_, unsigned l
 
 // Sum of the 32 rows of one pivot pair held by 4 lanes, lane r holding rows
 // r + 4k as v[k]: the xor butterfly 16,8,4,2,1 of the reference's 32-lane
-// reduction (levels 16, 8 and 4 inside the lane, 2 and 1 across lanes) --
-// the bits of sum8x4 on the same rows.
+// reduction (levels 16, 8 and 4 inside the lane, 2 and 1 across lanes).
 __device__ __forceinline__ double sum4x8(const double *v)
 {
   const double a0 = v[0] + v[4], a1 = v[1] + v[5], a2 = v[2] + v[6], a3 = v[3] + v[7];
@@ -580,7 +529,7 @@ __device__ __forceinline__ void wave_level0(double *R_, double *W_, const uint8_
         const unsigned PP = keep ? p : q, QQ = keep ? q : p;
 #pragma unroll
         for (unsigned k = 0u; k < 8u; ++k) {
-          // big rotation: scale by c; otherwise c == 1 exactly (dev_rot), and
+          // big rotation: scale by c; otherwise c == 1 exactly (rot_quad), and
           // c * x is x
           const double rp = __fma_rn(t_, Gq[k], Gp[k]), rq = __fma_rn(t, Gp[k], Gq[k]);
           const double wp = __fma_rn(t_, Vq[k], Vp[k]), wq = __fma_rn(t, Vp[k], Vq[k]);

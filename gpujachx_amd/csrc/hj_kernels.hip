@@ -967,20 +967,31 @@ __global__ void k_sweep_begin(RunCtl *ctl, unsigned long long *ring)
   }
 }
 
-// Scalar self-test kernel.
+// Scalar self-test kernel, four lanes an item as level-0's groups have at least.
+// Kind 0: oc = 1/sqrt(a) as the Cholesky takes it; 1: rot_quad (a, b, c as Apq,
+// Dp, Dq) where every pair is trigonometric, 2, 3: where they differ, a
+// hyperbolic and a trigonometric one; 4, 5, 6: as 1, 2, 3 with oc = sqrt(b) sqrt(c).
 __global__ void k_dbg_scalar(int kind, int n, const double *a, const double *b, const double *c,
                              double *oc, double *ot, int *ob)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double cc = 0.0, tt = 0.0;
-  int big = 0;
-  if (kind == 0) cc = dev_rsqrt(a[i]);
-  else if (kind == 1) big = dev_rot_t(a[i], b[i], c[i], cc, tt);
-  else big = dev_rot_h(a[i], b[i], c[i], cc, tt);
-  oc[i] = cc;
+  const size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x, i = t >> 2;
+  const unsigned l = threadIdx.x & 63u;
+  if (i >= (size_t)n) return;
+  double cc = 0.0, tt = 0.0, dd = 0.0;
+  bool big = false;
+  if (kind == 0) {
+    bool sure;
+    cc = rsqrt_bracket(a[i], sure);
+    if (!(sure && rsqrt_plain_range(a[i]))) cc = dev_rsqrt_any(a[i]);
+  }
+  else if (kind == 1 || kind == 4)
+    big = rot_quad<false>(true, a[i], b[i], c[i], l, cc, tt, dd);
+  else
+    big = rot_quad<true>(kind == 3 || kind == 6, a[i], b[i], c[i], l, cc, tt, dd);
+  if (t & 3u) return;
+  oc[i] = (kind >= 4) ? dd : cc;
   ot[i] = tt;
-  ob[i] = big;
+  ob[i] = big ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1076,7 +1087,7 @@ void launch_sweep_begin(hipStream_t s, RunCtl *ctl, unsigned long long *ring)
 void launch_dbg_scalar(hipStream_t s, int kind, int n, const double *a, const double *b,
                        const double *c, double *oc, double *ot, int *ob)
 {
-  hipLaunchKernelGGL(k_dbg_scalar, dim3((n + 255) / 256), dim3(256), 0, s, kind, n, a, b, c, oc, ot,
+  hipLaunchKernelGGL(k_dbg_scalar, dim3(((unsigned)n + 63u) / 64u), dim3(256), 0, s, kind, n, a, b, c, oc, ot,
                      ob);
 }
 

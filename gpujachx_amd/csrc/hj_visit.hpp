@@ -65,7 +65,7 @@ __device__ __forceinline__ void apply_pair(lds_f64 *ap, lds_f64 *aq, const doubl
   double a[ROWS], b[ROWS];
 #pragma unroll
   for (unsigned i = 0u; i < ROWS; ++i) {
-    // big rotation: scale by c; otherwise c == 1 exactly (dev_rot), and
+    // big rotation: scale by c; otherwise c == 1 exactly (rot_quad), and
     // c * x is x
     const double x = pin(c * __fma_rn(t_, Q[i], P[i])), y = pin(c * __fma_rn(t, P[i], Q[i]));
     a[i] = rot ? x : P[i];

@@ -336,9 +336,11 @@ int hj_last_staged(void);
 #define HJ_FACT_QR_DRMAC 2
 int hj_set_factorization(int f);
 
-/* Device self-test of the scalar kernels: for n inputs, kind 0 = rsqrt(a),
- * 1 = trigonometric rotation (a=Apq,b=Dp,c=Dq), 2 = hyperbolic rotation.
- * Outputs c, t, big per input.  Returns 0 on success. */
+/* Device self-test of the scalar arithmetic that the kernels run: for n inputs,
+ * kind 0 = rsqrt(a), 1 = trigonometric rotation (a=Apq,b=Dp,c=Dq) of the runs
+ * without mixed signs, 2 = hyperbolic, 3 = trigonometric rotation of those with;
+ * 4, 5, 6 = 1, 2, 3 with sqrt(b) sqrt(c), which comes with the rotation, in c's
+ * place.  Outputs c, t, big per input.  Returns 0 on success. */
 int hj_dbg_scalar(int kind, int n, const double *a, const double *b,
                   const double *c, double *out_c, double *out_t, int *out_big);
 
