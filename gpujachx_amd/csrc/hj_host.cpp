@@ -468,10 +468,11 @@ constexpr double UPGRAM_CACHED_BYTES = 2e8;
 // 16-row slab of its sub-chunk (56 FP64 MFMAs and their loads), and two
 // workgroups a CU fit; the two launches move half as much again at 5.2 TB/s,
 // no wave of theirs waits on a chain of products like that.  Measured, us a
-// step fused / not: 1024 x 1024 49 / 41, 1280 x 1024 (4 chunks of 320 rows)
-// 87 / 47, 1088 x 1024 (one of 1088) 201 / 56, 2048 x 1024 49 / 52, 4096 x
-// 1024 50 / 56, 2560 x 2048 90 / 57, 4096 x 2048 61 / 74, 5632 x 4096 151 /
-// 135, 4096 x 4096 86 / 110.
+// step fused / not: 1024 x 1024 50 / 41, 1280 x 1024 (4 chunks of 320 rows)
+// 88 / 48, 1088 x 1024 (one of 1088) 201 / 56, 2048 x 1024 49.9 / 49.2, with V
+// 51.2 / 48.1, 4096 x 1024 51 / 57, 2560 x 2048 90 / 58, 4096 x 2048 62 / 75,
+// 5632 x 4096 152 / 136, 4096 x 4096 87 / 111.  (On the wrong side by 2 %: 4096 x
+// 512, 49.2 / 50.3, not fused.)
 static bool fuse_pays(const Work &w, unsigned nrow, unsigned ncol)
 {
   const double e = (double)nrow * ncol;

@@ -393,7 +393,13 @@ __global__ __launch_bounds__(256, 2) void k_gram_split(const double *__restrict_
 // lanes per pivot pair of level-0 (see visit_core) in k_pair and k_stage
 constexpr unsigned PAIR_LANES = 16u;
 constexpr unsigned STAGE_LANES = 8u;
-constexpr unsigned GRAM_TILES_MAX = 512u;
+// Sub-chunks of a step up to which k_gram_tiles takes its Gram: one a SIMD.
+// Beyond, a wave each fills the chip.  Measured, us a step of three launches with
+// k_gram / k_gram_tiles: 1344 x 672 (21 sub-chunks) 87 / 59, 2560 x 2048 (512)
+// 62.8 / 57.6, 3072 x 1536 (768) 59.7 / 57.4, 2048 x 1024 (1024) 52.7 / 49.3,
+// 4096 x 512 (1024) 51.1 / 50.3, 7168 x 2048 (1024) 100 / 93, 2048 x 2048 (2048)
+// 57.3 / 57.3, 4096 x 1024 (2048) 56.6 / 58.3, 4096 x 2048 (4096) 75.5 / 78.0.
+constexpr unsigned GRAM_TILES_MAX = 1024u;
 
 // The plan a visit runs: a visit planned split whose Gram partials come from
 // the FP64 Gram (a fused transition's that forms FP64 Grams only) is an FP64
