@@ -291,8 +291,8 @@ STAGED_OFF, STAGED_AUTO, STAGED_ALWAYS = 0, 1, 2
 def set_staged(mode):
     """Staged sweeps (each step transition as two launches that overlap pair
     visits with half the block updates): STAGED_OFF, STAGED_AUTO (default:
-    where a step's block updates move at least 4.8e8 bytes) or
-    STAGED_ALWAYS; True means STAGED_AUTO.  Returns the previous mode."""
+    where a step's block updates move at least 4.8e8 bytes and four waves
+    share a row chunk of the Gram) or STAGED_ALWAYS; True means STAGED_AUTO.  Returns the previous mode."""
     return lib().hj_set_staged(int(mode))
 
 

@@ -355,12 +355,17 @@ static void check_tables(unsigned ncol)
 
 // Whether k_step (hj_step.hip) takes a step rather than k_gram, k_pair and
 // k_update: the pair fits its LDS, and its rows of G and V through one CU cost
-// less than two launches.  Measured, us a step (k_step against the three
-// launches): 64 x 64 39 / 44, 256 x 256 35 / 38, with V 37.3 / 37.7,
-// 384 x 256 37.5 / 39.7, 512 x 512 39.1 / 37.2, with V 44 / 37.5.  It loads 64
+// no more than two launches.  Measured, us a step on the device (k_step against
+// the three launches): 256 x 256 33.1 / 36.4, with V 35.5 / 36.5, 320 x 192 with
+// V 35.7 / 39.3, 448 x 448 38.0 / 42.2, 512 x 512 38.7 / 37.0, 512 x 64 36.3 /
+// 36.9; of a whole call, where the sweeps are queued ahead 512 x 512 40.1 / 39.7,
+// 512 x 256 40.2 / 40.1, 512 x 64 47.0 / 49.5, and without allocation, where they
+// are not, 512 x 512 41.3 / 39.9, 512 x 64 44.5 / 46.7, 448 x 448 40.8 / 45.2.
+// (512 x 512 with V, beyond the line: 44 / 37.5.)  It loads 64
 // rows at a time (a row count of the thin layer that 64 does not divide takes the
-// launches) and gives a Gram chunk to one wave (512 rows of more than 256 pairs,
-// the thin layer's again, are chunks of two).
+// launches) and gives a Gram chunk to one wave: 512 rows of more than 256 pairs,
+// the thin layer's again, are four chunks of two waves, whose tiles would have no
+// room behind the columns in LDS either.
 static bool step_fits(const Work &w, unsigned nrow, unsigned nrowV)
 {
   return nrow + nrowV <= STEP_MAX_ROWS && !(nrow % 64u) && gram_waves(w.CH) == 1u;
@@ -764,8 +769,8 @@ static void level2_core(unsigned routine, unsigned nrow, unsigned ncol, unsigned
   // host's round trip and the next graph's start (45 us a sweep; a 64 x 64
   // sweep's steps take 95 us), and no graph is built.  The sweep queued after
   // the last one finds done set and leaves everything as it is, at 1.5 us a
-  // launch: for sweeps of whole-step launches only (at most 15 a sweep where a
-  // pair has 512 rows of G and V).  64 x 64 1.60 -> 1.40 ms, 256 x 256 9.04 -> 8.87;
+  // launch: for sweeps of whole-step launches only (at most 32 a sweep: 512
+  // columns without V).  64 x 64 1.60 -> 1.40 ms, 256 x 256 9.04 -> 8.87;
   // 512 x 256 with V, three launches a step, 3.30 -> 3.39.
   const bool ahead = !eager && !staged && !planned && !qr && step_fits(w, nrow, V ? ncol : 0u) && !g_trace_buf;
   // graph path: events around each sweep's graph launch, and the launches

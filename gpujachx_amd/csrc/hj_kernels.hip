@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256, 2) void k_gram(const double *__restrict__ G, u
 // pairs, or a row count without powers of two: 1344 = 21 x 64 rows are one
 // chain of 336 MFMAs a tile): four waves a sub-chunk, three of them with one
 // tile's chain each, all four reading 64-row panels of the pair's columns
-// into LDS two panels ahead.  Workgroup (pair, chunk), NW sub-chunks.  One
+// into LDS, one panel's loads in flight over the one before.  Workgroup (pair, chunk), NW sub-chunks.  One
 // wave with all three chains and one 32-row group in flight took 46 us for
 // 1344 x 672.
 constexpr unsigned GT_LD = 66u;  // padded panel column: operands in 32 different banks
@@ -385,9 +385,7 @@ __global__ __launch_bounds__(256, 2) void k_gram_split(const double *__restrict_
 // ---------------------------------------------------------------------------
 // Block pair: Gram -> Cholesky -> inner Jacobi -> W, one workgroup per pair.
 // R and W live in LDS, column-major with a padded leading dimension.
-// Cholesky: one wave (chol32_wave).  Inner Jacobi: pair_visit.
-
-// (hj_visit.hpp)
+// Cholesky: one wave (chol32_wave).  Inner Jacobi: pair_visit (hj_visit.hpp).
 
 #define F32(A, r, c) (A)[(c) * 32u + (r)]
 // lanes per pivot pair of level-0 (see visit_core) in k_pair and k_stage
@@ -553,10 +551,6 @@ __global__ __launch_bounds__(32u * PAIR_LANES) void k_pair(
                                  strat0, s0steps, nswp, definite, nplus);
 }
 
-// ---------------------------------------------------------------------------
-// Column norms, G -> U, D = +-||g||^2 (share/device_code_common.hpp:187-219).
-// One wave per column: lane l sums rows l, l+64, ... by fma, then an xor
-// butterfly over 64 lanes (32,16,8,4,2,1).
 // ---------------------------------------------------------------------------
 // Fused step transition: the block update of step s for the two pairs of a
 // closed quad and the Gram partials of the two pairs of step s+1 they form,
@@ -894,6 +888,10 @@ void launch_order_visits(hipStream_t s, const uint16_t *plist, uint16_t *out, co
                      h2);
 }
 
+// ---------------------------------------------------------------------------
+// Column norms, G -> U, D = +-||g||^2 (share/device_code_common.hpp:187-219).
+// One wave per column: lane l sums rows l, l+64, ... by fma, then an xor
+// butterfly over 64 lanes (32,16,8,4,2,1).
 __global__ __launch_bounds__(256) void k_initD(double *__restrict__ G, double *__restrict__ D,
                                                unsigned ifc, unsigned nRow, unsigned nRank,
                                                unsigned nPlus, unsigned ldG)
@@ -935,9 +933,7 @@ __global__ __launch_bounds__(256) void k_initV(double *__restrict__ V, unsigned 
   }
 }
 
-// Start of a level-2 sweep: keep the previous counter, clear the running
-// one, advance the sweep index (a kernel, so no memset node in the graph).
-// Start of a level-2 sweep: the previous sweep's counter becomes prev_cvg,
+// Start of a level-2 sweep (a kernel, so no memset node in the graph): the previous sweep's counter becomes prev_cvg,
 // the counters restart, and the forms' switches for this sweep follow from
 // the previous sweep: a sweep after one that had skipped or split visits and
 // no big rotation certifies (every visit, FP64); otherwise skipping is on

@@ -59,8 +59,8 @@ __device__ __forceinline__ void step_gram(StepLds &L, unsigned ld, unsigned nsub
   }
   // The chains' tiles through LDS, entry by entry summed in sub-chunk order:
   // all three tiles at once behind the columns where there is room (fewer
-  // than STEP_WAVES sub-chunks: at most 448 rows), else one at a time through
-  // the still unused R and W.
+  // than STEP_WAVES sub-chunks, of one wave each: one of up to 448 rows, two of
+  // up to 384 or four of 256), else one at a time through the still unused R and W.
   static_assert(offsetof(PairLds, W) == sizeof(double) * 32u * LDR, "R and W adjoin");
   static_assert(2u * 32u * LDR >= STEP_WAVES * 256u, "room for a tile of every sub-chunk");
   const unsigned rounds = (nsub == STEP_WAVES) ? 3u : 1u;

@@ -47,7 +47,8 @@ __device__ __forceinline__ void apply_pair(lds_f64 *ap, lds_f64 *aq, const doubl
   lds_f64 *const A = cross ? aq : ap, *const B = cross ? ap : aq;
   const double t_ = (!HYP || trig) ? -t : t;
   // every pair of the wave rotates: no selects (worth the branch where a lane
-  // holds eight rows: 4608 x 2048 at width 32 264 -> 261 ms)
+  // holds eight rows: 4608 x 2048 at width 32 263.7 -> 260.3 ms, in three runs in
+  // turn, the runs of one side within 0.1 %)
   if (ROWS > 4u && __ballot(!rot) == 0ull) {
     double x[ROWS], y[ROWS];
 #pragma unroll
@@ -381,7 +382,8 @@ __device__ __forceinline__ void visit_load(unsigned tid, unsigned pi, PairLds &L
 // L: visit_init and the Gram's entries written, not yet synchronized.  plan:
 // the visit's plan (PLAN_FP64 without a plan); not PLAN_SKIP.  Returns, in
 // every thread, whether W (in L.W, synchronized) differs from the identity;
-// writes flags[pi] and, with rec, the record.
+// writes the record and, unless flags is null (k_step, which updates itself),
+// flags[pi].
 template <bool SORT, unsigned LANES>
 __device__ __forceinline__ bool visit_core(unsigned tid, unsigned pi, PairLds &L,
                                            const PairSigns &sg, unsigned *__restrict__ flags,

@@ -273,11 +273,11 @@ void hj_last_sweeps(unsigned *nswp, unsigned *rot_s, unsigned *rot_b,
  * hj_set_profile(1) (graphs are not used while profiling), per launch:
  * kind 0 = Gram, 1 = pair, 2 = update, 3 = unused,
  * 4 = the launches of a staged sweep after step 0's visits (k_stage, and
- * the last step's update).  Without profiling, kind 5 = the graph-launched
- * sweeps: their GPU time (events around each graph launch) and the
- * launches of each sweep's dominant kind they hold (staged launches, else
- * one update-class launch per step).  Returns
- * total ms and launch count. */
+ * the last step's update).  Without profiling, kind 5 = the sweeps: their
+ * GPU time (events around each graph launch, or between the starts of sweeps
+ * queued without one) and the launches of each sweep's dominant kind they
+ * hold (staged launches, else one update-class or whole-step launch per step).
+ * Returns total ms and launch count. */
 void hj_set_profile(int on);
 double hj_kernel_ms(int kind, unsigned long long *launches);
 
@@ -313,7 +313,8 @@ void hj_set_step_limit(long steps);
  * of the step-by-step launches.  mode 0: off; 1 (default): where a step's
  * block updates read and write at least 4.8e8 bytes (512 (nrow + nV)
  * ncol/32; below that the visits' latency is longer than half a step's
- * updates and step-by-step launches are faster); 2: wherever they apply.
+ * updates and step-by-step launches are faster) and four waves share a row
+ * chunk of the Gram (its rows a multiple of 256); 2: wherever they apply.
  * They apply when every step transition forms closed quads, ncol >= 128, no step limit is set and the factorization is
  * Cholesky.  Returns the previous mode; hj_last_staged() tells whether the
  * last hypJacL2 / hypJacL2_dev call used them. */
